@@ -122,13 +122,12 @@ def _stored(rows, cols, batch, pad, cplx, gen, data, dev, by_row=True):
     return x.reshape(-1), ld
 
 
-def prepare(case, seed):
+def _operands(case, seed):
+    """The matrices of a case, made from the seed alone."""
     dev = torch.device("cuda")
     gen = torch.Generator(device=dev)
     gen.manual_seed(seed)
-    handle = cg.Handle()
-    handle.set_stream(torch.cuda.current_stream())
-    s = {"case": case, "handle": handle}
+    s = {}
     cplx = case["cplx"]
     if case["kind"] == "gate":
         rows = case["rows"]
@@ -136,7 +135,6 @@ def prepare(case, seed):
         g = torch.randn((2, 2, 2) if cplx else (2, 2), generator=gen, device=dev).cpu()
         q, _ = torch.linalg.qr(torch.view_as_complex(g) if cplx else g)
         s["u"] = (torch.view_as_real(q.contiguous()) if cplx else q).reshape(-1).to(dev)
-        s["y"] = torch.zeros_like(s["x"])
         return s
     m, n, k, batch, pad = case["m"], case["n"], case["k"], case["batch"], case["pad"]
     op_a, op_b = case["op"]
@@ -152,7 +150,17 @@ def prepare(case, seed):
     if case["beta"]:
         c.normal_(generator=gen)
     s["c"] = c
-    if case["mode"] == "AUTO":
+    return s
+
+
+def prepare(case, seed):
+    s = _operands(case, seed)
+    handle = cg.Handle()
+    handle.set_stream(torch.cuda.current_stream())
+    s["case"], s["handle"] = case, handle
+    if case["kind"] == "gate":
+        s["y"] = torch.zeros_like(s["x"])
+    elif case["mode"] == "AUTO":
         # FP16TCEC while at most a tenth of the elements would lose their low half
         handle.set_exp_stats_params(0.0, 2.0 ** -15, 0.1)
     return s
@@ -208,3 +216,48 @@ def tolerance(case):
     rel = 2.0 ** -24 * (4.0 + 0.5 * math.sqrt(case["k"]))
     # (rows and columns of very different scale: single elements sit further from the root mean square)
     return {"rel": rel, "max": (64 if case["data"] == "spread" else 16) * rel}
+
+
+def exact(case, seed):
+    """What `run` returns, from products in 64 bits."""
+    s = _operands(case, seed)
+    cplx = case["cplx"]
+
+    def parts(x):
+        """Real and imaginary part (or the one part) of a stored operand, in 64 bits."""
+        return [x.view(-1, 2)[:, i].double() for i in (0, 1)] if cplx else [x.double()]
+
+    def product(p, q):
+        if not cplx:
+            return [p[0] @ q[0]]
+        return [p[0] @ q[0] - p[1] @ q[1], p[0] @ q[1] + p[1] @ q[0]]
+
+    def stored(xs):
+        return torch.stack([x.reshape(-1) for x in xs], -1).reshape(-1)
+
+    if case["kind"] == "gate":
+        rows = case["rows"]
+        x, u = parts(s["x"]), parts(s["u"])
+        if case["wide"]:  # column-major 2 x rows, times the 2 x 2 matrix from the left
+            return stored(product([p.view(rows, 2) for p in x], [p.view(2, 2) for p in u]))
+        return stored(product([p.view(2, 2) for p in u], [p.view(2, rows) for p in x]))
+    n, m, batch, ldc = case["n"], case["m"], case["batch"], s["ldc"]
+    out = s["c"].double()
+    per = out.numel() // batch
+    a, b = s["a"].view(batch, -1), s["b"].view(batch, -1)
+
+    def seen(x, op, ld, rows, cols):
+        """op(X) transposed, rows x cols being op(X)'s own sizes."""
+        if op == "N":
+            xs = [p.view(cols, ld)[:, :rows] for p in parts(x)]
+        else:
+            xs = [p.view(rows, ld)[:, :cols].t() for p in parts(x)]
+        return [xs[0], -xs[1]] if op == "C" else xs
+
+    for i in range(batch):
+        at = seen(a[i], case["op"][0], s["lda"], m, case["k"])
+        bt = seen(b[i], case["op"][1], s["ldb"], case["k"], n)
+        # row j of what a column-major matrix is in memory is its column j
+        c = out[i * per:(i + 1) * per].view((n, ldc, 2) if cplx else (n, ldc, 1))[:, :m]
+        c.copy_(torch.stack(product(bt, at), -1) + (case["beta"] * c if case["beta"] else 0))
+    return out
