@@ -686,13 +686,9 @@ PreSplit run_pre_split(cuMpSGEMM_handle *h, const GemmArgs &args, bool a_kc, boo
 int run_narrow(cuMpSGEMM_handle *h, Prec p, bool a_kc, bool b_kc, const GemmArgs &args) {
   const bool few_is_n = args.n <= args.m;
   const uint32_t wide = few_is_n ? args.m : args.n, few = few_is_n ? args.n : args.m;
-  // Measured, tiled -> this kernel, us.  bf16x3, whose tiled kernels are bound by the split: every shape tried,
-  // 8192 x 16 x 8192 65 - 83 -> 44 - 51, 16384 x 32 x 8192 144 - 180 -> 119 - 131, 1024 x 32 x 256 9.3 -> 5.7.
-  // FP16TCEC: 16 rows or columns at any K, 16384 x 1 x 1000 16.5 -> 12.5, 1024 x 16 x 16384 18.9 -> 17.0,
-  // 2048 x 8 x 8192 17 - 24 -> 15.5 - 17; more of them while K is short, 12000 x 30 x 777 17 -> 14,
-  // 1024 x 32 x 256 9.3 -> 6.0 (long K loses: 5000 x 20 x 5000 27 -> 30, 16384 x 32 x 8192 NN 95 -> 128).
-  if ((p != Prec::FP16TCEC && p != Prec::BF16X3) || few > kNarrowMax || wide < kNarrowMinWide) return -1;
-  if (p == Prec::FP16TCEC && few > 16 && args.k > 1024) return -1;
+  if (p != Prec::FP16TCEC && p != Prec::BF16X3) return -1;
+  const NarrowPlan plan = plan_narrow(p == Prec::BF16X3, wide, few, args.k, h->num_cus);
+  if (plan.chunks == 0) return -1;
   NarrowArgs na{};
   const float *a = static_cast<const float *>(args.a), *b = static_cast<const float *>(args.b);
   na.big = few_is_n ? a : b;
@@ -708,21 +704,12 @@ int run_narrow(cuMpSGEMM_handle *h, Prec p, bool a_kc, bool b_kc, const GemmArgs
   na.few_is_n = few_is_n ? 1u : 0u;
   na.alpha = args.alpha_re;
   na.beta = args.beta_re;
-  // Waves on a CU are what keeps loads in flight: 8 a workgroup where there are
-  // two workgroups per CU, 16 below, and K split over workgroups where there
-  // are fewer of them than CUs, as long as every wave has a few steps.
-  const uint32_t tiles = (wide + kNarrowRows - 1) / kNarrowRows, steps = args.k / 32;
-  const uint32_t waves = tiles >= 2u * (uint32_t)h->num_cus ? 8u : 16u;
-  uint32_t chunks = 1;
-  while (tiles * chunks * 2 <= (uint32_t)h->num_cus * 3 / 2 && steps / (chunks * 2) >= 4 * waves) chunks *= 2;
-  // (FP16TCEC, chunks that leave the second round of workgroups mostly empty: 3000 x 3 x 12345 TN 29.3 -> 32.4)
-  if (p == Prec::FP16TCEC && chunks > 1 && tiles * chunks > (uint32_t)h->num_cus) return -1;
-  na.steps_per_chunk = (steps + chunks - 1) / chunks;
-  if (na.steps_per_chunk != 0) chunks = std::max(1u, (steps + na.steps_per_chunk - 1) / na.steps_per_chunk);
-  na.atomic_out = chunks > 1 ? 1u : 0u;
-  if (chunks > 1) launch_prescale_c<false>(h->stream, args.c, args.m, args.n, args.ldc, 0, 1, args.beta_re, 0.0f);
-  launch_narrow(na, p, few_is_n ? a_kc : b_kc, few_is_n ? b_kc : a_kc, waves, chunks, h->stream);
-  return (few_is_n ? 3 : 4) + (chunks > 1 ? 100 : 0);
+  na.steps_per_chunk = plan.steps_per_chunk;
+  na.atomic_out = plan.chunks > 1 ? 1u : 0u;
+  if (plan.chunks > 1)
+    launch_prescale_c<false>(h->stream, args.c, args.m, args.n, args.ldc, 0, 1, args.beta_re, 0.0f);
+  launch_narrow(na, p, few_is_n ? a_kc : b_kc, few_is_n ? b_kc : a_kc, plan.waves, plan.chunks, h->stream);
+  return (few_is_n ? 3 : 4) + (plan.chunks > 1 ? 100 : 0);
 }
 
 template <class T>

@@ -2,13 +2,9 @@
 // one pass over the large operand, see narrow.hip.
 #pragma once
 #include "gemm_kernel.hpp"
+#include "narrow_rule.hpp"
 
 namespace cumpsgemm_amd {
-
-constexpr uint32_t kNarrowMax = 32;  // largest narrow side
-constexpr uint32_t kNarrowRows = 32; // rows of the large operand per workgroup
-
-constexpr uint32_t kNarrowMinWide = 1024; // smallest wide side
 
 struct NarrowArgs {
   const float *big, *small; // op(big): wide x k, op(small): few x k

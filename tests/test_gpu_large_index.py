@@ -43,6 +43,31 @@ def test_tall_operand_beyond_4gib(cg, torch_gpu, handle, op_a, mode):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("op_a,op_b,by_rows", [(N_OP, N_OP, False), (T_OP, N_OP, True)])
+@pytest.mark.parametrize("mode", [FP16TCEC, TF32TCEC])
+def test_narrow_result_of_2_to_the_28(cg, torch_gpu, handle, mode, op_a, op_b, by_rows):
+    """As many rows or columns as no launch can give a group of waves per 32 of them."""
+    torch = torch_gpu
+    dev = torch.device("cuda:0")
+    wide, few, k = 1 << 28, 2, 2
+    m, n = (wide, few) if by_rows else (few, wide)
+    g = torch.Generator(device=dev).manual_seed(8)
+    big = torch.randint(-8, 9, (wide, k), generator=g, device=dev).float()     # K-contiguous
+    small = torch.randint(-8, 9, (few, k), generator=g, device=dev).float()
+    c = torch.full((n, m), 7.0, device=dev)
+    if by_rows:                                                                # C = big * small^T
+        st = handle.gemm(T_OP, N_OP, m, n, k, 1.0, big, k, small, k, 0.0, c, m, mode)
+        want = torch.stack([big[:, 0] * s[0] + big[:, 1] * s[1] for s in small])
+    else:                                                                      # C = small^T's columns: m x k, lda = m
+        st = handle.gemm(N_OP, N_OP, m, n, k, 1.0, small.t().contiguous(), m, big, k, 0.0, c, m, mode)
+        want = torch.stack([big[:, 0] * s[0] + big[:, 1] * s[1] for s in small], 1)
+    assert st == 0
+    torch.cuda.synchronize()
+    assert torch.equal(c, want)                                                # small integers: exact
+    del big, c, want
+    torch.cuda.empty_cache()
+
+
 def test_result_beyond_4gib(cg, torch_gpu, handle):
     torch = torch_gpu
     dev = torch.device("cuda:0")
