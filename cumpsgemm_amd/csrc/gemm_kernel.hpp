@@ -617,7 +617,10 @@ struct tile_loader {
     } else {
       const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<float *>(base), 0, 0xffffffff, 0x00020000);
-      const uint32_t line = (uint32_t)ld * (uint32_t)(ES * 4); // bytes between K-lines
+      // bytes between K-lines.  (Said to be uniform: merged with load_tail's multiples of the same number, which are
+      // per lane, it ends up in vector registers otherwise, and every load of the K loop in a loop over the lanes'
+      // values.  4096 x 2048 x 2048 NN in bf16x2, us: 129 that way, 111 - 116 so.)
+      const uint32_t line = __builtin_amdgcn_readfirstlane((uint32_t)ld * (uint32_t)(ES * 4));
 #pragma unroll
       for (int u = 0; u < U; u++) {
 #pragma unroll
@@ -743,10 +746,7 @@ struct tile_loader {
     if (!active(tid)) return;
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), 0, 0xffffffff, 0x00020000);
-    uint32_t step = (KC ? 1u : (uint32_t)ld) * (uint32_t)(ES * 4); // bytes between K-values
-    // (kept apart from load_fast's scalar multiples of the same number: merged with them, the compiler
-    // holds those in vector registers and wraps every load of the K loop into a loop over the lanes' values)
-    asm("" : "+v"(step));
+    const uint32_t step = (KC ? 1u : (uint32_t)ld) * (uint32_t)(ES * 4); // bytes between K-values
 #pragma unroll
     for (int u = 0; u < U; u++) {
       int row, chunk;

@@ -1,0 +1,56 @@
+"""What the compiler made of the GEMM kernels, read back from the built library."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+import cumpsgemm_amd
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """Name of each kernel -> its instructions, (mnemonic and operands, address, branch target or None)."""
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("no llvm-objdump")
+    lib = os.path.join(os.path.dirname(cumpsgemm_amd.__file__), "libcumpsgemm.so")
+    d = tmp_path_factory.mktemp("code")
+    shutil.copy(lib, d)
+    subprocess.check_call([OBJDUMP, "--offloading", "libcumpsgemm.so"], cwd=d, stdout=subprocess.DEVNULL)
+    out = {}
+    for f in sorted(os.listdir(d)):
+        if not f.endswith("gfx950"):
+            continue
+        code = None
+        for line in subprocess.run([OBJDUMP, "-d", f], cwd=d, capture_output=True, text=True, check=True).stdout.split("\n"):
+            head = re.match(r"^[0-9a-f]+ <(\w+)>:", line)
+            if head:
+                code = out.setdefault(head.group(1), [])
+            elif line.startswith("\t") and code is not None and "//" in line:
+                text, note = line.strip().split("//", 1)
+                at = int(note.split(":")[0], 16)
+                jump = re.match(r"s_cbranch_\w+ (\d+)", text)
+                off = int(jump.group(1)) if jump else 0
+                code.append((text.strip(), at, at + 4 + 4 * (off - 65536 if off >= 32768 else off) if jump else None))
+    return out
+
+
+def loops_over_lane_values(code):
+    """Loads that run once per distinct value of an operand that must be uniform: a few instructions that
+    take one lane's value, load for the lanes that share it and branch back while any are left."""
+    found = 0
+    for i, (text, at, target) in enumerate(code):
+        if text.startswith("s_cbranch_execnz") and target <= at:
+            body = [t for t, a, _ in code[max(0, i - 40):i] if a >= target]
+            found += any(t.startswith("buffer_load") for t in body) and any(t.startswith("v_readfirstlane") for t in body)
+    return found
+
+
+def test_no_load_of_a_gemm_kernel_is_a_loop_over_lane_values(kernels):
+    gemm = {n: c for n, c in kernels.items() if "gemm_tcec_kernel" in n or "narrow_kernel" in n}
+    assert len(gemm) > 200 and all(any("v_mfma" in t for t, _, _ in c) for c in gemm.values())
+    bad = {n: k for n, k in ((n, loops_over_lane_values(c)) for n, c in gemm.items()) if k}
+    assert not bad, bad
