@@ -1007,17 +1007,27 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void gemm_tcec_kernel(c
 
   const int rows_a = (int)((args.m - ml0 < (uint32_t)BM) ? args.m - ml0 : BM);
   const int rows_b = (int)((args.n - nl0 < (uint32_t)BN) ? args.n - nl0 : BN);
+  // The 256x128 kernels of FP16TCEC with two K-contiguous operands: the scaled one has no register left.  With clamped
+  // rows and a partial K-step in front of the pipeline, however loaded, three addresses of its K loop are re-read from
+  // scratch memory in every step, behind the loads in flight.  It takes guarded loads for tiles beyond the edge and for
+  // the partial K-step, which it multiplies last -- and so does the unscaled one, whose sums it repeats bit for bit
+  // (TN, us, clamped and masked first -> guarded last: FP16TCEC_SCALING 2300 x 2100 x 1333 84 -> 76.5,
+  // 2500 x 2500 x 500 50.2 -> 48.5, 2000 x 3000 x 777 56.0 -> 52.3; FP16TCEC 2600 x 2600 x 1300 72.2 -> 71.5,
+  // 2000 x 3000 x 777 41.8 -> 41.9, 2560 x 2560 x 260 19.0 -> 19.8, 16 x 1000 x 1000 x 300 64.9 -> 67.0).
+  constexpr bool GUARD_EDGES = P == Prec::FP16TCEC && Cfg::DEEP && !Cfg::PERSIST && !Cfg::PACKED && !CPLX &&
+                               Cfg::A_KC && Cfg::B_KC && BM * BN == 256 * 128;
   // unguarded loads: every per-thread offset fits 31 bits (a tile higher or wider
   // than the matrix reads its last row or column again)
   // (pre-split operands are padded to whole tiles and K-steps: always unguarded)
-  const bool a_fit = Cfg::PACKED || LA::offsets_fit(args.lda);
-  const bool b_fit = Cfg::PACKED || LB::offsets_fit(args.ldb);
+  const bool a_fit = Cfg::PACKED || (LA::offsets_fit(args.lda) && !(GUARD_EDGES && rows_a != BM));
+  const bool b_fit = Cfg::PACKED || (LB::offsets_fit(args.ldb) && !(GUARD_EDGES && rows_b != BN));
 
+  constexpr bool CLAMP = !Cfg::PERSIST && !GUARD_EDGES; // (the tiles of a walking kernel lie inside the matrix)
   uint32_t offa[Cfg::UA], offb[Cfg::UB];
 #pragma unroll
-  for (int u = 0; u < Cfg::UA; u++) offa[u] = LA::unit_byte_offset(u, tid, (uint32_t)args.lda, Cfg::PERSIST ? BM : rows_a);
+  for (int u = 0; u < Cfg::UA; u++) offa[u] = LA::unit_byte_offset(u, tid, (uint32_t)args.lda, CLAMP ? rows_a : BM);
 #pragma unroll
-  for (int u = 0; u < Cfg::UB; u++) offb[u] = LB::unit_byte_offset(u, tid, (uint32_t)args.ldb, Cfg::PERSIST ? BN : rows_b);
+  for (int u = 0; u < Cfg::UB; u++) offb[u] = LB::unit_byte_offset(u, tid, (uint32_t)args.ldb, CLAMP ? rows_b : BN);
 
   // staging registers: the next tile this wave will split and write to LDS
   typename LA::Regs ra;
@@ -1806,7 +1816,15 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void gemm_tcec_kernel(c
   }
   if (a_fit && b_fit) {
     const int nk_full = klen / BK;
-    if (nk_full > 0) {
+    if constexpr (GUARD_EDGES) {
+      if (nk_full > 0) pipeline(nk_full, std::true_type{}, false);
+      if (klen % BK != 0) {
+        gload(nk_full, std::false_type{});
+        lstore(0);
+        block_sync_lds();
+        mma_tile(0);
+      }
+    } else if (nk_full > 0) {
       pipeline((klen + BK - 1) / BK, std::true_type{}, klen % BK != 0);
     } else { // less than one K-step
       gload_tail(0);

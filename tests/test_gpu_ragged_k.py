@@ -41,3 +41,25 @@ def test_partial_tiles_and_k_steps_read_nothing_but_the_matrices(O, handle, dev,
         # |x| <= 30: one plane holds the values, every partial sum is an integer below 2^24
         co = oracle_gemm(O, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, 0.0, c0, m)
         assert np.array_equal(c, co), (m, n, k)
+
+
+@pytest.mark.parametrize("opa,opb", [(N, N), (T, N), (N, T), (T, T)])
+def test_scaled_large_tiles_at_edges_and_partial_k_steps(handle, dev, monkeypatch, opa, opb):
+    """The 256x128 kernel with the scaling of A and B in it: one tile beyond the edges, moved tiles, K below a step,
+    inside one and a step more; integers times 2^40 stay exact, padding and what lies behind are NaN."""
+    monkeypatch.setenv("CUMPSGEMM_FORCE_TILE_CLASS", "0")
+    monkeypatch.setenv("CUMPSGEMM_PACKED", "0")
+    rng = np.random.default_rng(8)
+    for m, n, k in ((100, 100, 100), (256, 128, 31), (256, 100, 96), (300, 290, 127), (513, 129, 33)):
+        a, lda = _padded_ints(rng, opa, m, k, 3, False)
+        b, ldb = _padded_ints(rng, opb, k, n, 1, False)
+        s = np.float32(2.0 ** 40)
+        da, db, dc = dev.up(a * s), dev.up(b / s), dev.up(np.full(m * n, np.nan, np.float32))
+        st, _ = handle.gemm_pipeline(opa, opb, m, n, k, 1.0, da, lda, db, ldb, 0.0, dc, m, 11)  # FP16TCEC_SCALING
+        assert st == 0
+
+        def logical(x, op, ld, rows, cols):
+            v = x.reshape(-1, ld)[:cols if op == N else rows, :rows if op == N else cols].astype(np.float64)
+            return v.T if op == N else v
+        want = logical(a, opa, lda, m, k) @ logical(b, opb, ldb, k, n)
+        assert np.array_equal(dev.down(dc).reshape(n, m).T, want), (m, n, k)

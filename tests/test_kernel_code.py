@@ -54,3 +54,20 @@ def test_no_load_of_a_gemm_kernel_is_a_loop_over_lane_values(kernels):
     assert len(gemm) > 200 and all(any("v_mfma" in t for t, _, _ in c) for c in gemm.values())
     bad = {n: k for n, k in ((n, loops_over_lane_values(c)) for n, c in gemm.items()) if k}
     assert not bad, bad
+
+
+def scratch_accesses_of_k_loops(code):
+    """Scratch loads and stores inside loops that multiply."""
+    found = 0
+    for i, (text, at, target) in enumerate(code):
+        if target is not None and target <= at:
+            body = [t for t, a, _ in code[:i] if a >= target]
+            if any(t.startswith("v_mfma") for t in body):
+                found += sum(t.startswith("scratch_") for t in body)
+    return found
+
+
+def test_scaled_large_kernel_of_k_contiguous_operands_keeps_its_addresses_in_registers(kernels):
+    # GemmCfg<FP16TCEC, real, K-contiguous, K-contiguous, 256, 128, 64, 64, 2, DEEP, one tile, SCALED, in-loop>
+    (code,) = [c for n, c in kernels.items() if "PrecE0ELb0ELb1ELb1ELi256ELi128ELi64ELi64ELi2ELb1ELb0ELb1ELb0E" in n]
+    assert scratch_accesses_of_k_loops(code) == 0
