@@ -687,7 +687,8 @@ int run_narrow(cuMpSGEMM_handle *h, Prec p, bool a_kc, bool b_kc, const GemmArgs
   const bool few_is_n = args.n <= args.m;
   const uint32_t wide = few_is_n ? args.m : args.n, few = few_is_n ? args.n : args.m;
   if (p != Prec::FP16TCEC && p != Prec::BF16X3) return -1;
-  const NarrowPlan plan = plan_narrow(p == Prec::BF16X3, wide, few, args.k, h->num_cus);
+  const bool big_kc = few_is_n ? a_kc : b_kc, small_kc = few_is_n ? b_kc : a_kc;
+  const NarrowPlan plan = plan_narrow(p == Prec::BF16X3, big_kc, small_kc, wide, few, args.k, h->num_cus);
   if (plan.chunks == 0) return -1;
   NarrowArgs na{};
   const float *a = static_cast<const float *>(args.a), *b = static_cast<const float *>(args.b);
@@ -708,7 +709,7 @@ int run_narrow(cuMpSGEMM_handle *h, Prec p, bool a_kc, bool b_kc, const GemmArgs
   na.atomic_out = plan.chunks > 1 ? 1u : 0u;
   if (plan.chunks > 1)
     launch_prescale_c<false>(h->stream, args.c, args.m, args.n, args.ldc, 0, 1, args.beta_re, 0.0f);
-  launch_narrow(na, p, few_is_n ? a_kc : b_kc, few_is_n ? b_kc : a_kc, plan.waves, plan.chunks, h->stream);
+  launch_narrow(na, p, big_kc, small_kc, plan.waves, plan.chunks, h->stream);
   return (few_is_n ? 3 : 4) + (plan.chunks > 1 ? 100 : 0);
 }
 
