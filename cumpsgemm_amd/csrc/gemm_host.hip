@@ -680,9 +680,8 @@ PreSplit run_pre_split(cuMpSGEMM_handle *h, const GemmArgs &args, bool a_kc, boo
   return PreSplit::DONE;
 }
 
-// Real product with a narrow side (narrow.hip).  Launches it and returns the
-// class number of the tall / short tiles that take such a result otherwise
-// (+ 100: K split, as there), or -1: not one for this kernel.
+// Real product with a narrow side (narrow.hip).  Launches it and returns its
+// module id, or -1: not one for this kernel.
 int run_narrow(cuMpSGEMM_handle *h, Prec p, bool a_kc, bool b_kc, const GemmArgs &args) {
   const bool few_is_n = args.n <= args.m;
   const uint32_t wide = few_is_n ? args.m : args.n, few = few_is_n ? args.n : args.m;
@@ -710,7 +709,7 @@ int run_narrow(cuMpSGEMM_handle *h, Prec p, bool a_kc, bool b_kc, const GemmArgs
   if (plan.chunks > 1)
     launch_prescale_c<false>(h->stream, args.c, args.m, args.n, args.ldc, 0, 1, args.beta_re, 0.0f);
   launch_narrow(na, p, big_kc, small_kc, plan.waves, plan.chunks, h->stream);
-  return (few_is_n ? 3 : 4) + (plan.chunks > 1 ? 100 : 0);
+  return kNarrowModuleId + (plan.chunks > 1 ? 100 : 0);
 }
 
 template <class T>

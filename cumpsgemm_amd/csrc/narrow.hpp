@@ -1,10 +1,13 @@
 // Real products with one narrow side (C has at most kNarrowMax rows or columns):
 // one pass over the large operand, see narrow.hip.
 #pragma once
-#include "gemm_kernel.hpp"
+#include "gemm_table.hpp"
 #include "narrow_rule.hpp"
 
 namespace cumpsgemm_amd {
+
+// what used_kernel_module_id reports for it: the number behind the table's classes (+ 100: K split, as there)
+constexpr int kNarrowModuleId = kNumTileClasses;
 
 struct NarrowArgs {
   const float *big, *small; // op(big): wide x k, op(small): few x k
