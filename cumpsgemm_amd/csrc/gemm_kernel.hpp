@@ -587,6 +587,7 @@ struct tile_loader {
   //   KC:  16-byte global loads at base + constant per-thread offset.
   // (16-byte *buffer* loads are avoided on purpose: this toolchain narrows them
   // incorrectly when the loaded vector is taken apart element-wise.)
+  template <bool BESIDE_TAIL>
   __device__ static inline void load_fast(Regs &reg, const float *__restrict__ base, uint64_t ld,
                                           const uint32_t (&boff)[U]) {
     if (!active(threadIdx.x)) return;
@@ -617,10 +618,12 @@ struct tile_loader {
     } else {
       const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<float *>(base), 0, 0xffffffff, 0x00020000);
-      // bytes between K-lines.  (Said to be uniform: merged with load_tail's multiples of the same number, which are
-      // per lane, it ends up in vector registers otherwise, and every load of the K loop in a loop over the lanes'
-      // values.  4096 x 2048 x 2048 NN in bf16x2, us: 129 that way, 111 - 116 so.)
-      const uint32_t line = __builtin_amdgcn_readfirstlane((uint32_t)ld * (uint32_t)(ES * 4));
+      // bytes between K-lines.  (Said to be uniform beside load_tail: merged with its multiples of the same number,
+      // which are per lane, it ends up in vector registers otherwise, and every load of the K loop in a loop over the
+      // lanes' values.  4096 x 2048 x 2048 NN in bf16x2, us: 129 that way, 111 - 116 so.  A walking kernel has no
+      // load_tail, and the instruction would stay in its loop: batch 64 x 512^3 complex 225.4 without, 227.4 with it.)
+      uint32_t line = (uint32_t)ld * (uint32_t)(ES * 4);
+      if constexpr (BESIDE_TAIL) line = __builtin_amdgcn_readfirstlane(line);
 #pragma unroll
       for (int u = 0; u < U; u++) {
 #pragma unroll
@@ -1070,8 +1073,8 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void gemm_tcec_kernel(c
         LB::template load_packed<NP * NCOMP>(rb, bp, (uint32_t)args.ldb * 64u);
       }
     } else if constexpr (FAST) {
-      LA::load_fast(ra, ap, args.lda, offa);
-      LB::load_fast(rb, bp, args.ldb, offb);
+      LA::template load_fast<!Cfg::PERSIST>(ra, ap, args.lda, offa);
+      LB::template load_fast<!Cfg::PERSIST>(rb, bp, args.ldb, offb);
     } else {
       const int k_left = klen - kt * BK;
       LA::load_guarded(ra, ap, args.lda, rows_a, k_left, tid);
