@@ -511,7 +511,8 @@ __device__ inline void map_tile_batched(uint32_t vid, uint32_t tiles_m, uint32_t
 //         read consecutive addresses.
 // All addresses are "uniform base + per-thread 32-bit offset": the bases live
 // in scalar registers, the offsets are computed once per kernel.
-// Out-of-range elements read as zero, which contributes nothing to the sums.
+// Rows past the edge read the last row again (their products are not stored);
+// K-values past the end are replaced by zero, which adds nothing to the sums.
 // ---------------------------------------------------------------------------
 //   TID0: with fewer units than threads, the first thread that stages this
 //         operand (the ROWS * 4 threads from there on do).
@@ -743,7 +744,7 @@ struct tile_loader {
   // and replaced by zero -- so that all loads of a thread are in flight together.
   // (`boff`: the clamped offsets of an ordinary step.  With branches around every
   // load, in partial tiles around those of every step, 1000 products of 100^3 took
-  // 52.5 us and take 37.0; 1531 x 1021 x 777 TT 23.5 -> 22.8, 8192 x 16 x 8192 71.6 -> 70.4.)
+  // 52.5 us and take 37 - 38.5; 1531 x 1021 x 777 TT 23.5 -> 22.8.)
   __device__ static inline void load_tail(Regs &reg, const float *__restrict__ base, uint64_t ld,
                                           const uint32_t (&boff)[U], int k_left, int tid) {
     if (!active(tid)) return;
@@ -774,9 +775,10 @@ struct tile_loader {
     }
   }
 
-  // offsets beyond 31 bits (huge ld): element-wise and guarded.  The branches
-  // keep only one load in flight per thread, which keeps this rarely used path
-  // from dictating the kernel's register budget.
+  // offsets beyond 31 bits (huge ld), and what the kernels with GUARD_EDGES read
+  // at an edge: element-wise and guarded.  The branches keep only one load in
+  // flight per thread, which keeps this rarely used path from dictating the
+  // kernel's register budget.
   __device__ static inline void load_guarded(Regs &reg, const float *__restrict__ base, uint64_t ld,
                                              int rows_left, int k_left, int tid) {
     if (!active(tid)) return;
@@ -787,8 +789,8 @@ struct tile_loader {
       const int k0 = chunk * 8 + half_of(tid) * 4;
       if constexpr (KC) {
         // a unit that lies inside the matrix is 8 (complex: 16) consecutive
-        // floats: wide loads, like an interior tile (a narrow operand next to a
-        // long one -- C with a few columns -- sends both through this loader)
+        // floats: wide loads, like an interior tile (most units of a partial
+        // K-step do)
         if (row < rows_left && k0 + KV <= k_left) {
           typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
           const f4u_t *p = reinterpret_cast<const f4u_t *>(base + ((uint64_t)row * ld + k0) * ES);

@@ -270,7 +270,7 @@ def test_persistent_split_k(O, handle, dev, monkeypatch):
 @pytest.mark.parametrize("cplx,opa,opb,m,n,k,alpha,beta", [
     (False, N, N, 300, 200, 160, 1.5, -0.5),     # K a multiple of 32: persistent kernels
     (False, T, N, 257, 129, 96, 1.0, 1.0),
-    (False, N, T, 511, 383, 75, 1.0, 0.25),      # ragged K: one-tile kernels with a guarded tail
+    (False, N, T, 511, 383, 75, 1.0, 0.25),      # ragged K: one-tile kernels, the partial K-step first
     (False, T, T, 256, 131, 130, 2.0, 0.0),
     (True, N, N, 200, 150, 128, 1.0 - 0.5j, 0.5 + 0.25j),
     (True, C, T, 129, 65, 70, 1.0, 1.0),
@@ -298,8 +298,8 @@ def test_edge_tiles_split_k(O, handle, dev, monkeypatch, cls):
 
 # ---- C with a few columns, or a few rows -------------------------------------------
 # Tile classes 3 (256 x 32) and 4 (32 x 256) serve products whose result is at most 32 wide or high:
-# the long operand is streamed once, K is split so that every CU has a share, the narrow operand goes
-# through the guarded loader (wide loads where a unit lies inside the matrix).
+# the long operand is streamed once, K is split so that every CU has a share, tile rows beyond the narrow
+# operand read its last one again.  (Real FP16TCEC and bf16x3 mostly take a kernel of their own, test_gpu_narrow.py.)
 @pytest.mark.parametrize("mode", [FP16TCEC, TF32TCEC])
 @pytest.mark.parametrize("opa,opb", [(N, N), (T, N), (N, T), (T, T)])
 @pytest.mark.parametrize("m,n,k,want_cls", [
@@ -678,7 +678,7 @@ def test_k_zero_prepares_c_exactly(handle, dev, torch_gpu, cplx, m, n, ldc, batc
 @pytest.mark.parametrize("opa,opb,m,n,k", [
     (N, N, 1, 4096, 4096),      # row vector times matrix
     (T, N, 4096, 1, 300),       # matrix times column vector
-    (N, T, 5, 7, 10000),        # tiny output, long K: split-K with guarded loads
+    (N, T, 5, 7, 10000),        # tiny output, long K: split-K, tiles larger than C
     (T, T, 3, 1, 1),
     (N, N, 2000, 3, 64),
     (N, N, 31, 33, 17),

@@ -1,7 +1,7 @@
 """Results of at most 32 rows or columns: the kernel that reads the large operand once.
 Edges: a last tile that ends inside a tile of 32, one and two blocks of the narrow side, K below
-a step, inside one and split over workgroups.  NaN between and behind the matrices must not
-reach a result; |x| <= 30, so one plane holds the values and every sum is exact."""
+a step and inside one.  First without correction terms (NaN between and behind the matrices must not
+reach a result; |x| <= 30, so one plane holds the values and every sum is exact), then with them."""
 import numpy as np
 import pytest
 
