@@ -1,6 +1,7 @@
 // Host side of the GEMM path: handle life cycle, tile selection, launches and
 // the C ABI.  Takes the place of reference src/handle.cu:7-52 and
 // src/cumpsgemm.cu:19-605.
+#include "gemm_kwaves_table.hpp"
 #include "gemm_table.hpp"
 #include "handle.hpp"
 #include "narrow.hpp"
@@ -34,6 +35,8 @@ Tuning read_tuning_env() {
   t.no_column_split = std::getenv("CUMPSGEMM_NO_COLUMN_SPLIT") != nullptr;
   t.cut_percent = as_int("CUMPSGEMM_CUT_PERCENT", t.cut_percent);
   t.no_narrow = std::getenv("CUMPSGEMM_NO_NARROW") != nullptr;
+  t.kwaves = as_int("CUMPSGEMM_KWAVES", -1);
+  if (t.kwaves < 0 || t.kwaves > kKWavesForms) t.kwaves = -1;
   t.no_kslices = std::getenv("CUMPSGEMM_NO_KSLICE_GROUPS") != nullptr;
   t.no_edge16_twin = std::getenv("CUMPSGEMM_NO_EDGE16_TWIN") != nullptr;
   t.no_fused_scaling = std::getenv("CUMPSGEMM_NO_FUSED_SCALING") != nullptr;
@@ -345,6 +348,21 @@ bool persistent_ok(const KernelEntry *e, bool a_kc, bool b_kc, uint64_t m, uint6
   if (!fits(a_kc, (uint64_t)e->bm, lda) || !fits(b_kc, (uint64_t)e->bn, ldb)) return false;
   if ((uint64_t)plan.tiles_m * plan.tiles_n * batch > 0x7fffffffull) return false;
   return true;
+}
+
+// Small products (gemm_kwaves.hpp): instances of a precision, [layout][form].
+const KWavesEntry *lookup_kwaves(Prec p, bool cplx, bool a_kc, bool b_kc) {
+  const int layout = (a_kc ? 1 : 0) + (b_kc ? 2 : 0);
+  switch (p) {
+  case Prec::FP16TC:
+    return cplx ? g_kwaves_fp16tc_c[layout] : g_kwaves_fp16tc_s[layout];
+  case Prec::BF16X3:
+    return cplx ? g_kwaves_bf16x3_c[layout] : g_kwaves_bf16x3_s[layout];
+  case Prec::BF16X2:
+    return cplx ? g_kwaves_bf16x2_c[layout] : g_kwaves_bf16x2_s[layout];
+  default:
+    return cplx ? g_kwaves_fp16tcec_c[layout] : g_kwaves_fp16tcec_s[layout];
+  }
 }
 
 template <class T> struct scalar_parts;
@@ -870,13 +888,28 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
   // AUTO launches two gated kernels that must agree on how C is prepared, so
   // the split-K decision is taken once, from the first candidate.
   Plan plan0 = make_plan(h, launches[0].p, CPLX, a_kc, b_kc, m, n, k, batch, force_cls, force_split);
-  const bool split = plan0.ksplit > 1;
+
+  // Small products: K shared out over a workgroup's waves.  (AUTO: both candidates must agree on whether C is
+  // prepared and added to, so where the tiled plan splits K either both go this way or neither.)
+  int kwaves[2] = {-1, -1};
+  // (CUMPSGEMM_NO_KSLICE_GROUPS asks for the four-wave tiled kernel)
+  if (force_cls < 0 && force_split == 0 && h->ws_override == nullptr && !tuning().no_kslices) {
+    const KWavesProblem problem{CPLX, a_kc, b_kc, m, n, k, batch, lda, ldb};
+    for (int i = 0; i < nlaunch; i++) {
+      const Plan tiled = i == 0 ? plan0 : make_plan(h, launches[i].p, CPLX, a_kc, b_kc, m, n, k, batch, -1, 0);
+      kwaves[i] = choose_kwaves_form((int)launches[i].p, problem, h->num_cus, tiled.cost / (256.0 * 128.0),
+                                     tiled.ksplit > 1, tuning().kwaves);
+    }
+    if (plan0.ksplit > 1 && nlaunch == 2 && (kwaves[0] < 0 || kwaves[1] < 0)) kwaves[0] = kwaves[1] = -1;
+  }
+  const bool any_kwaves = kwaves[0] >= 0 || kwaves[1] >= 0;
+  const bool split = plan0.ksplit > 1 && !any_kwaves;
 
   // A tile count just above a multiple of the chip's CU slots leaves most CUs
   // idle for the last round.  C's columns are independent, so such a problem is
   // cut in two: a first part whose tiles fill whole rounds, and the remaining
   // columns, planned on their own (typically with K split to fill the chip).
-  if (!split && batch == 1 && depth == 0 && !fp16_served && k >= 256 &&
+  if (!split && !any_kwaves && batch == 1 && depth == 0 && !fp16_served && k >= 256 &&
       !tuning().no_column_split) {
     // (C's rows are independent as well: the cut that leaves the cheaper pair of
     // problems wins -- which one that is depends on the tile's aspect ratio)
@@ -911,6 +944,11 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
     if (cost_cut >= 0.0 && cost_cut < 0.01 * cut_percent * plan0.cost) return run_cut(by_rows, m1, n1, 1);
   }
 
+  auto set_fused_scaling = [&](GemmArgs &g) {
+    g.scale_max_a = &h->stats_slots[h->fused_slot_a].max_exp_bits;
+    g.scale_max_b = &h->stats_slots[h->fused_slot_b].max_exp_bits;
+    g.scale_flag = h->flag_buffer + h->fused_flag;
+  };
   if (split) {
     launch_prescale_c<CPLX>(h->stream, c, args.m, args.n, ldc, stridec, (uint32_t)batch, args.beta_re,
                             args.beta_im);
@@ -918,6 +956,23 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
   (void)beta_zero;
 
   for (int i = 0; i < nlaunch; i++) {
+    if (kwaves[i] >= 0) {
+      const KWavesForm &f = kwaves_model((int)launches[i].p, CPLX).form[kwaves[i]];
+      const KWavesEntry &e = lookup_kwaves(launches[i].p, CPLX, a_kc, b_kc)[kwaves[i]];
+      args.tiles_m = (uint32_t)((m + f.bm - 1) / f.bm);
+      args.tiles_n = (uint32_t)((n + f.bn - 1) / f.bn);
+      args.batch = (uint32_t)batch;
+      args.flag_accept_mask = launches[i].accept;
+      auto launch = e.launch;
+      if (h->fused_scaling && launches[i].p == Prec::FP16TCEC) {
+        launch = e.launch_scaled;
+        set_fused_scaling(args);
+      }
+      launch(args, dim3(args.tiles_m * args.tiles_n * args.batch, 1, 1), h->stream);
+      // (reported as the small tile class; a form that was asked for by its own id, so that a test can tell)
+      if (used_id != nullptr) *used_id = mode == CUMPSGEMM_AUTO ? ~0u : tuning().kwaves > 0 ? kKWavesModuleId : 2u;
+      continue;
+    }
     Plan plan = (i == 0) ? plan0
                          : make_plan(h, launches[i].p, CPLX, a_kc, b_kc, m, n, k, batch, force_cls, force_split);
     if (split) { // same K partition for every candidate
@@ -939,9 +994,7 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
     if (h->fused_scaling && launches[i].p == Prec::FP16TCEC) {
       launch_plain = e->launch_scaled;
       launch_walk = e->launch_scaled_persistent;
-      args.scale_max_a = &h->stats_slots[h->fused_slot_a].max_exp_bits;
-      args.scale_max_b = &h->stats_slots[h->fused_slot_b].max_exp_bits;
-      args.scale_flag = h->flag_buffer + h->fused_flag;
+      set_fused_scaling(args);
     }
     if (launch_walk != nullptr && !no_persist &&
         persistent_ok<T>(e, a_kc, b_kc, m, n, k, plan, lda, ldb, batch,

@@ -79,6 +79,8 @@ struct Tuning {
                                  // share of the uncut plan (unset: 93, complex 96, complex bf16x3 110)
   bool no_kslices = false;       // CUMPSGEMM_NO_KSLICE_GROUPS
   bool no_narrow = false;        // CUMPSGEMM_NO_NARROW: results with a narrow side take the tiled kernels
+  int kwaves = -1;               // CUMPSGEMM_KWAVES: 0 never, 1 ... the form of the small-product kernel, where it can
+                                 // serve the call (gemm_kwaves_*.hip)
   bool no_fused_scaling = false; // CUMPSGEMM_NO_FUSED_SCALING
   unsigned persistent_max_steps = 32; // CUMPSGEMM_PERSISTENT_MAX_STEPS
   // CUMPSGEMM_MAX_WORKSPACE_BYTES: the pre-split path is not taken when its

@@ -1,0 +1,110 @@
+// Which products the small-product kernel (gemm_kwaves.hpp) takes and with which
+// tile.  Host arithmetic on sizes and layouts alone.
+#pragma once
+#include <cstdint>
+
+namespace cumpsgemm_amd {
+
+constexpr int kKWavesForms = 3; // tiles per precision, real or complex
+constexpr unsigned kKWavesModuleId = 6;
+
+// Tile and waves of a form, workgroups that a CU holds at once, and the time of a
+// tile in us: `fill` for prologue, sums and write-out, `step` per K-step of a wave,
+// longer by `beside` for every other workgroup on the CU.  bm == 0: no such form.
+struct KWavesForm {
+  int bm, bn, waves, resident;
+  double fill, step, beside;
+};
+// ... and what the plan of the tiled kernels takes: us = tiled0 + tiled_per_step *
+// cost, the plan's cost in K-steps of a 256 x 128 tile, + tiled_split if K is split.
+//
+// All of it fitted on 128 products (84 real, m and n 64 - 4096, K 64 - 8192, 44
+// complex, half as large; four layouts, padded, with and without C), each timed with
+// every form and tiled, in every precision.  The form that the fit picks takes 1.9 %
+// (real) and 0.4 % (complex) longer than the fastest; times of all products with
+// the rule over times without: FP16TCEC 0.81 / 0.64 (real / complex), bf16x3
+// 0.80 / 0.59, FP16TC 0.76 / 0.64, bf16x2 0.80 / 0.64.
+struct KWavesModel {
+  KWavesForm form[kKWavesForms];
+  double tiled0, tiled_per_step, tiled_split;
+};
+// `prec`: 0 FP16TCEC, 1 FP16TC, 2 bf16x3, 3 bf16x2
+inline const KWavesModel &kwaves_model(int prec, bool cplx) {
+  static const KWavesModel real[4] = {
+      {{{64, 64, 4, 1, 3.3, 0.97, 0.0}, {32, 32, 8, 2, 0.90, 0.90, 0.79}, {32, 32, 4, 4, 0.76, 0.51, 0.76}}, 4.4, 1.50, -1.7},
+      {{{64, 64, 4, 1, 2.2, 0.79, 0.0}, {32, 32, 8, 2, 0.77, 0.89, 0.58}, {32, 32, 4, 4, 0.75, 0.48, 0.66}}, 4.9, 1.12, 1.6},
+      {{{64, 64, 4, 1, 3.3, 1.68, 0.0}, {32, 32, 8, 1, 1.50, 1.20, 0.0}, {32, 32, 4, 3, 1.12, 0.78, 0.53}}, 2.2, 2.16, -1.5},
+      {{{64, 64, 4, 1, 3.3, 1.00, 0.0}, {32, 32, 8, 2, 0.92, 0.88, 0.83}, {32, 32, 4, 4, 0.79, 0.52, 0.74}}, 4.0, 1.53, -1.0}};
+  static const KWavesModel complex[4] = {
+      {{{32, 32, 4, 1, 2.2, 1.02, 0.0}, {64, 32, 4, 1, 3.5, 1.67, 0.0}, {}}, 2.8, 2.05, -5.4},
+      {{{32, 32, 4, 1, 1.8, 0.74, 0.0}, {64, 32, 4, 1, 2.2, 1.12, 0.0}, {}}, 3.6, 1.50, -3.4},
+      {{{32, 32, 4, 1, 2.3, 1.71, 0.0}, {}, {}}, 0.9, 3.83, -14.3},
+      {{{32, 32, 4, 1, 2.2, 1.06, 0.0}, {64, 32, 4, 1, 3.7, 1.72, 0.0}, {}}, 3.1, 2.09, -6.1}};
+  return (cplx ? complex : real)[prec];
+}
+
+struct KWavesProblem {
+  bool cplx, a_kc, b_kc; // operand stored K-contiguous
+  uint64_t m, n, k, batch, lda, ldb;
+};
+
+inline uint64_t kwaves_tiles(const KWavesForm &f, const KWavesProblem &p) {
+  return (p.m + f.bm - 1) / f.bm * ((p.n + f.bn - 1) / f.bn) * p.batch;
+}
+
+inline double kwaves_time(const KWavesForm &f, const KWavesProblem &p, unsigned cus) {
+  const uint64_t steps = ((p.k + 31) / 32 + f.waves - 1) / f.waves;
+  const uint64_t per_cu = (kwaves_tiles(f, p) + cus - 1) / cus, rounds = (per_cu + f.resident - 1) / f.resident;
+  const double beside = (double)((per_cu < (uint64_t)f.resident ? per_cu : (uint64_t)f.resident) - 1);
+  return 2.2 + (double)rounds * (f.fill + (double)steps * f.step * (1.0 + f.beside * beside));
+}
+
+// Whether a form can serve the product at all.
+inline bool kwaves_can_serve(const KWavesForm &f, const KWavesProblem &p) {
+  if (f.bm == 0 || p.k == 0) return false;
+  // a row-contiguous operand is read 16 bytes a lane: its tile must lie inside the matrix
+  if ((!p.a_kc && p.m < (uint64_t)f.bm) || (!p.b_kc && p.n < (uint64_t)f.bn)) return false;
+  // byte offsets inside a tile's K-step are 31 bits
+  auto fits = [&](bool kc, uint64_t rows, uint64_t ld) {
+    return ld < 0x80000000ull && ((kc ? rows : 32) * ld + (kc ? 32 : rows)) * (p.cplx ? 8 : 4) < 0x7fffffffull;
+  };
+  if (!fits(p.a_kc, (uint64_t)f.bm, p.lda) || !fits(p.b_kc, (uint64_t)f.bn, p.ldb)) return false;
+  // threads of a launch along one axis (sizes below 2^31, at most 65535 matrices: see run_gemm)
+  if ((p.m + f.bm - 1) / f.bm * ((p.n + f.bn - 1) / f.bn) >= (1ull << 32)) return false;
+  return kwaves_tiles(f, p) * (uint64_t)f.waves * 64 < (1ull << 32);
+}
+
+// The form that serves the product, or -1: the tiled kernels do.  `tiled_steps`,
+// `tiled_split`: the tiled plan's cost as above, whether it splits K.  `asked`: -1, or
+// 0 never, 1 ... this form wherever it can.
+inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, double tiled_steps, bool tiled_split,
+                              int asked) {
+  if (asked == 0) return -1;
+  const KWavesModel &model = kwaves_model(prec, p.cplx);
+  // (complex tiles take 6 % longer per step with two row-contiguous operands, 7 % less with none)
+  const double layout = !p.cplx ? 1.0 : p.a_kc && p.b_kc ? 0.93 : !p.a_kc && !p.b_kc ? 1.06 : 1.0;
+  const double tiled = model.tiled0 + layout * model.tiled_per_step * tiled_steps + (tiled_split ? model.tiled_split : 0.0);
+  // Both sides are estimates, the tiled one within 15 % (95 % of 700 products within 25 %): with 1.0 here the number
+  // of products that get more than 3 % slower doubles and the mean stays.  Long ones have less to gain: 0.8.
+  double best_time = (tiled > 30.0 ? 0.8 : 0.9) * tiled;
+  int best = -1;
+  for (int i = 0; i < kKWavesForms; i++) {
+    const KWavesForm &f = model.form[i];
+    if (!kwaves_can_serve(f, p)) continue;
+    if (asked > 0) {
+      if (asked == i + 1) return i;
+      continue;
+    }
+    // More than two tiles per workgroup that a CU holds, and more than a short K: bound by what a tile this small
+    // reads, which the fit misses (1536^3 TT 41 us tiled, 52 here; 1664^3 NT 44, 53).
+    const uint64_t per_cu = (kwaves_tiles(f, p) + cus - 1) / cus;
+    if (per_cu > 2ull * f.resident && p.k > 512) continue;
+    const double t = kwaves_time(f, p, cus);
+    if (t < best_time) {
+      best = i;
+      best_time = t;
+    }
+  }
+  return best;
+}
+} // namespace cumpsgemm_amd

@@ -1,0 +1,98 @@
+"""Small products: the kernel whose waves share out K.  Edges: tiles that end at the edge of C, that
+start inside the one before and that are larger than C, fewer K-steps than waves, a K that ends inside a
+step in each of the waves.  Once with integers and NaN between and behind the matrices (exact), once with
+operands that fill every plane."""
+import numpy as np
+import pytest
+
+from cumpsgemm_amd import inputs
+from gpu_util import C, N, T, oracle_gemm, rel_diff, run_gemm
+from test_gpu_ragged_k import FP16TC, FP16TCEC, TF32TC, TF32TCEC, _padded_ints
+
+pytestmark = pytest.mark.gpu
+FP32, AUTO, SCALING = 12, 9, 11
+KWAVES = 6  # module id
+
+LAYOUTS = [(False, N, N), (False, T, N), (False, N, T), (False, T, T), (True, N, N), (True, C, N), (True, N, C), (True, T, T)]
+# (form 1: 64 x 64, four waves, 2: 32 x 32, eight, 3: 32 x 32, four; complex 1: 32 x 32, 2: 64 x 32; 32 K-values a step)
+SIZES = [(64, 64, 1), (65, 129, 31), (70, 100, 33), (127, 64, 128), (96, 65, 160), (129, 70, 257), (64, 130, 995), (200, 90, 64)]
+NARROWER = [(1, 1, 40), (31, 5, 33), (40, 17, 300)]  # than a tile: K-contiguous operands only
+
+
+def _sizes(opa, opb):
+    return SIZES + [s for s in NARROWER if opa != N and opb == N]
+
+
+@pytest.mark.parametrize("mode", [FP16TCEC, TF32TCEC, FP16TC, TF32TC])
+@pytest.mark.parametrize("cplx,opa,opb", LAYOUTS)
+@pytest.mark.parametrize("form", [1, 2, 3])
+def test_small_products_are_exact_on_integers(O, handle, dev, monkeypatch, mode, cplx, opa, opb, form):
+    monkeypatch.setenv("CUMPSGEMM_KWAVES", str(form))
+    rng = np.random.default_rng(5)
+    served = 0
+    for m, n, k in _sizes(opa, opb):
+        a, lda = _padded_ints(rng, opa, m, k, 3, cplx)
+        b, ldb = _padded_ints(rng, opb, k, n, 1, cplx)
+        beta = float(rng.integers(0, 2))
+        c0 = rng.integers(-9, 10, m * n).astype(np.complex64 if cplx else np.float32)
+        c, st, mid = run_gemm(handle, dev, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, beta, c0.copy(), m, cplx,
+                              want_module_id=True)
+        assert st == 0
+        served += mid == KWAVES
+        # |x| <= 30: one plane holds the values, every partial sum is an integer below 2^24
+        co = oracle_gemm(O, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, beta, c0.copy(), m)
+        assert np.array_equal(c, co), (m, n, k, beta)
+    forms = 3 if not cplx else 1 if mode == TF32TCEC else 2
+    assert served == (len(_sizes(opa, opb)) if form <= forms else 0)
+
+
+@pytest.mark.parametrize("mode", [FP16TCEC, TF32TCEC])
+@pytest.mark.parametrize("cplx,opa,opb", LAYOUTS)
+@pytest.mark.parametrize("form", [1, 2, 3])
+def test_small_products_with_correction_terms(O, handle, dev, monkeypatch, mode, cplx, opa, opb, form):
+    """Batches with gaps, alpha, beta, a padded C."""
+    monkeypatch.setenv("CUMPSGEMM_KWAVES", str(form))
+    gen = inputs.complex_normal if cplx else inputs.uniform
+    alpha, beta = (0.75 - 0.5j, -0.5 + 0.25j) if cplx else (0.75, -0.5)
+    for m, n, k, batch in ((64, 64, 500, 1), (101, 77, 129, 3), (130, 66, 1000, 2)):
+        ra, ca = (m, k) if opa == N else (k, m)
+        rb, cb = (k, n) if opb == N else (n, k)
+        lda, ldb, ldc = ra + 1, rb + 2, m + 3
+        sa, sb, sc = lda * ca + 5, ldb * cb + 3, ldc * n + 7
+        a, b, c0 = gen(81, sa * batch), gen(82, sb * batch), gen(83, sc * batch)
+        da, db, dc = dev.up(a), dev.up(b), dev.up(c0)
+        st = handle.gemm_strided_batch(opa, opb, m, n, k, alpha, da, lda, sa, db, ldb, sb, beta, dc, ldc, sc, batch, mode,
+                                       cplx=cplx)
+        assert st == 0
+        out = dev.down(dc, np.complex64 if cplx else np.float32)
+        for i in range(batch):
+            ai, bi, ci, x = a[i * sa:][:lda * ca], b[i * sb:][:ldb * cb], c0[i * sc:][:ldc * n], out[i * sc:][:ldc * n]
+            ref = O.gemm_fp64(opa, opb, m, n, k, alpha, ai, lda, bi, ldb, beta, ci, ldc)
+            cf = oracle_gemm(O, FP32, opa, opb, m, n, k, alpha, ai, lda, bi, ldb, beta, ci, ldc)
+            co = oracle_gemm(O, mode, opa, opb, m, n, k, alpha, ai, lda, bi, ldb, beta, ci, ldc)
+            # (bars as for the tiled kernels: twice FP32's error; the same products in another order)
+            assert O.residual(ref, x, m, n, ldc) <= 2.0 * O.residual(ref, cf, m, n, ldc) + 2.0 ** -24
+            assert rel_diff(x, co, m, n, ldc) <= 4 * 2.0 ** -24 * np.sqrt(k)
+            assert np.array_equal(x.reshape(n, ldc)[:, m:], ci.reshape(n, ldc)[:, m:])
+            assert np.array_equal(out[i * sc + ldc * n:(i + 1) * sc], c0[i * sc + ldc * n:(i + 1) * sc])
+
+
+@pytest.mark.parametrize("mode,exponent", [(SCALING, 40), (AUTO, 40), (AUTO, 0)])
+@pytest.mark.parametrize("cplx,opa,opb", LAYOUTS)
+def test_small_products_scaled_and_gated(handle, dev, monkeypatch, mode, exponent, cplx, opa, opb):
+    """Integers times 2^40 (A) and 2^-40 (B): exact in either mode that AUTO may decide for; with the form forced the
+    result is that of the tiled kernels bit for bit."""
+    rng = np.random.default_rng(8)
+    for m, n, k in ((64, 64, 31), (130, 100, 127), (96, 70, 300)):
+        a, lda = _padded_ints(rng, opa, m, k, 0, cplx)
+        b, ldb = _padded_ints(rng, opb, k, n, 0, cplx)
+        s = np.float32(2.0 ** exponent)
+        outs = []
+        for form in ("1", "2", "0"):
+            monkeypatch.setenv("CUMPSGEMM_KWAVES", form)
+            da, db, dc = dev.up(a * s), dev.up(b / s), dev.up(np.full(m * n, np.nan, np.complex64 if cplx else np.float32))
+            st, _ = handle.gemm_pipeline(opa, opb, m, n, k, 1.0, da, lda, db, ldb, 0.0, dc, m, mode, cplx=cplx)
+            assert st == 0
+            outs.append(dev.down(dc, np.complex64 if cplx else np.float32))
+        assert np.isfinite(outs[0].view(np.float32)).all()
+        assert np.array_equal(outs[0], outs[2]) and np.array_equal(outs[1], outs[2])

@@ -1,0 +1,73 @@
+"""The rule that sends small products to their kernel (csrc/kwaves_rule.hpp), compiled for the host: what
+it takes, the kernel can serve and a launch can hold; nothing else reaches the kernel, whatever is asked for."""
+import ctypes
+import itertools
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cumpsgemm_amd", "csrc")
+CUS = 256
+u64 = ctypes.c_uint64
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rule")
+    (d / "rule.cpp").write_text("""
+        #include "kwaves_rule.hpp"
+        using namespace cumpsgemm_amd;
+        extern "C" int form(int prec, int cplx, int a_kc, int b_kc, uint64_t m, uint64_t n, uint64_t k, uint64_t batch,
+                            uint64_t lda, uint64_t ldb, double steps, int split, int asked, int *tile) {
+          const KWavesProblem p{cplx != 0, a_kc != 0, b_kc != 0, m, n, k, batch, lda, ldb};
+          const int f = choose_kwaves_form(prec, p, 256, steps, split != 0, asked);
+          if (f >= 0) {
+            const KWavesForm &x = kwaves_model(prec, p.cplx).form[f];
+            tile[0] = x.bm, tile[1] = x.bn, tile[2] = x.waves;
+          }
+          return f;
+        }""")
+    so = d / "rule.so"
+    subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, "-o", str(so), str(d / "rule.cpp")])
+    lib = ctypes.CDLL(str(so))
+
+    def call(prec, cplx, op, m, n, k, batch=1, pad=0, steps=1e9, split=False, asked=-1):
+        """(form, bm, bn, waves) or None"""
+        lda, ldb = (m if op[0] == "N" else k) + pad, (k if op[1] == "N" else n) + pad
+        tile = (ctypes.c_int * 3)()
+        f = lib.form(prec, int(cplx), int(op[0] != "N"), int(op[1] == "N"), u64(m), u64(n), u64(k), u64(batch), u64(lda),
+                     u64(ldb), ctypes.c_double(steps), int(split), asked, tile)
+        return (f, *tile) if f >= 0 else None
+    return call
+
+
+@pytest.mark.parametrize("asked", [-1, 1, 2, 3])
+def test_what_the_rule_takes_can_be_served(rule, asked):
+    sizes = (1, 31, 32, 63, 64, 65, 1000, 1 << 20, (1 << 26) + 1, (1 << 31) - 1)
+    taken = 0
+    for prec, cplx, op in itertools.product(range(4), (False, True), ("NN", "TN", "NT", "TT")):
+        for m, n, k, batch, pad in itertools.product(sizes, sizes, (1, 33, 1000, (1 << 31) - 1), (1, 65535), (0, 3)):
+            p = rule(prec, cplx, op, m, n, k, batch, pad, asked=asked)
+            if p is None:
+                continue
+            taken += 1
+            _, bm, bn, waves = p
+            # a row-contiguous operand's tile lies inside the matrix
+            assert (op[0] != "N" or m >= bm) and (op[1] == "N" or n >= bn)
+            # HIP refuses 2^32 threads or more along an axis; byte offsets inside a tile are 31 bits
+            assert -(-m // bm) * -(-n // bn) * batch * waves * 64 < 1 << 32
+            es = 8 if cplx else 4
+            lda, ldb = (m if op[0] == "N" else k) + pad, (k if op[1] == "N" else n) + pad
+            for kc, rows, ld in ((op[0] != "N", bm, lda), (op[1] == "N", bn, ldb)):
+                assert ((rows - 1) * ld + 32 if kc else 31 * ld + rows) * es < 1 << 31
+    assert taken > 1000
+
+
+def test_the_rule_compares_with_the_tiled_plan(rule):
+    for prec, cplx in itertools.product(range(4), (False, True)):
+        assert rule(prec, cplx, "NN", 512, 512, 512) is not None                       # the tiled kernels take for ever
+        assert rule(prec, cplx, "NN", 512, 512, 512, steps=0.0) is None                # no time at all
+        assert rule(prec, cplx, "NN", 512, 512, 512, asked=0) is None                  # switched off
+        assert rule(prec, cplx, "NN", 512, 512, 0) is None                             # nothing to multiply
+        assert rule(prec, cplx, "NN", 8192, 8192, 8192) is None                        # too large for small tiles
