@@ -5,7 +5,7 @@
 
 namespace cumpsgemm_amd {
 
-constexpr int kKWavesForms = 3; // tiles per precision, real or complex
+constexpr int kKWavesForms = 4; // tiles per precision, real or complex
 constexpr unsigned kKWavesModuleId = 6;
 
 // Tile and waves of a form, workgroups that a CU holds at once, and the time of a
@@ -18,12 +18,18 @@ struct KWavesForm {
 // ... and what the plan of the tiled kernels takes: us = tiled0 + tiled_per_step *
 // cost, the plan's cost in K-steps of a 256 x 128 tile, + tiled_split if K is split.
 //
-// All of it fitted on 128 products (84 real, m and n 64 - 4096, K 64 - 8192, 44
-// complex, half as large; four layouts, padded, with and without C), each timed with
-// every form and tiled, in every precision.  The form that the fit picks takes 1.9 %
-// (real) and 0.4 % (complex) longer than the fastest; times of all products with
-// the rule over times without: FP16TCEC 0.81 / 0.64 (real / complex), bf16x3
-// 0.80 / 0.59, FP16TC 0.76 / 0.64, bf16x2 0.80 / 0.64.
+// All of it fitted on 188 products (84 real, m and n 64 - 4096, K 64 - 8192, 60 real
+// batches of up to 1024 matrices of 32 - 640, 44 complex; four layouts, padded, with
+// and without C), each timed with every form and tiled, in every precision.  Times of
+// all products with the rule over times without, and what picking the faster side by
+// hindsight would give:      real          real batches     complex
+//   FP16TCEC             0.81 (0.79)     0.84 (0.81)     0.64 (0.63)
+//   bf16x3               0.80 (0.78)     0.83 (0.81)     0.59 (0.59)
+//   FP16TC               0.76 (0.74)     0.84 (0.80)     0.64 (0.64)
+//   bf16x2               0.80 (0.78)     0.83 (0.81)     0.64 (0.64)
+// (Tried beside these and left out, within 1 %: 64 x 32 and 32 x 64 with four and
+// eight waves, 64 x 64 with one and two; 128 x 64 spills.  Complex with one or two
+// waves: batches are faster tiled.)
 struct KWavesModel {
   KWavesForm form[kKWavesForms];
   double tiled0, tiled_per_step, tiled_split;
@@ -31,15 +37,15 @@ struct KWavesModel {
 // `prec`: 0 FP16TCEC, 1 FP16TC, 2 bf16x3, 3 bf16x2
 inline const KWavesModel &kwaves_model(int prec, bool cplx) {
   static const KWavesModel real[4] = {
-      {{{64, 64, 4, 1, 3.3, 0.97, 0.0}, {32, 32, 8, 2, 0.90, 0.90, 0.79}, {32, 32, 4, 4, 0.76, 0.51, 0.76}}, 4.4, 1.50, -1.7},
-      {{{64, 64, 4, 1, 2.2, 0.79, 0.0}, {32, 32, 8, 2, 0.77, 0.89, 0.58}, {32, 32, 4, 4, 0.75, 0.48, 0.66}}, 4.9, 1.12, 1.6},
-      {{{64, 64, 4, 1, 3.3, 1.68, 0.0}, {32, 32, 8, 1, 1.50, 1.20, 0.0}, {32, 32, 4, 3, 1.12, 0.78, 0.53}}, 2.2, 2.16, -1.5},
-      {{{64, 64, 4, 1, 3.3, 1.00, 0.0}, {32, 32, 8, 2, 0.92, 0.88, 0.83}, {32, 32, 4, 4, 0.79, 0.52, 0.74}}, 4.0, 1.53, -1.0}};
+      {{{64, 64, 4, 1, 3.6, 0.93, 0.0}, {32, 32, 8, 2, 1.13, 0.88, 0.71}, {32, 32, 4, 4, 1.08, 0.50, 0.74}, {32, 32, 1, 16, 2.4, 0.37, 0.22}}, 4.1, 1.63, -2.1},
+      {{{64, 64, 4, 1, 3.0, 0.72, 0.0}, {32, 32, 8, 2, 0.98, 0.87, 0.55}, {32, 32, 4, 4, 1.00, 0.47, 0.67}, {32, 32, 1, 16, 2.4, 0.23, 0.37}}, 4.8, 1.27, 0.9},
+      {{{64, 64, 4, 1, 3.6, 1.65, 0.0}, {32, 32, 8, 1, 1.62, 1.17, 0.0}, {32, 32, 4, 3, 1.29, 0.76, 0.55}, {32, 32, 1, 12, 2.2, 0.68, 0.17}}, 2.5, 2.29, -2.4},
+      {{{64, 64, 4, 1, 3.7, 0.95, 0.0}, {32, 32, 8, 2, 1.12, 0.87, 0.78}, {32, 32, 4, 4, 1.09, 0.50, 0.73}, {32, 32, 1, 16, 2.5, 0.39, 0.21}}, 4.0, 1.61, -1.6}};
   static const KWavesModel complex[4] = {
-      {{{32, 32, 4, 1, 2.2, 1.02, 0.0}, {64, 32, 4, 1, 3.5, 1.67, 0.0}, {}}, 2.8, 2.05, -5.4},
-      {{{32, 32, 4, 1, 1.8, 0.74, 0.0}, {64, 32, 4, 1, 2.2, 1.12, 0.0}, {}}, 3.6, 1.50, -3.4},
-      {{{32, 32, 4, 1, 2.3, 1.71, 0.0}, {}, {}}, 0.9, 3.83, -14.3},
-      {{{32, 32, 4, 1, 2.2, 1.06, 0.0}, {64, 32, 4, 1, 3.7, 1.72, 0.0}, {}}, 3.1, 2.09, -6.1}};
+      {{{32, 32, 4, 1, 2.2, 1.02, 0.0}, {64, 32, 4, 1, 3.5, 1.67, 0.0}, {}, {}}, 2.8, 2.05, -5.4},
+      {{{32, 32, 4, 1, 1.8, 0.74, 0.0}, {64, 32, 4, 1, 2.2, 1.12, 0.0}, {}, {}}, 3.6, 1.50, -3.4},
+      {{{32, 32, 4, 1, 2.3, 1.71, 0.0}, {}, {}, {}}, 0.9, 3.83, -14.3},
+      {{{32, 32, 4, 1, 2.2, 1.06, 0.0}, {64, 32, 4, 1, 3.7, 1.72, 0.0}, {}, {}}, 3.1, 2.09, -6.1}};
   return (cplx ? complex : real)[prec];
 }
 

@@ -14,7 +14,7 @@ FP32, AUTO, SCALING = 12, 9, 11
 KWAVES = 6  # module id
 
 LAYOUTS = [(False, N, N), (False, T, N), (False, N, T), (False, T, T), (True, N, N), (True, C, N), (True, N, C), (True, T, T)]
-# (form 1: 64 x 64, four waves, 2: 32 x 32, eight, 3: 32 x 32, four; complex 1: 32 x 32, 2: 64 x 32; 32 K-values a step)
+# (form 1: 64 x 64, four waves, 2, 3, 4: 32 x 32, eight, four, one; complex 1: 32 x 32, 2: 64 x 32; 32 K-values a step)
 SIZES = [(64, 64, 1), (65, 129, 31), (70, 100, 33), (127, 64, 128), (96, 65, 160), (129, 70, 257), (64, 130, 995), (200, 90, 64)]
 NARROWER = [(1, 1, 40), (31, 5, 33), (40, 17, 300)]  # than a tile: K-contiguous operands only
 
@@ -25,7 +25,7 @@ def _sizes(opa, opb):
 
 @pytest.mark.parametrize("mode", [FP16TCEC, TF32TCEC, FP16TC, TF32TC])
 @pytest.mark.parametrize("cplx,opa,opb", LAYOUTS)
-@pytest.mark.parametrize("form", [1, 2, 3])
+@pytest.mark.parametrize("form", [1, 2, 3, 4])
 def test_small_products_are_exact_on_integers(O, handle, dev, monkeypatch, mode, cplx, opa, opb, form):
     monkeypatch.setenv("CUMPSGEMM_KWAVES", str(form))
     rng = np.random.default_rng(5)
@@ -42,13 +42,13 @@ def test_small_products_are_exact_on_integers(O, handle, dev, monkeypatch, mode,
         # |x| <= 30: one plane holds the values, every partial sum is an integer below 2^24
         co = oracle_gemm(O, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, beta, c0.copy(), m)
         assert np.array_equal(c, co), (m, n, k, beta)
-    forms = 3 if not cplx else 1 if mode == TF32TCEC else 2
+    forms = 4 if not cplx else 1 if mode == TF32TCEC else 2
     assert served == (len(_sizes(opa, opb)) if form <= forms else 0)
 
 
 @pytest.mark.parametrize("mode", [FP16TCEC, TF32TCEC])
 @pytest.mark.parametrize("cplx,opa,opb", LAYOUTS)
-@pytest.mark.parametrize("form", [1, 2, 3])
+@pytest.mark.parametrize("form", [1, 2, 3, 4])
 def test_small_products_with_correction_terms(O, handle, dev, monkeypatch, mode, cplx, opa, opb, form):
     """Batches with gaps, alpha, beta, a padded C."""
     monkeypatch.setenv("CUMPSGEMM_KWAVES", str(form))

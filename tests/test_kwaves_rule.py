@@ -42,7 +42,7 @@ def rule(tmp_path_factory):
     return call
 
 
-@pytest.mark.parametrize("asked", [-1, 1, 2, 3])
+@pytest.mark.parametrize("asked", [-1, 1, 2, 3, 4])
 def test_what_the_rule_takes_can_be_served(rule, asked):
     sizes = (1, 31, 32, 63, 64, 65, 1000, 1 << 20, (1 << 26) + 1, (1 << 31) - 1)
     taken = 0
