@@ -30,6 +30,41 @@ struct Acc {
   unsigned under;
 };
 
+// Sum / maximum over the 64 lanes of a wave, in every lane of the result, by DPP moves: within the rows of 16 lanes
+// (shifts by 1, 2, 4, 8: lane 15 of a row has the row), then row 0 into 1 and 2 into 3, then the lower half into the
+// upper (lane 63 has all).  A lane whose source does not exist takes 0, the neutral element of both: maxima are bits of
+// non-negative floats.  Six moves of ~ 8 clocks; a shuffle goes through the LDS pipe and takes ~ 64 (see the kernel).
+template <int CTRL, int ROWS> __device__ inline uint32_t dpp_move(const uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+}
+template <class F> __device__ inline void wave_steps(F &&f) {
+  f(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{}); // row_shr:1
+  f(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+  f(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+  f(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+  f(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{}); // row_bcast:15 into rows 1 and 3
+  f(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{}); // row_bcast:31 into rows 2 and 3
+}
+__device__ inline uint32_t wave_max(uint32_t x) {
+  wave_steps([&](auto ctrl, auto rows) {
+    const uint32_t y = dpp_move<decltype(ctrl)::value, decltype(rows)::value>(x);
+    x = y > x ? y : x;
+  });
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+__device__ inline uint32_t wave_sum(uint32_t x) {
+  wave_steps([&](auto ctrl, auto rows) { x += dpp_move<decltype(ctrl)::value, decltype(rows)::value>(x); });
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+__device__ inline unsigned long long wave_sum(unsigned long long x) {
+  wave_steps([&](auto ctrl, auto rows) {
+    constexpr int C = decltype(ctrl)::value, R = decltype(rows)::value;
+    x += (unsigned long long)dpp_move<C, R>((uint32_t)(x >> 32)) << 32 | dpp_move<C, R>((uint32_t)x);
+  });
+  return (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), 63) << 32 |
+         (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
 __device__ inline void count_one(Acc &a, float x, float ignore_thr, float under_thr) {
   const float ax = fabsf(x);
   a.mx = fmaxf(a.mx, ax); // NaN operands are ignored
@@ -113,6 +148,10 @@ __device__ inline void finish_pair_job(int *flag_out, unsigned *pair_ticket, Sta
   __hip_atomic_store(pair_ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// What bounds a small matrix is a chain: kernel arguments, data, reductions, record, ticket, records, slot, each a round
+// trip of ~ 0.7 us or a row of dependent lane moves.  With DPP moves instead of shuffles, the records folded by one wave,
+// no counts where only the maximum is asked for and no hand-over in a job of one workgroup: FP16TCEC_SCALING calls, us,
+// 128^3 11.7 -> 9.4, 180^3 12.6 -> 9.5, 512^3 12.6 -> 9.8, 1024^3 21.9 -> 20.0 (two launches take 9.3 whatever they do).
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void exp_stats_kernel(const StatsJob job0, const StatsJob job1,
                                                            float ignore_thr, float under_thr,
@@ -191,43 +230,40 @@ __global__ __launch_bounds__(kBlock) void exp_stats_kernel(const StatsJob job0, 
     }
   }
 
-  // wave64 butterfly
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    acc.mx = fmaxf(acc.mx, __shfl_xor(acc.mx, off, 64));
-    acc.total += __shfl_xor(acc.total, off, 64);
-    acc.under += __shfl_xor(acc.under, off, 64);
-  }
-  __shared__ float s_mx[kBlock / 64];
-  __shared__ unsigned s_total[kBlock / 64], s_under[kBlock / 64];
+  // Per wave, then per workgroup.  (MODE 2 needs the maximum only, MODE 1 the counts.)
+  constexpr bool MAX = MODE != 1, COUNTS = MODE != 2;
+  __shared__ unsigned s_mx[kWaves], s_total[kWaves], s_under[kWaves];
   __shared__ bool s_last;
+  const unsigned wave_mx = MAX ? wave_max(__float_as_uint(acc.mx)) : 0u;
+  const unsigned wave_total = COUNTS ? wave_sum(acc.total) : 0u, wave_under = COUNTS ? wave_sum(acc.under) : 0u;
   if ((tid & 63) == 0) {
-    s_mx[tid >> 6] = acc.mx;
-    s_total[tid >> 6] = acc.total;
-    s_under[tid >> 6] = acc.under;
+    s_mx[tid >> 6] = wave_mx;
+    s_total[tid >> 6] = wave_total;
+    s_under[tid >> 6] = wave_under;
   }
   __syncthreads();
+  unsigned mxb = 0;
+  unsigned long long t = 0, u = 0;
   if (tid < 64) {
-    // first wave: fold the per-wave results with a second butterfly
-    float mx = tid < kWaves ? s_mx[tid] : 0.0f;
-    unsigned long long t = tid < kWaves ? s_total[tid] : 0ull;
-    unsigned long long u = tid < kWaves ? s_under[tid] : 0ull;
-#pragma unroll
-    for (int off = kWaves / 2; off >= 1; off >>= 1) {
-      mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-      t += __shfl_xor(t, off, 64);
-      u += __shfl_xor(u, off, 64);
+    if (MAX) mxb = wave_max(tid < kWaves ? s_mx[tid] & 0x7f800000u : 0u);
+    if (COUNTS) {
+      t = wave_sum((unsigned long long)(tid < kWaves ? s_total[tid] : 0u));
+      u = wave_sum((unsigned long long)(tid < kWaves ? s_under[tid] : 0u));
     }
+  }
+  // A job of one workgroup has nothing to hand over: it saves three round trips to memory.
+  if (nblocks > 1) {
     if (tid == 0) {
       // Publish the partial record with device-scope (write-through) stores, wait
       // for them to be acknowledged, then take a ticket.  A device-scope release
       // fence here instead would write back the whole L2 once per workgroup, and
       // those write-backs serialise: they cost several times the streaming loop.
       StatsPartial *p = partials + bid;
-      __hip_atomic_store(&p->max_bits, __float_as_uint(mx) & 0x7f800000u, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(&p->total, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(&p->underflow, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&p->max_bits, mxb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (COUNTS) {
+        __hip_atomic_store(&p->total, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&p->underflow, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
 #if CUMPSGEMM_STATS_STRICT_ORDER
       // the portable form: the ticket is a release / acquire operation at device scope
       const unsigned arrived =
@@ -240,51 +276,31 @@ __global__ __launch_bounds__(kBlock) void exp_stats_kernel(const StatsJob job0, 
 #endif
       s_last = (arrived == nblocks - 1);
     }
-  }
-  __syncthreads();
-  if (!s_last) return;
+    __syncthreads();
+    if (!s_last || tid >= 64) return;
 
-  // last workgroup: fold all partials (device-scope loads, independent of each
-  // other so that they are all in flight together).  No fence is needed: every
-  // partial was acknowledged by memory before its workgroup took a ticket, the
-  // last ticket was taken before the barrier above, and device-scope loads do
-  // not look at this XCD's L2.
-  unsigned mxb = 0;
-  unsigned long long t = 0, u = 0;
-  for (unsigned i = tid; i < nblocks; i += kBlock) {
-    StatsPartial *p = partials + i;
-    const unsigned b = __hip_atomic_load(&p->max_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long pt = __hip_atomic_load(&p->total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long pu = __hip_atomic_load(&p->underflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    mxb = b > mxb ? b : mxb;
-    t += pt;
-    u += pu;
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const unsigned ob = __shfl_xor(mxb, off, 64);
-    mxb = ob > mxb ? ob : mxb;
-    t += __shfl_xor(t, off, 64);
-    u += __shfl_xor(u, off, 64);
-  }
-  __shared__ unsigned r_mx[kBlock / 64];
-  __shared__ unsigned long long r_t[kBlock / 64], r_u[kBlock / 64];
-  if ((tid & 63) == 0) {
-    r_mx[tid >> 6] = mxb;
-    r_t[tid >> 6] = t;
-    r_u[tid >> 6] = u;
-  }
-  __syncthreads();
-  if (tid >= 64) return;
-  mxb = tid < kWaves ? r_mx[tid] : 0u;
-  t = tid < kWaves ? r_t[tid] : 0ull;
-  u = tid < kWaves ? r_u[tid] : 0ull;
-#pragma unroll
-  for (int off = kWaves / 2; off >= 1; off >>= 1) {
-    const unsigned ob = __shfl_xor(mxb, off, 64);
-    mxb = ob > mxb ? ob : mxb;
-    t += __shfl_xor(t, off, 64);
-    u += __shfl_xor(u, off, 64);
+    // last workgroup: its first wave folds all partials (device-scope loads,
+    // independent of each other so that they are all in flight together).  No fence
+    // is needed: every partial was acknowledged by memory before its workgroup took
+    // a ticket, the last ticket was taken before the barrier above, and
+    // device-scope loads do not look at this XCD's L2.
+    mxb = 0;
+    t = 0, u = 0;
+#pragma unroll 4
+    for (unsigned i = tid; i < nblocks; i += 64) {
+      StatsPartial *p = partials + i;
+      const unsigned b = __hip_atomic_load(&p->max_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      mxb = b > mxb ? b : mxb;
+      if (COUNTS) {
+        t += __hip_atomic_load(&p->total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        u += __hip_atomic_load(&p->underflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    if (MAX) mxb = wave_max(mxb);
+    if (COUNTS) {
+      t = wave_sum(t);
+      u = wave_sum(u);
+    }
   }
   if (tid == 0) {
     if (MODE == 0) {
@@ -313,7 +329,7 @@ __global__ __launch_bounds__(kBlock) void exp_stats_kernel(const StatsJob job0, 
     }
     // ready for the next pass on this stream
     // (the slot and the ticket become visible to later kernels at the end of this one)
-    __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (nblocks > 1) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (MODE == 1 && flag_out != nullptr) finish_pair_job(flag_out, pair_ticket, job0.slot, job1.slot);
   }
 }
@@ -342,7 +358,9 @@ View make_view(const cuMpSGEMM_handle *h, unsigned m, unsigned n, unsigned ld, u
   unsigned long long blocks;
   if (dense_cols && dense_batch) {
     v.count_f = total_f;
-    blocks = (total_f / 4 + kBlock * 4 - 1) / (kBlock * 4);
+    // 64 KiB a workgroup; up to 128 KiB one, which has nothing to hand over (two round trips more
+    // to read it, three fewer to publish)
+    blocks = total_f <= 8ull * 4 * kBlock ? 1 : (total_f / 4 + kBlock * 4 - 1) / (kBlock * 4);
   } else {
     v.count_f = 0;
     blocks = ((unsigned long long)n * v.nbatch + kWaves - 1) / kWaves;
