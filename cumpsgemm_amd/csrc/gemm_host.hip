@@ -1021,14 +1021,15 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
       // At most one small workgroup per CU: its four waves, one per SIMD, are
       // bound by the latency of their own chain of LDS reads, MFMAs and staging,
       // so the form with two wave groups (a K-slice of every step each) is
-      // launched -- where it was measured faster: an operand K-contiguous and a
-      // mode with correction terms or bf16 planes (1024^3, plain -> two groups,
-      // us: FP16TCEC NN 19.3 -> 16.4, TN 16.2 -> 13.8, TT 18.6 -> 16.1, bf16x3 NN
-      // 28.1 -> 21.5, bf16x2 NN 19.7 -> 16.5; complex FP16TCEC NN 38.6 -> 34.5,
-      // bf16x2 38.0 -> 33.5; FP16TC level or slower; op(A) = N with op(B) = T level).
+      // launched -- where it was measured faster: complex or with an operand
+      // K-contiguous, and a mode with correction terms or bf16 planes (1024^3, plain
+      // -> two groups, us: FP16TCEC NN 19.3 -> 16.4, TN 16.2 -> 13.8, TT 18.6 -> 16.1,
+      // bf16x3 NN 28.1 -> 21.5, bf16x2 NN 19.7 -> 16.5; complex FP16TCEC NN 38.6 ->
+      // 30.0, NT 41.9 -> 32.0, bf16x2 NT 41.2 -> 30.9; FP16TC level or slower; real
+      // op(A) = N with op(B) = T level).
       const uint64_t groups = (uint64_t)grid.x * grid.y * grid.z;
       auto launch_groups = launch_plain == e->launch_scaled ? e->launch_scaled_kslices : e->launch_kslices;
-      if (launch_groups != nullptr && groups <= (uint64_t)h->num_cus && (a_kc || b_kc) &&
+      if (launch_groups != nullptr && groups <= (uint64_t)h->num_cus && (CPLX || a_kc || b_kc) &&
           launches[i].p != Prec::FP16TC && !tuning().no_kslices) {
         launch_groups(args, grid, h->stream);
       } else {

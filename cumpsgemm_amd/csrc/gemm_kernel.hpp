@@ -522,14 +522,18 @@ struct tile_loader {
   static constexpr int ES = CPLX ? 2 : 1;
   static constexpr bool PARTIAL = (ROWS * 4) < NT; // fewer units than threads
   // An operand with half as many units as threads: every thread takes
-  // half a unit (4 of its 8 K-values; even threads the lower four, odd threads
-  // the upper four, so that a pair of lanes fills one 16-byte chunk of a plane
-  // and a wave's 8-byte LDS writes cover all banks), so that all waves have the
-  // same work and the K loop no branch around an idle half.
+  // half a unit (4 of its 8 K-values), so that all waves have the same work and
+  // the K loop no branch around an idle half.  Bit HALF_BIT of the thread's number
+  // says which half.  K-contiguous: a pair of lanes reads one unit and fills one
+  // 16-byte chunk of a plane.  Row-contiguous: 16 lanes read 16 consecutive rows and
+  // the next 16 the same rows' other half (with pairs of lanes on two K-lines no two
+  // neighbours read neighbouring addresses: complex 800^3 NN 23.6 -> 22.4 us, real
+  // 1024^3 TT 18.8 -> 17.4).  Both ways 32 lanes' 8-byte LDS writes cover all banks.
   // (HALF_UNITS: the precisions this pays for, measured -- FP16TCEC and bf16x2; the
   // costlier bf16x3 split and the single-product FP16TC kernels keep whole units)
   static constexpr bool HALF = HALF_UNITS && (ROWS * 4 * 2 == NT);
   static_assert(TID0 == 0 || (PARTIAL && !HALF), "TID0: partial tiles of whole units");
+  static constexpr int HALF_BIT = KC ? 0 : 4;
   static constexpr int KV = HALF ? 4 : 8; // K-values a thread handles per unit
 
   // whether this thread stages anything of this operand (wave-uniform)
@@ -539,10 +543,11 @@ struct tile_loader {
   // ... in the register-staged copy of pre-split planes (whole 16-byte chunks)
   __device__ static inline bool copy_active(int tid) { return !PARTIAL || tid < ROWS * 4; }
   // which half of its unit (0 unless HALF)
-  __device__ static inline int half_of(int tid) { return HALF ? (tid & 1) : 0; }
+  __device__ static inline int half_of(int tid) { return HALF ? (tid >> HALF_BIT) & 1 : 0; }
 
   __device__ static inline void unit_coords(int u, int tid, int &row, int &chunk) {
-    const int id = (HALF ? tid >> 1 : tid - TID0) + u * NT;
+    constexpr int BELOW = (1 << HALF_BIT) - 1; // (HALF: the thread's number without the bit that picks the half)
+    const int id = (HALF ? (tid & BELOW) | ((tid >> 1) & ~BELOW) : tid - TID0) + u * NT;
     if constexpr (KC) {
       chunk = id & 3;
       row = id >> 2;
@@ -831,6 +836,27 @@ struct tile_loader {
     }
   }
 
+  // (half units) component C of `store`
+  template <Prec P, bool SCALED, int C>
+  __device__ static inline void store_half_component(const Regs &reg, char *lds_op, int tid, float s, float s2048) {
+    static_assert(HALF && U == 1, "half units");
+    constexpr int NP = prec_traits<P>::NP;
+    int row, chunk;
+    unit_coords(0, tid, row, chunk);
+    f8_t x = reg.v[0][C];
+#pragma unroll
+    for (int j = 4; j < 8; j++) x[j] = 0.0f;
+    u4_t out[NP];
+    if constexpr (SCALED) splitter<P>::run_scaled(x, out, s, s2048);
+    else splitter<P>::run(x, out);
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      typedef uint32_t u2v_t __attribute__((ext_vector_type(2)));
+      *reinterpret_cast<u2v_t *>(lds_op + (C * NP + p) * ROWS * 64 + lds_offset(row, chunk) + half_of(tid) * 8) =
+          u2v_t{out[p][0], out[p][1]};
+    }
+  }
+
   // split and write to LDS: planes laid out [comp][plane][row][chunk]
   // SCALED: the values are multiplied by s (s2048 = s * 2^11) on the way
   template <Prec P, bool SCALED = false>
@@ -1037,6 +1063,11 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void gemm_tcec_kernel(c
   // staging registers: the next tile this wave will split and write to LDS
   typename LA::Regs ra;
   typename LB::Regs rb;
+  // (complex two-wave-group kernels: the step after that one)
+  constexpr bool KS2_AHEAD = Cfg::KS2 && CPLX && LA::HALF && LB::HALF && TM == 1 && TN == 1;
+  struct NoRegs {};
+  std::conditional_t<KS2_AHEAD, typename LA::Regs, NoRegs> ra2;
+  std::conditional_t<KS2_AHEAD, typename LB::Regs, NoRegs> rb2;
 
   // accumulators: [component][main/corr][TN][TM]; MFMA rows run along N and
   // MFMA columns along M so that a lane's 64 outputs of one register are 32
@@ -1660,6 +1691,79 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void gemm_tcec_kernel(c
       gload(0, fast_tag);
     };
     Frags f0, f1;
+    if constexpr (KS2_AHEAD && decltype(fast_tag)::value) {
+      // Two wave groups, complex: a wave's MFMAs of a step in four parts, and beside
+      // each the splitting of one component of one operand of the next step -- MFMAs
+      // in a row keep the vector unit from the SIMD's other wave as well -- with the
+      // loads of the step after that in flight.  What is left bounds a step about
+      // equally: 64 KB of LDS writes and reads, 768 cycles of MFMAs per SIMD and 32 KB
+      // from L2 (all CUs together 10 TB/s).  us, MFMAs after the splitting -> so, and
+      // with row-contiguous half units by 16 lanes: FP16TCEC 600^3 NN 20.8 -> 17.7,
+      // 800^3 NN 26.0 -> 21.4, CN 22.4 -> 21.5, 1000^3 NN 33.5 -> 31.2, NT (two-buffer
+      // kernel before) 42.5 -> 32.8; bf16x2 1000^3 NN 33.0 -> 30.2.
+      auto load = [&](auto &xa, auto &xb, const int kt) {
+        LA::template load_fast<true>(xa, a_tile + (uint64_t)kt * a_kstep, args.lda, offa);
+        LB::template load_fast<true>(xb, b_tile + (uint64_t)kt * b_kstep, args.ldb, offb);
+      };
+      auto mma_part = [&](const Frags &f, auto part) { // a quarter of them: products outside, real products inside
+        auto one = [&](auto x) {
+          constexpr int X = decltype(x)::value, t = X / 4, q = X % 4;
+          constexpr int s = PT::ACC[t], pa = PT::PA[t], pb = PT::PB[t];
+          constexpr int ca = (q == 1 || q == 3) ? 1 : 0, cb = (q == 1 || q == 2) ? 1 : 0;
+          acc[q][s][0][0] = mfma_block<PT::IS_BF16>(f.b[cb][pb][0], f.a[ca][pa][0], acc[q][s][0][0]);
+        };
+        constexpr int X0 = PT::NPROD * decltype(part)::value;
+        one(std::integral_constant<int, X0>{});
+        if constexpr (PT::NPROD > 1) one(std::integral_constant<int, X0 + 1>{});
+        if constexpr (PT::NPROD > 2) one(std::integral_constant<int, X0 + 2>{});
+      };
+      static_assert(PT::NPROD <= 3, "four parts");
+      using i0 = std::integral_constant<int, 0>;
+      using i1 = std::integral_constant<int, 1>;
+      using i2 = std::integral_constant<int, 2>;
+      using i3 = std::integral_constant<int, 3>;
+      // step in buffer `cur`; xa, xb: the next step's operands, then those of step `ahead`
+      auto step = [&](const int cur, auto &xa, auto &xb, const int ahead) {
+        char *const sa = lds + (cur ^ 1) * Cfg::STAGE_BYTES, *const sb = sa + Cfg::A_STAGE_BYTES;
+        Frags f;
+        frag_load(f, cur, 0);
+        mma_part(f, i0{});
+        LA::template store_half_component<P, Cfg::SCALED, 0>(xa, sa, tid, coef_a, coef_a2048);
+        __builtin_amdgcn_sched_barrier(0);
+        mma_part(f, i1{});
+        LA::template store_half_component<P, Cfg::SCALED, 1>(xa, sa, tid, coef_a, coef_a2048);
+        __builtin_amdgcn_sched_barrier(0);
+        mma_part(f, i2{});
+        LB::template store_half_component<P, Cfg::SCALED, 0>(xb, sb, tid, coef_b, coef_b2048);
+        __builtin_amdgcn_sched_barrier(0);
+        mma_part(f, i3{});
+        LB::template store_half_component<P, Cfg::SCALED, 1>(xb, sb, tid, coef_b, coef_b2048);
+        load(xa, xb, clamp(ahead));
+        block_sync_lds();
+      };
+      if (ragged) {
+        gload_tail(last);
+        a_tile -= a_kstep; // (step i >= 1 of the loop is the operands' step i - 1)
+        b_tile -= b_kstep;
+      } else {
+        load(ra, rb, 0);
+      }
+      load(ra2, rb2, clamp(1));
+      lstore(0);
+      load(ra, rb, clamp(2));
+      block_sync_lds();
+      int t = 0;
+      for (; t + 2 < nk; t += 2) {
+        step(0, ra2, rb2, t + 3);
+        step(1, ra, rb, t + 4);
+      }
+      if (t + 1 < nk) {
+        step(0, ra2, rb2, last);
+        t++;
+      }
+      mma_tile(t & 1);
+      return;
+    }
     if constexpr (!Cfg::DEEP) {
       // Double-buffered: every wave multiplies tile t from one LDS buffer,
       // stages tile t+1 into the other and prefetches tile t+2 into registers;

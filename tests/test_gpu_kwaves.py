@@ -96,3 +96,24 @@ def test_small_products_scaled_and_gated(handle, dev, monkeypatch, mode, exponen
             outs.append(dev.down(dc, np.complex64 if cplx else np.float32))
         assert np.isfinite(outs[0].view(np.float32)).all()
         assert np.array_equal(outs[0], outs[2]) and np.array_equal(outs[1], outs[2])
+
+
+@pytest.mark.parametrize("mode", [FP16TCEC, TF32TC, SCALING])
+@pytest.mark.parametrize("opa,opb", [(N, N), (C, N), (N, T), (T, C)])
+def test_complex_two_wave_groups_are_exact_on_integers(O, handle, dev, monkeypatch, mode, opa, opb):
+    """The tiled kernel that complex products of a few tiles take otherwise, its operands loaded two steps
+    ahead: one to six K-steps, with and without a partial one, tiles at the edge and larger than C."""
+    monkeypatch.setenv("CUMPSGEMM_KWAVES", "0")
+    rng = np.random.default_rng(6)
+    for k in (31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 190, 995):
+        for m, n in ((64, 128), (131, 70), (37, 9)):
+            a, lda = _padded_ints(rng, opa, m, k, 3, True)
+            b, ldb = _padded_ints(rng, opb, k, n, 1, True)
+            beta = float(rng.integers(0, 2))
+            c0 = rng.integers(-9, 10, m * n).astype(np.complex64)
+            c, st = run_gemm(handle, dev, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, beta,
+                             c0.copy(), m, True)
+            assert st == 0
+            co = oracle_gemm(O, FP16TCEC if mode == SCALING else mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, beta,
+                             c0.copy(), m)
+            assert np.array_equal(c, co), (m, n, k, beta)
