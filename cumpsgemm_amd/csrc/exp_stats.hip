@@ -1,7 +1,7 @@
 // Exponent statistics: per-matrix max exponent, element count above the
 // "ignore" threshold and count of elements that would underflow the fp16 lo
 // term.  HBM-bound streaming reductions for gfx950: 16-byte loads, wave64
-// butterfly reduction, one partial record per workgroup, and the last
+// reductions by DPP moves, one partial record per workgroup, and the last
 // workgroup to arrive folds the partials and takes the mode decision, so a
 // statistics pass is a single launch with no zero-initialisation step.
 //
@@ -78,6 +78,7 @@ __device__ inline void count_one(Acc &a, float x, float ignore_thr, float under_
 // MODE 1: stage 2 (counts only, thresholds relative to the slot's max exponent;
 //                  runs only if the slot is UNDEFINED)
 // MODE 2: max exponent only
+// MODE 3: stage 1, and stage 2 by the workgroup that took decision 1
 // One matrix to scan: result slot, scratch for the per-workgroup partials,
 // arrival counter, the view of the data and how many workgroups work on it.
 struct StatsJob {
@@ -121,7 +122,7 @@ struct StatsJob {
 #if !CUMPSGEMM_STATS_STRICT_ORDER && defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
 #error "the fence-free hand-over of exp_stats_kernel is written for gfx950; build with -DCUMPSGEMM_STATS_STRICT_ORDER=1"
 #endif
-// Stage 2 of a pair can also write the launch flag that the two decisions
+// Stage 2 of a pair (MODE 1, 3) can also write the launch flag that the two decisions
 // give (flag_out != nullptr; the combination of src/dynamic_scaling.cu:364-385),
 // which saves the one-thread kernel that would otherwise follow, i.e. one more
 // kernel boundary per AUTO call.  Each job has one finishing thread -- thread 0
@@ -151,7 +152,7 @@ __device__ inline void finish_pair_job(int *flag_out, unsigned *pair_ticket, Sta
 // What bounds a small matrix is a chain: kernel arguments, data, reductions, record, ticket, records, slot, each a round
 // trip of ~ 0.7 us or a row of dependent lane moves.  With DPP moves instead of shuffles, the records folded by one wave,
 // no counts where only the maximum is asked for and no hand-over in a job of one workgroup: FP16TCEC_SCALING calls, us,
-// 128^3 11.7 -> 9.4, 180^3 12.6 -> 9.5, 512^3 12.6 -> 9.8, 1024^3 21.9 -> 20.0 (two launches take 9.3 whatever they do).
+// 128^3 11.7 -> 8.2, 180^3 12.6 -> 8.2, 512^3 12.6 -> 9.8, 1024^3 21.9 -> 20.0 (two launches take about 8 whatever they do).
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void exp_stats_kernel(const StatsJob job0, const StatsJob job1,
                                                            float ignore_thr, float under_thr,
@@ -176,81 +177,99 @@ __global__ __launch_bounds__(kBlock) void exp_stats_kernel(const StatsJob job0, 
     ignore_thr *= max_exp;
     under_thr *= max_exp;
   }
-  Acc acc{0.0f, 0u, 0u};
   const unsigned tid = threadIdx.x;
-  if (count_f != 0) {
-    // contiguous data: head up to 16-byte alignment, float4 body, tail
-    const unsigned long long mis = ((16 - ((uintptr_t)ptr & 15)) & 15) / 4;
-    const unsigned long long head = mis < count_f ? mis : count_f;
-    const float4 *body = reinterpret_cast<const float4 *>(ptr + head);
-    const unsigned long long nvec = (count_f - head) / 4;
-    const unsigned long long gsz = (unsigned long long)nblocks * kBlock;
-    unsigned long long i = (unsigned long long)bid * kBlock + tid;
-    auto count4 = [&](const float4 &v) {
-      count_one(acc, v.x, ignore_thr, under_thr); count_one(acc, v.y, ignore_thr, under_thr);
-      count_one(acc, v.z, ignore_thr, under_thr); count_one(acc, v.w, ignore_thr, under_thr);
-    };
-    // Eight independent 16-byte loads in flight per thread.  A workgroup takes
-    // contiguous chunks of 8 * kBlock vectors, so that what the whole grid
-    // streams at any moment is one compact window (windows a power-of-two
-    // stride apart would fall on the same memory channels).
-    constexpr unsigned long long kChunk = 8ull * kBlock;
-    const unsigned long long nfull = nvec / kChunk;
-    for (unsigned long long c = bid; c < nfull; c += nblocks) {
-      const float4 *cp = body + c * kChunk + tid;
-      float4 v[8];
+  // this workgroup's part, as number `bid` of `nblocks`
+  auto scan = [&](const unsigned bid, const unsigned nblocks) {
+    Acc acc{0.0f, 0u, 0u};
+    if (count_f != 0) {
+      // contiguous data: head up to 16-byte alignment, float4 body, tail
+      const unsigned long long mis = ((16 - ((uintptr_t)ptr & 15)) & 15) / 4;
+      const unsigned long long head = mis < count_f ? mis : count_f;
+      const float4 *body = reinterpret_cast<const float4 *>(ptr + head);
+      const unsigned long long nvec = (count_f - head) / 4;
+      const unsigned long long gsz = (unsigned long long)nblocks * kBlock;
+      unsigned long long i = (unsigned long long)bid * kBlock + tid;
+      auto count4 = [&](const float4 &v) {
+        count_one(acc, v.x, ignore_thr, under_thr); count_one(acc, v.y, ignore_thr, under_thr);
+        count_one(acc, v.z, ignore_thr, under_thr); count_one(acc, v.w, ignore_thr, under_thr);
+      };
+      // Eight independent 16-byte loads in flight per thread.  A workgroup takes
+      // contiguous chunks of 8 * kBlock vectors, so that what the whole grid
+      // streams at any moment is one compact window (windows a power-of-two
+      // stride apart would fall on the same memory channels).
+      constexpr unsigned long long kChunk = 8ull * kBlock;
+      const unsigned long long nfull = nvec / kChunk;
+      for (unsigned long long c = bid; c < nfull; c += nblocks) {
+        const float4 *cp = body + c * kChunk + tid;
+        float4 v[8];
 #pragma unroll
-      for (int j = 0; j < 8; j++) v[j] = cp[j * kBlock];
+        for (int j = 0; j < 8; j++) v[j] = cp[j * kBlock];
 #pragma unroll
-      for (int j = 0; j < 8; j++) count4(v[j]);
-    }
-    i += nfull * kChunk;
-    for (; i < nvec; i += gsz) {
-      count4(body[i]);
-    }
-    if (bid == 0) {
-      if (tid < head) count_one(acc, ptr[tid], ignore_thr, under_thr);
-      const unsigned long long tail0 = head + nvec * 4;
-      if (tail0 + tid < count_f) count_one(acc, ptr[tail0 + tid], ignore_thr, under_thr);
-    }
-  } else {
-    // strided view: one column (of m_f floats) per wave iteration
-    const unsigned long long ncols = (unsigned long long)n * nbatch;
-    const unsigned lane = tid & 63;
-    for (unsigned long long col = (unsigned long long)bid * kWaves + (tid >> 6); col < ncols;
-         col += (unsigned long long)nblocks * kWaves) {
-      const float *cp = ptr + (col / n) * stride_f + (col % n) * ld_f;
-      unsigned i = lane;
-      for (; i + 192 < m_f; i += 256) {
-        const float x0 = cp[i], x1 = cp[i + 64], x2 = cp[i + 128], x3 = cp[i + 192];
-        count_one(acc, x0, ignore_thr, under_thr); count_one(acc, x1, ignore_thr, under_thr);
-        count_one(acc, x2, ignore_thr, under_thr); count_one(acc, x3, ignore_thr, under_thr);
+        for (int j = 0; j < 8; j++) count4(v[j]);
       }
-      for (; i < m_f; i += 64) count_one(acc, cp[i], ignore_thr, under_thr);
+      i += nfull * kChunk;
+      // Less than a chunk is left.  For few workgroups that is several rounds, for one it can be all: their loads in
+      // flight together as well (AUTO 181^3, us: one after the other 17.5, so 11.5).
+      if (nvec - nfull * kChunk > gsz) {
+        float4 v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = body[i + j * gsz < nvec ? i + j * gsz : 0];
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          if (i + j * gsz < nvec) count4(v[j]);
+      } else if (i < nvec) {
+        count4(body[i]);
+      }
+      if (bid == 0) {
+        if (tid < head) count_one(acc, ptr[tid], ignore_thr, under_thr);
+        const unsigned long long tail0 = head + nvec * 4;
+        if (tail0 + tid < count_f) count_one(acc, ptr[tail0 + tid], ignore_thr, under_thr);
+      }
+    } else {
+      // strided view: one column (of m_f floats) per wave iteration
+      const unsigned long long ncols = (unsigned long long)n * nbatch;
+      const unsigned lane = tid & 63;
+      for (unsigned long long col = (unsigned long long)bid * kWaves + (tid >> 6); col < ncols;
+           col += (unsigned long long)nblocks * kWaves) {
+        const float *cp = ptr + (col / n) * stride_f + (col % n) * ld_f;
+        unsigned i = lane;
+        for (; i + 192 < m_f; i += 256) {
+          const float x0 = cp[i], x1 = cp[i + 64], x2 = cp[i + 128], x3 = cp[i + 192];
+          count_one(acc, x0, ignore_thr, under_thr); count_one(acc, x1, ignore_thr, under_thr);
+          count_one(acc, x2, ignore_thr, under_thr); count_one(acc, x3, ignore_thr, under_thr);
+        }
+        for (; i < m_f; i += 64) count_one(acc, cp[i], ignore_thr, under_thr);
+      }
     }
-  }
+    return acc;
+  };
 
   // Per wave, then per workgroup.  (MODE 2 needs the maximum only, MODE 1 the counts.)
   constexpr bool MAX = MODE != 1, COUNTS = MODE != 2;
   __shared__ unsigned s_mx[kWaves], s_total[kWaves], s_under[kWaves];
   __shared__ bool s_last;
-  const unsigned wave_mx = MAX ? wave_max(__float_as_uint(acc.mx)) : 0u;
-  const unsigned wave_total = COUNTS ? wave_sum(acc.total) : 0u, wave_under = COUNTS ? wave_sum(acc.under) : 0u;
-  if ((tid & 63) == 0) {
-    s_mx[tid >> 6] = wave_mx;
-    s_total[tid >> 6] = wave_total;
-    s_under[tid >> 6] = wave_under;
-  }
-  __syncthreads();
-  unsigned mxb = 0;
+  __shared__ bool s_again;    // MODE 3: stage 2 follows ...
+  __shared__ unsigned s_max;  // ... relative to this maximum
+  unsigned mxb = 0;            // of the workgroup, in its first wave
   unsigned long long t = 0, u = 0;
-  if (tid < 64) {
-    if (MAX) mxb = wave_max(tid < kWaves ? s_mx[tid] & 0x7f800000u : 0u);
-    if (COUNTS) {
-      t = wave_sum((unsigned long long)(tid < kWaves ? s_total[tid] : 0u));
-      u = wave_sum((unsigned long long)(tid < kWaves ? s_under[tid] : 0u));
+  auto reduce = [&](const Acc &acc) {
+    const unsigned wave_mx = MAX ? wave_max(__float_as_uint(acc.mx)) : 0u;
+    const unsigned wave_total = COUNTS ? wave_sum(acc.total) : 0u, wave_under = COUNTS ? wave_sum(acc.under) : 0u;
+    if ((tid & 63) == 0) {
+      s_mx[tid >> 6] = wave_mx;
+      s_total[tid >> 6] = wave_total;
+      s_under[tid >> 6] = wave_under;
     }
-  }
+    __syncthreads();
+    if (tid < 64) {
+      if (MAX) mxb = wave_max(tid < kWaves ? s_mx[tid] & 0x7f800000u : 0u);
+      if (COUNTS) {
+        t = wave_sum((unsigned long long)(tid < kWaves ? s_total[tid] : 0u));
+        u = wave_sum((unsigned long long)(tid < kWaves ? s_under[tid] : 0u));
+      }
+    }
+  };
+  reduce(scan(bid, nblocks));
   // A job of one workgroup has nothing to hand over: it saves three round trips to memory.
   if (nblocks > 1) {
     if (tid == 0) {
@@ -277,60 +296,77 @@ __global__ __launch_bounds__(kBlock) void exp_stats_kernel(const StatsJob job0, 
       s_last = (arrived == nblocks - 1);
     }
     __syncthreads();
-    if (!s_last || tid >= 64) return;
+    if (!s_last || (MODE != 3 && tid >= 64)) return;
 
     // last workgroup: its first wave folds all partials (device-scope loads,
     // independent of each other so that they are all in flight together).  No fence
     // is needed: every partial was acknowledged by memory before its workgroup took
     // a ticket, the last ticket was taken before the barrier above, and
     // device-scope loads do not look at this XCD's L2.
-    mxb = 0;
-    t = 0, u = 0;
+    if (tid < 64) {
+      mxb = 0;
+      t = 0, u = 0;
 #pragma unroll 4
-    for (unsigned i = tid; i < nblocks; i += 64) {
-      StatsPartial *p = partials + i;
-      const unsigned b = __hip_atomic_load(&p->max_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      mxb = b > mxb ? b : mxb;
-      if (COUNTS) {
-        t += __hip_atomic_load(&p->total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        u += __hip_atomic_load(&p->underflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (unsigned i = tid; i < nblocks; i += 64) {
+        StatsPartial *p = partials + i;
+        const unsigned b = __hip_atomic_load(&p->max_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        mxb = b > mxb ? b : mxb;
+        if (COUNTS) {
+          t += __hip_atomic_load(&p->total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          u += __hip_atomic_load(&p->underflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
       }
-    }
-    if (MAX) mxb = wave_max(mxb);
-    if (COUNTS) {
-      t = wave_sum(t);
-      u = wave_sum(u);
+      if (MAX) mxb = wave_max(mxb);
+      if (COUNTS) {
+        t = wave_sum(t);
+        u = wave_sum(u);
+      }
     }
   }
   if (tid == 0) {
-    if (MODE == 0) {
+    if (MODE == 0 || MODE == 3) {
       slot->max_exp_bits = mxb;
       const float max_exp = __uint_as_float(mxb);
       // decision 1: counters compared as floats, like the reference's mixed
       // u64 * float expression
-      if (((float)u > (float)t * tolerance) || (max_exp > 0.0f && t == 0)) {
-        slot->mode = CUMPSGEMM_UNDEFINED;
-        slot->total = 0;
-        slot->underflow = 0;
-      } else {
-        slot->mode = CUMPSGEMM_FP16TCEC;
-        slot->total = t;
-        slot->underflow = u;
+      const bool undecided = ((float)u > (float)t * tolerance) || (max_exp > 0.0f && t == 0);
+      slot->total = undecided ? 0 : t;
+      slot->underflow = undecided ? 0 : u;
+      if (MODE == 3) {
+        s_again = undecided;
+        s_max = mxb;
       }
-    } else if (MODE == 1) {
+      // (MODE 3: the slot's mode is stored once, when it is final, and at device scope: the other
+      // job's finishing thread may read it in this launch)
+      if (MODE == 0) slot->mode = undecided ? CUMPSGEMM_UNDEFINED : CUMPSGEMM_FP16TCEC;
+      else if (!undecided)
+        __hip_atomic_store(&slot->mode, (int)CUMPSGEMM_FP16TCEC, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if (MODE == 2) {
+      slot->max_exp_bits = mxb;
+    }
+    // ready for the next pass on this stream
+    // (the slot and the ticket become visible to later kernels at the end of this one)
+    if (nblocks > 1) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if constexpr (MODE == 3) {
+    __syncthreads();
+    if (s_again) {
+      const float max_exp = __uint_as_float(s_max);
+      ignore_thr = ignore_thr / 2 * max_exp;
+      under_thr = under_thr / 2 * max_exp;
+      reduce(scan(0, 1));
+    }
+  }
+  if (tid == 0 && (MODE == 1 || MODE == 3)) {
+    if (MODE == 1 || s_again) {
       slot->total = t;
       slot->underflow = u;
       const int decided = ((float)u <= (float)t * tolerance) ? CUMPSGEMM_FP16TCEC_SCALING
                                                              : CUMPSGEMM_TF32TCEC;
       // (a device-scope store: the other job's finishing thread may read it in this launch)
       __hip_atomic_store(&slot->mode, decided, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-      slot->max_exp_bits = mxb;
     }
-    // ready for the next pass on this stream
-    // (the slot and the ticket become visible to later kernels at the end of this one)
-    if (nblocks > 1) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (MODE == 1 && flag_out != nullptr) finish_pair_job(flag_out, pair_ticket, job0.slot, job1.slot);
+    if (flag_out != nullptr) finish_pair_job(flag_out, pair_ticket, job0.slot, job1.slot);
   }
 }
 
@@ -398,7 +434,13 @@ StatsJob make_job(cuMpSGEMM_handle *h, const View &v, const T *ptr, unsigned slo
   return j;
 }
 
-// MODE 0 + 1 (full statistics) or 2 (maximum only) over one job or two
+// Both stages in one launch: dense matrices of up to 256 KiB.  The second launch takes 1 - 2.5 us whether stage 2
+// is needed or not, one workgroup reads 256 KiB again in about 2.  AUTO calls, us, two launches -> one: 64^3 13.2 ->
+// 10.6, 181^3 17.5 -> 11.5, 256^3 14.3 -> 12.9; with data that need stage 2 128^3 18.3 -> 12.6, 256^3 19.4 -> 18.2,
+// but with 512 KiB a matrix 21.8 -> 24.3 (and strided views are read in smaller pieces: two launches).
+constexpr unsigned long long kOneLaunchFloats = 64 * 1024;
+
+// MODE 0 + 1 or 3 (full statistics) or 2 (maximum only) over one job or two
 template <bool FULL>
 void launch_stats(cuMpSGEMM_handle *h, const StatsJob &j0, const StatsJob &j1, int *flag_out = nullptr) {
   // (a null matrix would fault on the device; an empty one has nothing to read)
@@ -409,7 +451,13 @@ void launch_stats(cuMpSGEMM_handle *h, const StatsJob &j0, const StatsJob &j1, i
     return;
   }
   const dim3 grid(j0.blocks + j1.blocks);
-  if (FULL) {
+  auto once = [](const StatsJob &j) { return j.blocks == 0 || (j.count_f != 0 && j.count_f <= kOneLaunchFloats); };
+  if (FULL && once(j0) && once(j1) && !h->profiler.enabled) { // (the profile names the stages)
+    const bool with_flag = flag_out != nullptr && j0.blocks != 0 && j1.blocks != 0;
+    hipLaunchKernelGGL(exp_stats_kernel<3>, grid, dim3(kBlock), 0, h->stream, j0, j1, h->ignore_threshold,
+                       h->underflow_threshold, h->underflow_tolerance_rate, with_flag ? flag_out : (int *)nullptr,
+                       h->stats_ticket + 2);
+  } else if (FULL) {
     {
       ProfileScope prof(h, "exp_stats_1");
       hipLaunchKernelGGL(exp_stats_kernel<0>, grid, dim3(kBlock), 0, h->stream, j0, j1, h->ignore_threshold,

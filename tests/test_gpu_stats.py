@@ -218,3 +218,33 @@ def test_pair_launch_matches_two_single_launches(O, handle, dev, shapes):
     ja, jb = handle.exp_max_pair(ma, na, da, ma, mb, nb, db, mb)
     assert int(np.float32(handle.get_max_exp(ja)).view(np.uint32)) == oa.max_exp_bits
     assert int(np.float32(handle.get_max_exp(jb)).view(np.uint32)) == ob.max_exp_bits
+
+
+@pytest.mark.parametrize("mode_a", [FP16TCEC, SCALING, TF32TCEC])
+@pytest.mark.parametrize("mode_b", [FP16TCEC, SCALING, TF32TCEC])
+@pytest.mark.parametrize("count", [1, 5, 1024, 4099, 32767, 32768, 32769, 65535, 65536, 65537])
+def test_pairs_at_the_edges_of_one_workgroup_and_one_launch(O, handle, dev, mode_a, mode_b, count):
+    """32768 floats are one workgroup's, up to 65536 both stages are one launch.  Every combination of
+    decisions, matrices at odd addresses, several times over so that tickets left behind would show."""
+    rng = np.random.default_rng(count)
+
+    def data(mode, n):
+        x = rng.uniform(0.5, 1.0, n).astype(np.float32)  # no element below 2^-15
+        if mode == SCALING:
+            return (x * np.float32(2.0 ** -20)).astype(np.float32)
+        if mode == TF32TCEC:
+            x[n // 2:] *= np.float32(2.0 ** -30)  # (one element: 2^-30 of the largest, itself -> scaling)
+        return x
+
+    for na, nb in ((count, count), (count, 300), (7, count)):
+        a, b = data(mode_a, na + 1), data(mode_b, nb + 3)
+        da, db = dev.up(a), dev.up(b)
+        oa, ob = O.exp_stats(a[1:], na, 1, na), O.exp_stats(b[3:], nb, 1, nb)
+        for _ in range(2):
+            flag = handle.get_next_dynamic_launch_buffer_id()
+            ids = handle.exp_stats_pair(na, 1, da.data_ptr() + 4, na, nb, 1, db.data_ptr() + 12, nb, flag_id=flag)
+            for sid, o in zip(ids, (oa, ob)):
+                assert handle.get_exp_stats(sid) == (o.underflow, o.total)
+                assert _bits(handle.get_max_exp(sid)) == o.max_exp_bits
+                assert handle.get_exp_stats_compute_mode_level(sid) == o.mode
+            assert handle.get_dynamic_launch_flag(flag) == O.lib().oracle_combine_flag(oa.mode, ob.mode)
