@@ -969,8 +969,7 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
         set_fused_scaling(args);
       }
       launch(args, dim3(args.tiles_m * args.tiles_n * args.batch, 1, 1), h->stream);
-      // (reported as the small tile class; a form that was asked for by its own id, so that a test can tell)
-      if (used_id != nullptr) *used_id = mode == CUMPSGEMM_AUTO ? ~0u : tuning().kwaves > 0 ? kKWavesModuleId : 2u;
+      if (used_id != nullptr) *used_id = mode == CUMPSGEMM_AUTO ? ~0u : kKWavesModuleId;
       continue;
     }
     Plan plan = (i == 0) ? plan0

@@ -6,7 +6,7 @@
 namespace cumpsgemm_amd {
 
 constexpr int kKWavesForms = 4; // tiles per precision, real or complex
-constexpr unsigned kKWavesModuleId = 6;
+constexpr unsigned kKWavesModuleId = 6; // what used_kernel_module_id reports (0 - 4 are the tile classes, 5 the narrow kernel)
 
 // Tile and waves of a form, workgroups that a CU holds at once, and the time of a
 // tile in us: `fill` for prologue, sums and write-out, `step` per K-step of a wave,

@@ -20,8 +20,8 @@ inline void set_stream(handle_t &handle, hipStream_t stream) {
 
 // reference cumpsgemm.hpp:16-24 (src/cumpsgemm.cu:228-419).
 // used_kernel_module_id receives the index into the gfx950 tile-config table
-// (0 - 4), 5 for the kernel of results with a narrow side, 200 for the pre-split
-// path; + 100 when K was split; ~0u for AUTO.
+// (0 - 4), 5 for the kernel of results with a narrow side, 6 for the kernel of
+// small products, 200 for the pre-split path; + 100 when K was split; ~0u for AUTO.
 template <class T>
 hipblasStatus_t gemm(handle_t handle, hipblasOperation_t op_A,
                      hipblasOperation_t op_B, uint64_t m, uint64_t n, uint64_t k,

@@ -15,8 +15,8 @@ extern "C" {
 
 /* cumpsgemm::gemm<T> with the used_kernel_module_id out-parameter
  * (reference cumpsgemm.hpp:16-24): index into the tile-config table (0 - 4), 5
- * for the kernel of results with a narrow side, 200 for the pre-split path; +100
- * when K was split; ~0u for AUTO. */
+ * for the kernel of results with a narrow side, 6 for the kernel of small
+ * products, 200 for the pre-split path; +100 when K was split; ~0u for AUTO. */
 hipblasStatus_t cuMpSGEMM_sgemm_ex(cuMpSGEMM_handle_t handle, hipblasOperation_t op_A,
                                    hipblasOperation_t op_B, uint64_t m, uint64_t n, uint64_t k,
                                    const float *alpha, const float *a, uint64_t lda,

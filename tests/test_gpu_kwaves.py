@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from cumpsgemm_amd import inputs
-from gpu_util import C, N, T, oracle_gemm, rel_diff, run_gemm
+from gpu_util import C, N, T, make_operand, oracle_gemm, rel_diff, run_gemm
 from test_gpu_ragged_k import FP16TC, FP16TCEC, TF32TC, TF32TCEC, _padded_ints
 
 pytestmark = pytest.mark.gpu
@@ -44,6 +44,20 @@ def test_small_products_are_exact_on_integers(O, handle, dev, monkeypatch, mode,
         assert np.array_equal(c, co), (m, n, k, beta)
     forms = 4 if not cplx else 1 if mode == TF32TCEC else 2
     assert served == (len(_sizes(opa, opb)) if form <= forms else 0)
+
+
+@pytest.mark.parametrize("mode", [FP16TCEC, TF32TCEC, FP16TC, TF32TC])
+@pytest.mark.parametrize("cplx,opa,opb,m,n,k", [(False, N, N, 512, 512, 512), (False, N, T, 128, 128, 128),
+                                                (False, T, T, 1000, 900, 777), (True, N, T, 256, 256, 256),
+                                                (True, C, N, 512, 512, 512)])
+def test_small_products_come_here_and_say_so(handle, dev, mode, cplx, opa, opb, m, n, k):
+    """Without any tuning variable: the rule takes them, the module id names the kernel that ran."""
+    gen = inputs.complex_normal if cplx else inputs.uniform
+    a, lda = make_operand(gen, 1, opa, m, k)
+    b, ldb = make_operand(gen, 2, opb, k, n)
+    c0 = np.zeros(m * n, a.dtype)
+    assert run_gemm(handle, dev, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, 0.0, c0, m, cplx,
+                    want_module_id=True)[1:] == (0, KWAVES)
 
 
 @pytest.mark.parametrize("mode", [FP16TCEC, TF32TCEC])

@@ -18,7 +18,7 @@ def test_cpp_api_client():
     assert r.returncode == 0 and "DONE" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
     res = dict(re.findall(r"RESULT (\S+) (\S+)", r.stdout))
     assert res["sgemm_status"] == "0" and float(res["sgemm_relerr"]) < 2.0 ** -23 * 170 ** 0.5
-    assert res["sgemm_module"] in ("0", "1", "2")                 # a tile class, as in the reference
+    assert res["sgemm_module"] in ("0", "1", "2", "6")   # a tile class, as in the reference, or the small-product kernel
     assert res["cgemm_batch_status"] == "0" and float(res["cgemm_batch_relerr"]) < 2.0 ** -23 * 72 ** 0.5
     assert res["stats_max_ok"] == "1"
     # |x| <= 0.01 with a seventh of the entries near 1e-6: stage 1 sees underflow, stage 2
