@@ -892,8 +892,7 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
   // Small products: K shared out over a workgroup's waves.  (AUTO: both candidates must agree on whether C is
   // prepared and added to, so where the tiled plan splits K either both go this way or neither.)
   int kwaves[2] = {-1, -1};
-  // (CUMPSGEMM_NO_KSLICE_GROUPS asks for the four-wave tiled kernel)
-  if (force_cls < 0 && force_split == 0 && h->ws_override == nullptr && !tuning().no_kslices) {
+  if (force_cls < 0 && force_split == 0 && h->ws_override == nullptr) {
     const KWavesProblem problem{CPLX, a_kc, b_kc, m, n, k, batch, lda, ldb};
     for (int i = 0; i < nlaunch; i++) {
       const Plan tiled = i == 0 ? plan0 : make_plan(h, launches[i].p, CPLX, a_kc, b_kc, m, n, k, batch, -1, 0);

@@ -77,7 +77,7 @@ struct Tuning {
   bool no_edge16_twin = false;   // CUMPSGEMM_NO_EDGE16_TWIN: never the 16x16x32 instance of the large in-loop tile
   int cut_percent = -1;          // CUMPSGEMM_CUT_PERCENT: C is cut when the model prices the two parts below this
                                  // share of the uncut plan (unset: 93, complex 96, complex bf16x3 110)
-  bool no_kslices = false;       // CUMPSGEMM_NO_KSLICE_GROUPS
+  bool no_kslices = false;       // CUMPSGEMM_NO_KSLICE_GROUPS: tiled kernels with one wave group throughout
   bool no_narrow = false;        // CUMPSGEMM_NO_NARROW: results with a narrow side take the tiled kernels
   int kwaves = -1;               // CUMPSGEMM_KWAVES: 0 never, 1 ... the form of the small-product kernel, where it can
                                  // serve the call (gemm_kwaves_*.hip)

@@ -570,23 +570,30 @@ def test_pre_split_path_on_the_whole_rounds_of_a_cut_problem(handle, dev, monkey
 
 
 # ---- small problems: two wave groups per workgroup --------------------------------------
-# A problem of no more small tiles than CUs (an operand K-contiguous) runs the 64 x 64 kernel with twice the waves:
+# A problem of no more small tiles than CUs (complex, or an operand K-contiguous) that the small-product kernel
+# leaves to the tiled ones (here: switched off) runs the 64 x 64 kernel with twice the waves:
 # each group takes one K-slice of every step and the sums meet in LDS at the end.  Same products
-# as the four-wave kernel, another order of summation.
+# as the four-wave kernel, another order of summation -- so some sum must differ in its last bits.
 @pytest.mark.parametrize("mode", [FP16TCEC, TF32TCEC, TF32TC])
 @pytest.mark.parametrize("cplx,opa,opb,m,n,k,batch,alpha,beta", [
     (False, N, N, 1024, 1024, 1024, 1, 1.0, 0.0),        # 256 interior tiles
     (False, T, N, 1000, 900, 777, 1, 1.5, -0.5),         # edge tiles, ragged K, beta != 0
-    (False, N, N, 300, 200, 4100, 1, 1.0, 1.0),          # K split between workgroups as well (atomic write-out)
+    (False, N, N, 300, 200, 4100, 1, 1.0, 1.0),          # K split into more workgroups than CUs: the four-wave kernel
+    (False, T, N, 300, 260, 3000, 1, 1.0, 1.0),          # K split between workgroups as well (atomic write-out)
     (False, T, N, 256, 192, 520, 16, -1.0, 0.25),        # a batch: 12 tiles x 16 matrices
     (False, N, N, 70, 33, 50, 1, 1.0, 0.0),              # one partial tile, two K-steps
-    (False, T, T, 640, 500, 300, 1, 1.0, 0.0),           # op(B) = T: the groups trade operands
+    (False, T, T, 640, 500, 300, 1, 1.0, 0.0),           # op(B) = T: half units of a row-contiguous operand
+    (False, T, T, 1000, 900, 777, 1, 1.0, 1.0),          # ... ragged K
     (True, N, N, 512, 512, 512, 1, 1.0, 0.0),            # complex: every thread stages half a unit of A and of B
     (True, C, N, 500, 450, 333, 2, 1.0 - 0.5j, 0.5j),    # conjugated A, edge tiles, ragged K, complex scalars
+    (True, N, N, 900, 1000, 333, 1, 1.0, 0.0),           # ... both layouts with op(A) = N: loads two steps ahead
+    (True, N, C, 1000, 900, 777, 1, 0.5j, 1.0),
+    (True, T, T, 600, 600, 1000, 1, 1.0, 0.0),
 ])
 def test_two_wave_groups_match_the_four_wave_kernel(O, handle, dev, monkeypatch, mode, cplx, opa, opb, m, n, k,
                                                     batch, alpha, beta):
     gen = _gen(cplx)   # (complex bf16x3 has no two-group form: both runs launch the same kernel)
+    monkeypatch.setenv("CUMPSGEMM_KWAVES", "0")
     ar, ac = (m, k) if opa == N else (k, m)
     br, bc = (k, n) if opb == N else (n, k)
     lda, ldb, ldc = ar + 1, br + 2, m + 3
@@ -604,6 +611,8 @@ def test_two_wave_groups_match_the_four_wave_kernel(O, handle, dev, monkeypatch,
                                        batch, mode, cplx=cplx)
         assert st == 0
         outs.append(dev.down(dc, np.complex64 if cplx else np.float32))
+    same_kernel = (cplx and mode == TF32TCEC) or (m, n, k) == (300, 200, 4100)
+    assert same_kernel or not np.array_equal(outs[0], outs[1])
     for i in (0, batch - 1):
         x, y = outs[0][i * sc:i * sc + ldc * n], outs[1][i * sc:i * sc + ldc * n]
         assert rel_diff(x, y, m, n, ldc) < 2.0 ** -22 * np.sqrt(k)

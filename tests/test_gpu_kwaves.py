@@ -112,6 +112,14 @@ def test_small_products_scaled_and_gated(handle, dev, monkeypatch, mode, exponen
         assert np.array_equal(outs[0], outs[2]) and np.array_equal(outs[1], outs[2])
 
 
+def test_no_kslice_groups_leaves_small_products_alone(handle, dev, monkeypatch):
+    """CUMPSGEMM_NO_KSLICE_GROUPS chooses between two forms of the tiled kernel, nothing else."""
+    a, b, c0 = inputs.uniform(1, 512 * 512), inputs.uniform(2, 512 * 512), np.zeros(512 * 512, np.float32)
+    monkeypatch.setenv("CUMPSGEMM_NO_KSLICE_GROUPS", "1")
+    assert run_gemm(handle, dev, FP16TCEC, N, N, 512, 512, 512, 1.0, a, 512, b, 512, 0.0, c0, 512, False,
+                    want_module_id=True)[1:] == (0, KWAVES)
+
+
 @pytest.mark.parametrize("mode", [FP16TCEC, TF32TC, SCALING])
 @pytest.mark.parametrize("opa,opb", [(N, N), (C, N), (N, T), (T, C)])
 def test_complex_two_wave_groups_are_exact_on_integers(O, handle, dev, monkeypatch, mode, opa, opb):
