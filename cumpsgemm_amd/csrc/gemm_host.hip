@@ -886,19 +886,23 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
   }
 
   // AUTO launches two gated kernels that must agree on how C is prepared, so
-  // the split-K decision is taken once, from the first candidate.
-  Plan plan0 = make_plan(h, launches[0].p, CPLX, a_kc, b_kc, m, n, k, batch, force_cls, force_split);
+  // the split-K decision is taken once, from the first candidate; where that
+  // one does not split K the second is planned unsplit, as it will run.
+  Plan plans[2]{};
+  plans[0] = make_plan(h, launches[0].p, CPLX, a_kc, b_kc, m, n, k, batch, force_cls, force_split);
+  const Plan &plan0 = plans[0];
+  if (nlaunch > 1)
+    plans[1] = make_plan(h, launches[1].p, CPLX, a_kc, b_kc, m, n, k, batch, force_cls,
+                         force_split == 0 && plan0.ksplit == 1 ? 1 : force_split);
 
   // Small products: K shared out over a workgroup's waves.  (AUTO: both candidates must agree on whether C is
   // prepared and added to, so where the tiled plan splits K either both go this way or neither.)
   int kwaves[2] = {-1, -1};
   if (force_cls < 0 && force_split == 0 && h->ws_override == nullptr) {
     const KWavesProblem problem{CPLX, a_kc, b_kc, m, n, k, batch, lda, ldb};
-    for (int i = 0; i < nlaunch; i++) {
-      const Plan tiled = i == 0 ? plan0 : make_plan(h, launches[i].p, CPLX, a_kc, b_kc, m, n, k, batch, -1, 0);
-      kwaves[i] = choose_kwaves_form((int)launches[i].p, problem, h->num_cus, tiled.cost / (256.0 * 128.0),
-                                     tiled.ksplit > 1, tuning().kwaves);
-    }
+    for (int i = 0; i < nlaunch; i++)
+      kwaves[i] = choose_kwaves_form((int)launches[i].p, problem, h->num_cus, plans[i].cost / (256.0 * 128.0),
+                                     plans[i].ksplit > 1, tuning().kwaves);
     if (plan0.ksplit > 1 && nlaunch == 2 && (kwaves[0] < 0 || kwaves[1] < 0)) kwaves[0] = kwaves[1] = -1;
   }
   const bool any_kwaves = kwaves[0] >= 0 || kwaves[1] >= 0;
@@ -971,8 +975,7 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
       if (used_id != nullptr) *used_id = mode == CUMPSGEMM_AUTO ? ~0u : kKWavesModuleId;
       continue;
     }
-    Plan plan = (i == 0) ? plan0
-                         : make_plan(h, launches[i].p, CPLX, a_kc, b_kc, m, n, k, batch, force_cls, force_split);
+    Plan plan = plans[i];
     if (split) { // same K partition for every candidate
       plan.ksplit = plan0.ksplit;
       plan.k_chunk = plan0.k_chunk;

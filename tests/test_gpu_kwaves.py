@@ -120,6 +120,27 @@ def test_no_kslice_groups_leaves_small_products_alone(handle, dev, monkeypatch):
                     want_module_id=True)[1:] == (0, KWAVES)
 
 
+def test_auto_compares_small_products_with_the_tiled_plan_that_runs(handle, dev, monkeypatch):
+    """AUTO's FP16TCEC candidate where its own tiled plan would split K, but cannot, as the bf16x3 plan does not: the
+    unsplit plan is the one that it would run, and it is slower than the small-product kernel."""
+    m, n, k = 795, 1259, 1765
+    a, b = inputs.uniform(1, m * k), inputs.uniform(2, k * n)
+    da, db = dev.up(a), dev.up(b)
+    outs = []
+    handle.set_exp_stats_params(0.0, 2.0 ** -15, 0.1)  # FP16TCEC for these operands
+    try:
+        for form in (None, "2"):
+            if form:
+                monkeypatch.setenv("CUMPSGEMM_KWAVES", form)
+            dc = dev.up(np.zeros(m * n, np.float32))
+            st, (_, _, flag) = handle.gemm_pipeline(N, N, m, n, k, 1.0, da, m, db, k, 0.0, dc, m, AUTO)
+            assert st == 0 and handle.get_dynamic_launch_flag(flag) == FP16TCEC
+            outs.append(dev.down(dc))
+    finally:
+        handle.set_exp_stats_params(0.0, 2.0 ** -15, 0.0)
+    assert np.array_equal(outs[0], outs[1])  # (a tiled kernel adds in another order)
+
+
 @pytest.mark.parametrize("mode", [FP16TCEC, TF32TC, SCALING])
 @pytest.mark.parametrize("opa,opb", [(N, N), (C, N), (N, T), (T, C)])
 def test_complex_two_wave_groups_are_exact_on_integers(O, handle, dev, monkeypatch, mode, opa, opb):
