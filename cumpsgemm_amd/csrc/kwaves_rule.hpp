@@ -6,6 +6,7 @@
 namespace cumpsgemm_amd {
 
 constexpr int kKWavesForms = 4; // tiles per precision, real or complex
+constexpr int kKWavesFourWaves = 2; // real: the tile of the eight-wave form with four
 constexpr unsigned kKWavesModuleId = 6; // what used_kernel_module_id reports (0 - 4 are the tile classes, 5 the narrow kernel)
 
 // Tile and waves of a form, workgroups that a CU holds at once, and the time of a
@@ -112,6 +113,16 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
       best = i;
       best_time = t;
     }
+  }
+  // Eight waves on a tile pay while all workgroups are on the chip at once: the fit makes their second round too cheap.
+  // 36 of 10000 drawn products were sent to one.  The 32 up to K = 512 take 0.72 - 1.01 of the time with four waves on the
+  // same tile (2560 x 586 x 224 FP16TC NN, us: 9.1, four waves 6.8, tiled 6.7; 231^3 x 22 NT 11.4, 8.9, 11.1).  Beyond, the
+  // tiled kernels are faster where they split K (736 x 1349 x 8128 NN 147, four waves 157, tiled 88), but not where
+  // AUTO keeps them from it (2763 x 347 x 5808 NN 122, tiled 148).
+  if (asked < 0 && best >= 0 && model.form[best].waves == 8 &&
+      (kwaves_tiles(model.form[best], p) + cus - 1) / cus > (uint64_t)model.form[best].resident) {
+    if (p.k <= 512) best = kKWavesFourWaves;
+    else if (tiled_split) best = -1;
   }
   return best;
 }

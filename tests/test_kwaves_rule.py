@@ -71,3 +71,17 @@ def test_the_rule_compares_with_the_tiled_plan(rule):
         assert rule(prec, cplx, "NN", 512, 512, 512, asked=0) is None                  # switched off
         assert rule(prec, cplx, "NN", 512, 512, 0) is None                             # nothing to multiply
         assert rule(prec, cplx, "NN", 8192, 8192, 8192) is None                        # too large for small tiles
+
+
+@pytest.mark.parametrize("prec,op,m,n,k,batch,steps,split,waves", [
+    (1, "NN", 2560, 586, 224, 1, 4.5, False, 4), (0, "TN", 637, 64, 256, 34, 4.9, False, 4),
+    (0, "TT", 64, 40, 243, 352, 4.9, False, 4), (0, "NN", 736, 1349, 8128, 1, 77.7, True, None),
+    (0, "NN", 1920, 544, 4354, 1, 47.1, True, None)])
+def test_eight_waves_on_a_tile_in_one_round_only(rule, prec, op, m, n, k, batch, steps, split, waves):
+    """Products whose eight-wave workgroups a chip of 256 CUs cannot hold at once (`steps`: the tiled plan's cost):
+    measured slower than with four waves, or than tiled where K is long and the tiled plan splits it."""
+    p = rule(prec, False, op, m, n, k, batch, steps=steps, split=split)
+    assert p is None if waves is None else p[3] == waves
+    for m, n in itertools.product((512, 736, 1024, 1333), (512, 1024, 1536)):
+        p = rule(prec, False, op, m, n, k, steps=1e3, split=split)
+        assert p is None or p[3] != 8 or -(-m // 32) * -(-n // 32) <= 2 * CUS
