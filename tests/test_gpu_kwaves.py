@@ -102,14 +102,51 @@ def test_small_products_scaled_and_gated(handle, dev, monkeypatch, mode, exponen
         b, ldb = _padded_ints(rng, opb, k, n, 0, cplx)
         s = np.float32(2.0 ** exponent)
         outs = []
-        for form in ("1", "2", "0"):
+        for form in ("1", "2", "3", "4", "0"):
             monkeypatch.setenv("CUMPSGEMM_KWAVES", form)
             da, db, dc = dev.up(a * s), dev.up(b / s), dev.up(np.full(m * n, np.nan, np.complex64 if cplx else np.float32))
             st, _ = handle.gemm_pipeline(opa, opb, m, n, k, 1.0, da, lda, db, ldb, 0.0, dc, m, mode, cplx=cplx)
             assert st == 0
             outs.append(dev.down(dc, np.complex64 if cplx else np.float32))
         assert np.isfinite(outs[0].view(np.float32)).all()
-        assert np.array_equal(outs[0], outs[2]) and np.array_equal(outs[1], outs[2])
+        assert all(np.array_equal(x, outs[-1]) for x in outs[:-1])
+
+
+@pytest.mark.parametrize("mode,scaled_b,want", [(SCALING, True, FP16TCEC), (AUTO, False, FP16TCEC), (AUTO, True, FP16TCEC),
+                                                (AUTO, None, TF32TCEC)])
+@pytest.mark.parametrize("cplx,opa,opb,form", [(*layout, form) for layout in LAYOUTS for form in ((1, 2) if layout[0] else (1, 2, 3, 4))])
+def test_small_products_scaled_and_gated_with_correction_terms(handle, dev, monkeypatch, mode, scaled_b, want, cplx, opa,
+                                                               opb, form):
+    """Operands that fill every plane: with the form forced a pipeline call gives, bit for bit, what the decided mode
+    gives for operands scaled beforehand -- which is checked against the oracle above, and whose module id says that
+    the form ran.  (K < 256: no tiled plan splits it, so each of AUTO's candidates takes the form if it has it.)"""
+    monkeypatch.setenv("CUMPSGEMM_KWAVES", str(form))
+    gen = inputs.complex_normal if cplx else inputs.uniform
+    dtype = np.complex64 if cplx else np.float32
+    handle.set_exp_stats_params(0.0, 2.0 ** -15, 0.1)
+    try:
+        for m, n, k in ((130, 100, 250), (66, 129, 95)):
+            a, lda = make_operand(gen, 91, opa, m, k)
+            b, ldb = make_operand(gen, 92, opb, k, n)
+            if scaled_b:
+                b *= np.float32(2.0 ** -40)       # every element below fp16's range
+            elif scaled_b is None:
+                b[::2] *= np.float32(2.0 ** -60)  # too far from the others for any scaling
+            c0 = gen(93, m * n)
+            da, db, dc = dev.up(a), dev.up(b), dev.up(c0)
+            st, (_, _, flag) = handle.gemm_pipeline(opa, opb, m, n, k, 0.75, da, lda, db, ldb, -0.5, dc, m, mode, cplx=cplx)
+            assert st == 0 and handle.get_dynamic_launch_flag(flag) & 31 == want
+            got = dev.down(dc, dtype)
+
+            def factor(x):  # 2^14 over the largest element's power of two
+                return np.float32(2.0 ** (14 - np.floor(np.log2(np.abs(x.view(np.float32)).max()))))
+            sa, sb = factor(a) if mode == SCALING else np.float32(1), factor(b) if scaled_b else np.float32(1)
+            ref, st, mid = run_gemm(handle, dev, want, opa, opb, m, n, k, 0.75 / float(sa * sb), a * sa, lda, b * sb, ldb,
+                                    -0.5, c0, m, cplx, want_module_id=True)
+            assert st == 0 and (mid == KWAVES) == (not cplx or form == 1 or want == FP16TCEC)
+            assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (m, n, k)
+    finally:
+        handle.set_exp_stats_params(0.0, 2.0 ** -15, 0.0)
 
 
 def test_no_kslice_groups_leaves_small_products_alone(handle, dev, monkeypatch):
