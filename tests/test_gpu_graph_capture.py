@@ -16,8 +16,11 @@ FP16TCEC, TF32TCEC, AUTO, SCALING = 1, 2, 9, 11
 
 @pytest.mark.parametrize("mode,cplx", [(FP16TCEC, False), (TF32TCEC, False), (FP16TCEC, True),
                                        (SCALING, False), (AUTO, False)])
-def test_captured_calls_replay_like_eager_calls(cg, torch_gpu, mode, cplx):
+@pytest.mark.parametrize("tiled", [False, True])   # the small-product kernel, the tiled ones (real: K split)
+def test_captured_calls_replay_like_eager_calls(cg, torch_gpu, monkeypatch, mode, cplx, tiled):
     torch = torch_gpu
+    if tiled:
+        monkeypatch.setenv("CUMPSGEMM_KWAVES", "0")
     m, n, k = 640, 384, 512
     es = 2 if cplx else 1
     dev = torch.device("cuda:0")
@@ -51,6 +54,7 @@ def test_captured_calls_replay_like_eager_calls(cg, torch_gpu, mode, cplx):
                              want_module_id=True)
             assert st == 0
         k_is_split = 100 <= mid < 200
+        assert (mid == 6) == (not tiled) and k_is_split == (tiled and not cplx), mid
         torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g, stream=side):

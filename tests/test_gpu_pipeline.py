@@ -148,10 +148,13 @@ def test_auto_complex_batched(O, handle, dev):
     (True, N, N, 256, 128, 192),
     (True, T, T, 70, 90, 50),
 ])
-def test_fused_scaling_matches_in_place_scaling(O, handle, dev, monkeypatch, mode, cplx, opa, opb, m, n, k):
+@pytest.mark.parametrize("tiled", [False, True])   # (most of these go to the small-product kernel)
+def test_fused_scaling_matches_in_place_scaling(O, handle, dev, monkeypatch, mode, cplx, opa, opb, m, n, k, tiled):
     """The pipelines scale A, B and C inside the GEMM kernel; the stand-alone
     passes (scale A, B in place, GEMM, scale C, undo) must give the same bits:
     every factor is a power of two."""
+    if tiled:
+        monkeypatch.setenv("CUMPSGEMM_KWAVES", "0")
     gen = (lambda s, c: inputs.complex_normal(s, c, 1.0)) if cplx else inputs.uniform
     a = (gen(31, m * k) * np.float32(2.0 ** -21)).astype(np.complex64 if cplx else np.float32)
     b = (gen(32, k * n) * np.float32(2.0 ** -3)).astype(np.complex64 if cplx else np.float32)
