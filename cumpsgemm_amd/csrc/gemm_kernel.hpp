@@ -1712,12 +1712,12 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void gemm_tcec_kernel(c
           constexpr int ca = (q == 1 || q == 3) ? 1 : 0, cb = (q == 1 || q == 2) ? 1 : 0;
           acc[q][s][0][0] = mfma_block<PT::IS_BF16>(f.b[cb][pb][0], f.a[ca][pa][0], acc[q][s][0][0]);
         };
-        constexpr int X0 = PT::NPROD * decltype(part)::value;
+        constexpr int X0 = 3 * decltype(part)::value;
         one(std::integral_constant<int, X0>{});
-        if constexpr (PT::NPROD > 1) one(std::integral_constant<int, X0 + 1>{});
-        if constexpr (PT::NPROD > 2) one(std::integral_constant<int, X0 + 2>{});
+        one(std::integral_constant<int, X0 + 1>{});
+        one(std::integral_constant<int, X0 + 2>{});
       };
-      static_assert(PT::NPROD <= 3, "four parts");
+      static_assert(PT::NPROD == 3, "four parts of three MFMAs");
       using i0 = std::integral_constant<int, 0>;
       using i1 = std::integral_constant<int, 1>;
       using i2 = std::integral_constant<int, 2>;

@@ -6,16 +6,8 @@
 namespace cumpsgemm_amd {
 
 template <class Cfg> void launch_kwaves(const GemmArgs &args, dim3 grid, hipStream_t stream) {
-  if (Cfg::LDS_BYTES > 64 * 1024) { // (allowed once per kernel and device, as in launch_cfg)
-    static std::atomic<bool> attr_done[64] = {};
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    if (dev < 0 || dev >= 64 || !attr_done[dev].load(std::memory_order_acquire)) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&kwaves_gemm_tcec_kernel<Cfg>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
-      if (dev >= 0 && dev < 64) attr_done[dev].store(true, std::memory_order_release);
-    }
-  }
+  static device_flags_t done = {};
+  allow_dynamic_lds(reinterpret_cast<const void *>(&kwaves_gemm_tcec_kernel<Cfg>), Cfg::LDS_BYTES, done);
   hipLaunchKernelGGL(kwaves_gemm_tcec_kernel<Cfg>, grid, dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
 }
 

@@ -20,7 +20,7 @@ struct KernelEntry {
   void (*launch_scaled)(const GemmArgs &, dim3 grid, hipStream_t stream);
   void (*launch_scaled_persistent)(const GemmArgs &, dim3 grid, hipStream_t stream);
   // variant with twice the waves, each group taking one K-slice of every step
-  // (small real tiles only, else nullptr): for problems of no more tiles than CUs
+  // (64x64 tiles on 32x32x16 MFMAs, real and complex, else nullptr): for problems of no more tiles than CUs
   void (*launch_kslices)(const GemmArgs &, dim3 grid, hipStream_t stream);
   void (*launch_scaled_kslices)(const GemmArgs &, dim3 grid, hipStream_t stream); // (FP16TCEC tables only)
   // the persistent variants on 16x16x32 MFMAs (real FP16TCEC 256x128 and 128x128,
@@ -53,21 +53,24 @@ void prepare_cfg() {
   (void)hipGetLastError();
 }
 
+// More than 64 KiB of dynamic LDS must be allowed once per kernel and device.
+// `done`: the kernel's own flags, one a device (setting the attribute twice is
+// harmless, so threads that race here only need a flag to be free of a data race).
+typedef std::atomic<bool> device_flags_t[64];
+inline void allow_dynamic_lds(const void *kernel, int bytes, device_flags_t &done) {
+  if (bytes <= 64 * 1024) return;
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  if (dev < 0 || dev >= 64 || !done[dev].load(std::memory_order_acquire)) {
+    (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (dev >= 0 && dev < 64) done[dev].store(true, std::memory_order_release);
+  }
+}
+
 template <class Cfg>
 void launch_cfg(const GemmArgs &args, dim3 grid, hipStream_t stream) {
-  if (Cfg::LDS_BYTES > 64 * 1024) {
-    // more than 64 KiB of dynamic LDS must be allowed once per kernel and device
-    // (setting it twice is harmless, so threads that race here only need the
-    // flag itself to be free of a data race)
-    static std::atomic<bool> attr_done[64] = {};
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    if (dev < 0 || dev >= 64 || !attr_done[dev].load(std::memory_order_acquire)) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tcec_kernel<Cfg>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
-      if (dev >= 0 && dev < 64) attr_done[dev].store(true, std::memory_order_release);
-    }
-  }
+  static device_flags_t done = {};
+  allow_dynamic_lds(reinterpret_cast<const void *>(&gemm_tcec_kernel<Cfg>), Cfg::LDS_BYTES, done);
   hipLaunchKernelGGL(gemm_tcec_kernel<Cfg>, grid, dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
 }
 
