@@ -114,15 +114,22 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
       best_time = t;
     }
   }
-  // Eight waves on a tile pay while all workgroups are on the chip at once: the fit makes their second round too cheap.
-  // 36 of 10000 drawn products were sent to one.  The 32 up to K = 512 take 0.72 - 1.01 of the time with four waves on the
-  // same tile (2560 x 586 x 224 FP16TC NN, us: 9.1, four waves 6.8, tiled 6.7; 231^3 x 22 NT 11.4, 8.9, 11.1).  Beyond, the
-  // tiled kernels are faster where they split K (736 x 1349 x 8128 NN 147, four waves 157, tiled 88), but not where
-  // AUTO keeps them from it (2763 x 347 x 5808 NN 122, tiled 148).
-  if (asked < 0 && best >= 0 && model.form[best].waves == 8 &&
-      (kwaves_tiles(model.form[best], p) + cus - 1) / cus > (uint64_t)model.form[best].resident) {
-    if (p.k <= 512) best = kKWavesFourWaves;
-    else if (tiled_split) best = -1;
+  if (asked < 0 && best >= 0 && model.form[best].waves == 8) {
+    // Eight waves on a tile pay while all workgroups are on the chip at once: the fit makes their second round too cheap.
+    // 36 of 10000 drawn products were sent to one.  The 32 up to K = 512 take 0.72 - 1.01 of the time with four waves on
+    // the same tile (2560 x 586 x 224 FP16TC NN, us: 9.1, four waves 6.8, tiled 6.7; 231^3 x 22 NT 11.4, 8.9, 11.1).
+    // Beyond, the tiled kernels are faster where they split K (736 x 1349 x 8128 NN 147, four waves 157, tiled 88), but
+    // not where AUTO keeps them from it (2763 x 347 x 5808 NN 122, tiled 148).
+    const uint64_t per_cu = (kwaves_tiles(model.form[best], p) + cus - 1) / cus;
+    if (per_cu > (uint64_t)model.form[best].resident) {
+      if (p.k <= 512) best = kKWavesFourWaves;
+      else if (tiled_split) best = -1;
+    } else if (per_cu > 1 && p.k >= 2560 && tiled_split && !p.a_kc && !p.b_kc) {
+      // Two of them on a CU read a long K of two row-contiguous operands slower than the fit has it: 20 of 18000 drawn
+      // products, 19 of them 1.05 - 1.63 times as long as with K split (1090 x 256 x 3360 FP16TC 34.0 us, tiled 22.3;
+      // FP16TCEC 528 x 528 x 2880 24.3, 22.3).  K 2048 - 2559: 8 of 18 longer, 7 shorter; other layouts level.
+      best = -1;
+    }
   }
   return best;
 }

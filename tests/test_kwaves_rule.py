@@ -81,7 +81,15 @@ def test_eight_waves_on_a_tile_in_one_round_only(rule, prec, op, m, n, k, batch,
     """Products whose eight-wave workgroups a chip of 256 CUs cannot hold at once (`steps`: the tiled plan's cost):
     measured slower than with four waves, or than tiled where K is long and the tiled plan splits it."""
     p = rule(prec, False, op, m, n, k, batch, steps=steps, split=split)
-    assert p is None if waves is None else p[3] == waves
+    assert (p and p[3]) == waves
     for m, n in itertools.product((512, 736, 1024, 1333), (512, 1024, 1536)):
         p = rule(prec, False, op, m, n, k, steps=1e3, split=split)
         assert p is None or p[3] != 8 or -(-m // 32) * -(-n // 32) <= 2 * CUS
+
+
+@pytest.mark.parametrize("prec,m,n,k,steps", [(1, 1090, 256, 3360, 15.4), (1, 2549, 112, 2560, 12.6), (0, 528, 528, 2880, 13.7)])
+def test_a_long_k_of_two_row_contiguous_operands_is_split(rule, prec, m, n, k, steps):
+    """Two eight-wave workgroups on a CU, K as long and split by the tiled plan (`steps`: its cost): measured slower."""
+    assert rule(prec, False, "NT", m, n, k, steps=steps, split=True) is None
+    for op, kk, split in (("TN", k, True), ("NT", 1500, True), ("NT", k, False)):
+        assert rule(prec, False, op, m, n, kk, steps=2 * steps, split=split) is not None
