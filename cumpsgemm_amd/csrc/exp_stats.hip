@@ -152,7 +152,8 @@ __device__ inline void finish_pair_job(int *flag_out, unsigned *pair_ticket, Sta
 // What bounds a small matrix is a chain: kernel arguments, data, reductions, record, ticket, records, slot, each a round
 // trip of ~ 0.7 us or a row of dependent lane moves.  With DPP moves instead of shuffles, the records folded by one wave,
 // no counts where only the maximum is asked for and no hand-over in a job of one workgroup: FP16TCEC_SCALING calls, us,
-// 128^3 11.7 -> 8.2, 180^3 12.6 -> 8.2, 512^3 12.6 -> 9.8, 1024^3 21.9 -> 20.0 (two launches take about 8 whatever they do).
+// 128^3 11.7 -> 9.4, 180^3 12.6 -> 9.5, 512^3 12.6 -> 9.8, 1024^3 21.9 -> 20.0; with the loads of the remainder in flight
+// together (below) 128^3 and 180^3 8.2.  Two launches take about 8 whatever they do.
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void exp_stats_kernel(const StatsJob job0, const StatsJob job1,
                                                            float ignore_thr, float under_thr,

@@ -1023,11 +1023,13 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
       // bound by the latency of their own chain of LDS reads, MFMAs and staging,
       // so the form with two wave groups (a K-slice of every step each) is
       // launched -- where it was measured faster: complex or with an operand
-      // K-contiguous, and a mode with correction terms or bf16 planes (1024^3, plain
-      // -> two groups, us: FP16TCEC NN 19.3 -> 16.4, TN 16.2 -> 13.8, TT 18.6 -> 16.1,
-      // bf16x3 NN 28.1 -> 21.5, bf16x2 NN 19.7 -> 16.5; complex FP16TCEC NN 38.6 ->
-      // 30.0, NT 41.9 -> 32.0, bf16x2 NT 41.2 -> 30.9; FP16TC level or slower; real
-      // op(A) = N with op(B) = T level).
+      // K-contiguous, and a mode with correction terms or bf16 planes (complex 1000^3,
+      // plain -> two groups, us: FP16TCEC NN 38.6 -> 30.0, NT 41.9 -> 32.0, bf16x2 NT
+      // 41.2 -> 30.9; FP16TC level or slower; real op(A) = N with op(B) = T level).
+      // Real products come here with K split (from K = 1000 or so on), in bf16x3 with a
+      // few K-steps as well; the others go to the small-product kernel.  With that one
+      // switched off, 1024^3, us: FP16TCEC NN 19.3 -> 16.4, TN 16.2 -> 13.8, TT 18.6 ->
+      // 16.1, bf16x3 NN 28.1 -> 21.5.
       const uint64_t groups = (uint64_t)grid.x * grid.y * grid.z;
       auto launch_groups = launch_plain == e->launch_scaled ? e->launch_scaled_kslices : e->launch_kslices;
       if (launch_groups != nullptr && groups <= (uint64_t)h->num_cus && (CPLX || a_kc || b_kc) &&

@@ -528,7 +528,9 @@ struct tile_loader {
   // 16-byte chunk of a plane.  Row-contiguous: 16 lanes read 16 consecutive rows and
   // the next 16 the same rows' other half (with pairs of lanes on two K-lines no two
   // neighbours read neighbouring addresses: complex 800^3 NN 23.6 -> 22.4 us, real
-  // 1024^3 TT 18.8 -> 17.4).  Both ways 32 lanes' 8-byte LDS writes cover all banks.
+  // 1024^3 TT 18.8 -> 17.4).  The 8-byte LDS writes of pairs of lanes are free of bank
+  // conflicts; those of 16 rows at once meet two by two (complex 1000^3 NN, one such
+  // operand: 1.05e6 conflict cycles for 1.6e5 writes), which is the smaller cost.
   // (HALF_UNITS: the precisions this pays for, measured -- FP16TCEC and bf16x2; the
   // costlier bf16x3 split and the single-product FP16TC kernels keep whole units)
   static constexpr bool HALF = HALF_UNITS && (ROWS * 4 * 2 == NT);
@@ -1695,12 +1697,12 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void gemm_tcec_kernel(c
       // Two wave groups, complex: a wave's MFMAs of a step in four parts, and beside
       // each the splitting of one component of one operand of the next step -- MFMAs
       // in a row keep the vector unit from the SIMD's other wave as well -- with the
-      // loads of the step after that in flight.  What is left bounds a step about
-      // equally: 64 KB of LDS writes and reads, 768 cycles of MFMAs per SIMD and 32 KB
-      // from L2 (all CUs together 10 TB/s).  us, MFMAs after the splitting -> so, and
-      // with row-contiguous half units by 16 lanes: FP16TCEC 600^3 NN 20.8 -> 17.7,
-      // 800^3 NN 26.0 -> 21.4, CN 22.4 -> 21.5, 1000^3 NN 33.5 -> 31.2, NT (two-buffer
-      // kernel before) 42.5 -> 32.8; bf16x2 1000^3 NN 33.0 -> 30.2.
+      // loads of the step after that in flight.  A step takes about 2300 clocks (1000^3
+      // NN: 32 of them in 30.6 us): 768 of MFMAs per SIMD, 5.7 vector instructions for
+      // each MFMA and 32 KB from L2 (all CUs together 9 TB/s).  us, MFMAs after the
+      // splitting -> so, and with row-contiguous half units by 16 lanes: FP16TCEC 600^3
+      // NN 20.8 -> 17.7, 800^3 NN 26.0 -> 21.4, CN 22.4 -> 21.5, 1000^3 NN 33.5 -> 31.2,
+      // NT (two-buffer kernel before) 42.5 -> 32.8; bf16x2 1000^3 NN 33.0 -> 30.2.
       auto load = [&](auto &xa, auto &xb, const int kt) {
         LA::template load_fast<true>(xa, a_tile + (uint64_t)kt * a_kstep, args.lda, offa);
         LB::template load_fast<true>(xb, b_tile + (uint64_t)kt * b_kstep, args.ldb, offb);

@@ -14,14 +14,13 @@
 // One K-step of a wave is multiplied beside the splitting of the next and the
 // loads of the one after that, piece by piece (a wave issues its MFMAs and vector
 // instructions one after the other, and MFMAs issued in a row keep the vector
-// unit from the SIMD's other waves).  All loads are 16 bytes a lane: the address
-// path takes about 16 clocks a load whatever its width, and a row-contiguous
-// operand read 4 bytes a lane took 2100 instead of 1000 clocks a step of four waves.
+// unit from the SIMD's other waves).  All loads are 16 bytes a lane, of a
+// row-contiguous operand too: a quarter of the load instructions.
 //
-// FP16TCEC, us, tiled -> here (one call among others; 5.0 is what the host takes):
-// 512^3 NN 9.9 -> 5.1, NT 10.1 -> 5.1, 1024^3 NN 17.5 -> 13.1, NT 20.7 -> 12.7, TN 16.1 -> 13.0;
-// complex 256^3 NN 13.2 -> 6.1, NT 14.3 -> 6.0, 512^3 NN 17.9 -> 8.6, NT 23.0 -> 8.5.
-// Larger products are bound by what a small tile reads (2048^3 58 -> 85): see kwaves_rule.hpp.
+// FP16TCEC, us, tiled -> here (calls of a graph; a loop of single calls takes 5 at least):
+// 512^3 NN 9.5 -> 4.4, NT 9.7 -> 4.3, 1024^3 NN 16.1 -> 13.5, NT 22.1 -> 13.0, TN 13.9 -> 13.2;
+// complex 256^3 NN 12.9 -> 5.8, NT 13.3 -> 5.7, 512^3 NN 14.8 -> 8.3, NT 16.8 -> 8.1.
+// Larger products are bound by what a small tile reads (2048^3 NN 58 -> 92): see kwaves_rule.hpp.
 #pragma once
 #include "gemm_kernel.hpp"
 
@@ -53,7 +52,10 @@ struct KWavesCfg {
 // fourth row instead of a swizzle: a lane of a row-contiguous operand writes one
 // chunk of four consecutive rows, lanes l and l + 1 the same chunk of rows four
 // apart; that, the 8-byte writes of a K-contiguous operand (8 rows x 64 bytes) and
-// the fragment reads (32 rows, two chunks) all spread evenly over the banks.
+// the fragment reads (32 rows, two chunks) all spread evenly over the banks (real
+// 512^3: no conflicts; the sums of 64 x 64 tiles add 256 cycles a workgroup).  A complex
+// row-contiguous operand writes rows two apart, which meet in pairs: 512^3 NT 5.6e5
+// conflict cycles in all, 2200 a workgroup, NN 3.0e5, TN 3e4.
 __device__ constexpr int kwave_lds(const int row, const int chunk) { return row * 64 + (row >> 2) * 16 + chunk * 16; }
 
 // K-value at position j of 16-byte chunk c of an LDS row (complex: the order in

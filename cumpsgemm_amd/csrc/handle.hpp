@@ -65,7 +65,7 @@ constexpr unsigned kMaxStatsBlocks = 4096;     // partial-result scratch entries
 struct Tuning {
   int packed = -1;      // CUMPSGEMM_PACKED: 0 never / 1 whenever possible take the pre-split path
   int packed_walk = -1; // CUMPSGEMM_PACKED_WALK: 0 / 1 force the one-tile / persistent pre-split kernel
-  int raster_group = 0; // CUMPSGEMM_RASTER_GROUP: tile rows per column group (0: built-in choice)
+  int raster_group = 0; // CUMPSGEMM_RASTER_GROUP: tile rows per column group (0: built-in choice; not for small products)
   // CUMPSGEMM_EXP_FETCH_FROM_ONE_PATCH (profiler experiment, WRONG RESULTS): the
   // tile-walking pre-split kernel reads every tile's operands from one
   // L2-resident patch, which shows what its operand traffic over the fabric costs
@@ -80,7 +80,7 @@ struct Tuning {
   bool no_kslices = false;       // CUMPSGEMM_NO_KSLICE_GROUPS: tiled kernels with one wave group throughout
   bool no_narrow = false;        // CUMPSGEMM_NO_NARROW: results with a narrow side take the tiled kernels
   int kwaves = -1;               // CUMPSGEMM_KWAVES: 0 never, 1 ... the form of the small-product kernel, where it can
-                                 // serve the call (gemm_kwaves_*.hip)
+                                 // serve the call (gemm_kwaves_*.hip; a forced class or split goes before)
   bool no_fused_scaling = false; // CUMPSGEMM_NO_FUSED_SCALING
   unsigned persistent_max_steps = 32; // CUMPSGEMM_PERSISTENT_MAX_STEPS
   // CUMPSGEMM_MAX_WORKSPACE_BYTES: the pre-split path is not taken when its

@@ -21,13 +21,16 @@ struct KWavesForm {
 //
 // All of it fitted on 188 products (84 real, m and n 64 - 4096, K 64 - 8192, 60 real
 // batches of up to 1024 matrices of 32 - 640, 44 complex; four layouts, padded, with
-// and without C), each timed with every form and tiled, in every precision.  Times of
-// all products with the rule over times without, and what picking the faster side by
-// hindsight would give:      real          real batches     complex
-//   FP16TCEC             0.81 (0.79)     0.84 (0.81)     0.64 (0.63)
-//   bf16x3               0.80 (0.78)     0.83 (0.81)     0.59 (0.59)
-//   FP16TC               0.76 (0.74)     0.84 (0.80)     0.64 (0.64)
-//   bf16x2               0.80 (0.78)     0.83 (0.81)     0.64 (0.64)
+// and without C), each timed with every form and tiled, in every precision.  On 10000
+// other products that the rule sends here, drawn over the same ranges: time over the
+// tiled time, geometric mean (the fastest side by hindsight); share that is slower by
+// 5 % and 10 %, and the largest loss:
+//               real                             real batches
+//   FP16TCEC    0.65 (0.64) 2.4 %, 1.4 %, 1.25   0.64 (0.63) 3.3 %, 1.7 %, 1.34
+//   bf16x3      0.64 (0.63) 0.7 %, 0.1 %, 1.10   0.64 (0.63) 1.9 %, 1.1 %, 1.15
+//   FP16TC      0.59 (0.58) 3.6 %, 1.9 %, 1.46   0.63 (0.62) 2.4 %, 1.1 %, 1.31
+//   bf16x2      0.64 (0.63) 1.5 %, 0.7 %, 1.33   0.64 (0.63) 2.7 %, 1.3 %, 1.25
+// complex 0.50 - 0.60, none slower by 5 %; AUTO calls 0.84 real, 0.74 complex.
 // (Tried beside these and left out, within 1 %: 64 x 32 and 32 x 64 with four and
 // eight waves, 64 x 64 with one and two; 128 x 64 spills.  Complex with one or two
 // waves: batches are faster tiled.)
@@ -91,8 +94,9 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
   // (complex tiles take 6 % longer per step with two row-contiguous operands, 7 % less with none)
   const double layout = !p.cplx ? 1.0 : p.a_kc && p.b_kc ? 0.93 : !p.a_kc && !p.b_kc ? 1.06 : 1.0;
   const double tiled = model.tiled0 + layout * model.tiled_per_step * tiled_steps + (tiled_split ? model.tiled_split : 0.0);
-  // Both sides are estimates, the tiled one within 15 % (95 % of 700 products within 25 %): with 1.0 here the number
-  // of products that get more than 3 % slower doubles and the mean stays.  Long ones have less to gain: 0.8.
+  // Both sides are estimates, within 10 - 30 % of the times: with 1.0 here the number of products that get more than
+  // 3 % slower doubles and the mean stays; with 0.8 (long ones 0.7) a third of the losses is left, and the mean of 10000
+  // real products goes from 0.643 to 0.660 of the tiled time.  Long ones have less to gain: 0.8.
   double best_time = (tiled > 30.0 ? 0.8 : 0.9) * tiled;
   int best = -1;
   for (int i = 0; i < kKWavesForms; i++) {
@@ -125,7 +129,7 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
       if (p.k <= 512) best = kKWavesFourWaves;
       else if (tiled_split) best = -1;
     } else if (per_cu > 1 && p.k >= 2560 && tiled_split && !p.a_kc && !p.b_kc) {
-      // Two of them on a CU read a long K of two row-contiguous operands slower than the fit has it: 20 of 18000 drawn
+      // Two of them on a CU read a long K of two row-contiguous operands slower than the fit has it: 20 of 17000 drawn
       // products, 19 of them 1.05 - 1.63 times as long as with K split (1090 x 256 x 3360 FP16TC 34.0 us, tiled 22.3;
       // FP16TCEC 528 x 528 x 2880 24.3, 22.3).  K 2048 - 2559: 8 of 18 longer, 7 shorter; other layouts level.
       best = -1;

@@ -83,7 +83,9 @@ const void *cuMpSGEMM_get_workspace_pointer(cuMpSGEMM_handle_t handle);
 
 /* The tuning variables of the GEMM path (CUMPSGEMM_PACKED, _PACKED_WALK,
  * _RASTER_GROUP, _FORCE_TILE_CLASS, _FORCE_KSPLIT, _NO_PERSISTENT,
- * _NO_COLUMN_SPLIT, _CUT_PERCENT, _NO_KSLICE_GROUPS, _NO_NARROW, _KWAVES, _NO_EDGE16_TWIN, _NO_FUSED_SCALING,
+ * _NO_COLUMN_SPLIT, _CUT_PERCENT, _NO_KSLICE_GROUPS, _NO_NARROW, _KWAVES (0: no call
+ * takes the small-product kernel, 1 - 4: this form of it wherever it can),
+ * _NO_EDGE16_TWIN, _NO_FUSED_SCALING,
  * _PERSISTENT_MAX_STEPS, _MAX_WORKSPACE_BYTES) are read from the environment
  * once per process; this reads them again and publishes the new set as one
  * immutable snapshot.  Safe to call while other threads run GEMMs: a call in
@@ -192,7 +194,10 @@ void cuMpSGEMM_disable_exp_stats(cuMpSGEMM_handle_t h);
  * get_..._entry is debug::get_exp_stats_profiling_result for one label
  * ("exp_stats_1", "exp_stats_2", "exp_max", "scaling_AB", "scaling_C",
  * "reset_scaling_AB", a GEMM label): returns 1 and fills seconds / count when
- * the label has been recorded, else 0. */
+ * the label has been recorded, else 0.  While it is on, every launch is waited
+ * for, and the two stages of exponent statistics are launched one after the other
+ * so that each has its time: two small matrices, whose statistics are otherwise
+ * one launch, take 1 - 2.5 us longer then. */
 void cuMpSGEMM_enable_exp_stats_profiling(cuMpSGEMM_handle_t h);
 void cuMpSGEMM_disable_exp_stats_profiling(cuMpSGEMM_handle_t h);
 void cuMpSGEMM_reset_exp_stats_profiling(cuMpSGEMM_handle_t h);
