@@ -204,25 +204,38 @@ template <> struct splitter<Prec::FP16TC> {
     out[0] = __builtin_bit_cast(u4_t, __builtin_convertvector(x, h8_t));
   }
 };
+// Pair by pair: one conversion instruction rounds two values, and both are
+// taken back out of its packed result by a shift and a mask.  (Written on whole
+// vectors the compiler converts every value once more on its own to widen it:
+// 60 and 32 vector instructions for eight values in three and two terms, 44 and
+// 24 so.)  `x0`, `x1` are left as what the first term does not hold.
+__device__ inline uint32_t split_pair_bf16(float &x0, float &x1) {
+  typedef __bf16 b2_t __attribute__((ext_vector_type(2)));
+  typedef float f2_t __attribute__((ext_vector_type(2)));
+  const f2_t x = {x0, x1};
+  const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, b2_t));
+  x0 -= __uint_as_float(b << 16);
+  x1 -= __uint_as_float(b & 0xffff0000u);
+  return b;
+}
 template <> struct splitter<Prec::BF16X3> {
   __device__ static inline void run(const f8_t x, u4_t (&out)[3]) {
-    const b8_t b0 = __builtin_convertvector(x, b8_t);
-    const f8_t r1 = x - __builtin_convertvector(b0, f8_t);
-    const b8_t b1 = __builtin_convertvector(r1, b8_t);
-    const f8_t r2 = r1 - __builtin_convertvector(b1, f8_t);
-    const b8_t b2 = __builtin_convertvector(r2, b8_t);
-    out[0] = __builtin_bit_cast(u4_t, b0);
-    out[1] = __builtin_bit_cast(u4_t, b1);
-    out[2] = __builtin_bit_cast(u4_t, b2);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      float r0 = x[2 * i], r1 = x[2 * i + 1];
+#pragma unroll
+      for (int p = 0; p < 3; p++) out[p][i] = split_pair_bf16(r0, r1);
+    }
   }
 };
 template <> struct splitter<Prec::BF16X2> {
   __device__ static inline void run(const f8_t x, u4_t (&out)[2]) {
-    const b8_t b0 = __builtin_convertvector(x, b8_t);
-    const f8_t r1 = x - __builtin_convertvector(b0, f8_t);
-    const b8_t b1 = __builtin_convertvector(r1, b8_t);
-    out[0] = __builtin_bit_cast(u4_t, b0);
-    out[1] = __builtin_bit_cast(u4_t, b1);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      float r0 = x[2 * i], r1 = x[2 * i + 1];
+#pragma unroll
+      for (int p = 0; p < 2; p++) out[p][i] = split_pair_bf16(r0, r1);
+    }
   }
 };
 
