@@ -239,6 +239,32 @@ template <> struct splitter<Prec::BF16X2> {
   }
 };
 
+// Terms of one pair of values, packed (SCALED: of the pair times s, a power of
+// two; s2048 = s * 2^11), for kernels that are bound by issuing vector
+// instructions.  FP16TCEC: fma(hi, -2^11, x * 2^11) as above, but on values widened
+// again: 8 instructions instead of 5, which one wave alone on a SIMD issues in
+// 27 clocks instead of 29 (37 with the wait that two half writes in a row need):
+// the mixed-precision FMA that writes fp16 has a quarter of the FMA's rate.
+template <Prec P, bool SCALED>
+__device__ inline void split_pair(float x0, float x1, const float s, const float s2048,
+                                  uint32_t (&out)[prec_traits<P>::NP]) {
+  typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+  typedef float f2_t __attribute__((ext_vector_type(2)));
+  if constexpr (P == Prec::BF16X3 || P == Prec::BF16X2) {
+#pragma unroll
+    for (int p = 0; p < prec_traits<P>::NP; p++) out[p] = split_pair_bf16(x0, x1);
+  } else {
+    const f2_t x = SCALED ? f2_t{x0 * s, x1 * s} : f2_t{x0, x1};
+    const h2_t hi = __builtin_convertvector(x, h2_t);
+    out[0] = __builtin_bit_cast(uint32_t, hi);
+    if constexpr (P == Prec::FP16TCEC) {
+      const float t = SCALED ? s2048 : 2048.0f;
+      const f2_t r = {__builtin_fmaf((float)hi[0], -2048.0f, x0 * t), __builtin_fmaf((float)hi[1], -2048.0f, x1 * t)};
+      out[1] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, h2_t));
+    }
+  }
+}
+
 template <bool IS_BF16>
 __device__ inline f16v_t mfma_block(const u4_t a, const u4_t b, const f16v_t c) {
   if constexpr (IS_BF16) {

@@ -17,23 +17,33 @@
 // unit from the SIMD's other waves).  All loads are 16 bytes a lane, of a
 // row-contiguous operand too: a quarter of the load instructions.
 //
+// Two waves to a SIMD where the registers allow it (not bf16x3): a wave alone issues a
+// vector instruction every 5 clocks and a conversion every 8, two of them together one
+// every 2 - 4, and MFMAs of one run beside splitting of the other.  On a 64 x 64 (complex
+// 32 x 32) tile that is two workgroups of four waves on a CU; complex products of no more
+// tiles than CUs take one of eight.  us, one workgroup of four waves per CU -> so: real
+// FP16TCEC 1152^3 NN 25.4 -> 20.3 (tiled 24.4), 1408^3 30.5 -> 26.8, 1531 x 1021 x 777 TT
+// 22.7 -> 18.8 (tiled 19.6); FP16TC 1152^3 17.5 -> 15.0; complex FP16TCEC 512^3 NN 8.5 -> 7.6,
+// 640^3 16.6 -> 12.9, 900 x 300 x 900 22.9 -> 17.5, 512 x 512 x 2048 22.0 -> 20.8; level on
+// 1024^3 (12.9), whose 256 tiles are one to a CU either way.
+//
 // FP16TCEC, us, tiled -> here (calls of a graph; a loop of single calls takes 5 at least):
-// 512^3 NN 9.5 -> 4.4, NT 9.7 -> 4.3, 1024^3 NN 16.1 -> 13.5, NT 22.1 -> 13.0, TN 13.9 -> 13.2;
-// complex 256^3 NN 12.9 -> 5.8, NT 13.3 -> 5.7, 512^3 NN 14.8 -> 8.3, NT 16.8 -> 8.1.
-// Larger products are bound by what a small tile reads (2048^3 NN 58 -> 92): see kwaves_rule.hpp.
+// 512^3 NN 9.5 -> 4.4, NT 9.7 -> 4.3, 1024^3 NN 16.1 -> 13.0, NT 22.1 -> 12.2, TN 13.4 -> 12.5;
+// complex 256^3 NN 13.1 -> 5.3, NT 13.5 -> 5.2, 512^3 NN 14.9 -> 7.6, NT 16.6 -> 7.5.
+// Larger products are bound by what a small tile reads (2048^3 NN 58 -> 74): see kwaves_rule.hpp.
 #pragma once
 #include "gemm_kernel.hpp"
 
 namespace cumpsgemm_amd {
 
 // W waves; OCC waves per SIMD that the register allocator must leave room for.
-
 template <Prec P_, bool CPLX_, bool A_KC_, bool B_KC_, int BM_, int BN_, int W_, int OCC_, bool SCALED_ = false>
 struct KWavesCfg {
   static constexpr Prec P = P_;
   static constexpr bool CPLX = CPLX_, A_KC = A_KC_, B_KC = B_KC_, SCALED = SCALED_;
   static constexpr int BM = BM_, BN = BN_, W = W_, OCC = OCC_;
   static constexpr int NT = W * 64;
+  static constexpr bool TWO_PER_SIMD = OCC == 2;
   static constexpr int TM = BM / 32, TN = BN / 32;
   static constexpr int NP = prec_traits<P>::NP, NC = CPLX ? 2 : 1;
   // LDS: planes of 64-byte rows (32 K-values), 16 bytes of padding after every fourth row
@@ -165,12 +175,14 @@ template <Prec P, bool CPLX, bool KC, int ROWS, bool SCALED> struct WaveOperand 
     const int pos = pos_of(I, lane), at = kwave_lds(row_of(I, lane), pos >> 3) + (pos & 7) * 2;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-      f8_t x;
-#pragma unroll
-      for (int j = 0; j < 8; j++) x[j] = j < KV ? value<I>(j < KV ? j : 0, c) : 0.0f;
       u4_t out[NP];
-      if constexpr (SCALED) splitter<P>::run_scaled(x, out, s, s2048);
-      else splitter<P>::run(x, out);
+#pragma unroll
+      for (int q = 0; q < KV / 2; q++) {
+        uint32_t terms[NP];
+        split_pair<P, SCALED>(value<I>(2 * q, c), value<I>(2 * q + 1, c), s, s2048, terms);
+#pragma unroll
+        for (int p = 0; p < NP; p++) out[p][q] = terms[p];
+      }
 #pragma unroll
       for (int p = 0; p < NP; p++) {
         char *const to = lds_op + (c * NP + p) * PLANE + at;
@@ -329,37 +341,67 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void kwaves_gemm_tcec_k
       static_for<0, PA + PB>(load_after);
       advance();
     }
-    Frags f0, f1;
     static_for<0, PA + PB>(store_piece);
     if (steps > 1) {
       static_for<0, PA + PB>(load_after);
       advance();
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-    frag_load(f0, 0);
-    // one K-step beside the staging of the next
-    constexpr int LAST = STEP_MFMAS / 6, BESIDE = STEP_MFMAS - LAST;
-    auto step = [&](auto load_tag) {
-      frag_load(f1, 1);
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-      static_for<0, PA + PB>([&](auto i_tag) {
-        constexpr int I = decltype(i_tag)::value;
-        constexpr int w0 = I < PA ? I * WA : PA * WA + (I - PA) * WB, w1 = w0 + (I < PA ? WA : WB);
-        static_for<BESIDE * w0 / WSUM, BESIDE * w1 / WSUM>([&](auto x) { mma(f0, f1, x); });
-        store_piece(i_tag);
-        if constexpr (decltype(load_tag)::value) load_after(i_tag);
+    if constexpr (Cfg::TWO_PER_SIMD) {
+      // One set of fragments: 128 accumulator registers, 64 of loads in flight and
+      // 32 of fragments leave room for a second wave on the SIMD.  The first half of
+      // a step's MFMAs run beside the other wave's splitting, the second half beside
+      // this wave's.
+      Frags f;
+      auto step = [&](auto stage_tag, auto load_tag) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        frag_load(f, 0);
+        static_for<0, HALF_MFMAS>([&](auto x) { mma(f, f, x); });
         __builtin_amdgcn_sched_barrier(0);
-      });
-      if constexpr (decltype(load_tag)::value) advance();
+        frag_load(f, 1);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        static_for<0, PA + PB>([&](auto i_tag) {
+          constexpr int I = decltype(i_tag)::value;
+          constexpr int w0 = I < PA ? I * WA : PA * WA + (I - PA) * WB, w1 = w0 + (I < PA ? WA : WB);
+          static_for<HALF_MFMAS + HALF_MFMAS * w0 / WSUM, HALF_MFMAS + HALF_MFMAS * w1 / WSUM>(
+              [&](auto x) { mma(f, f, x); });
+          if constexpr (decltype(stage_tag)::value) store_piece(i_tag);
+          if constexpr (decltype(load_tag)::value) load_after(i_tag);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (decltype(load_tag)::value) advance();
+      };
+      int t = 0;
+      for (; t + 2 < steps; t++) step(std::true_type{}, std::true_type{});
+      if (t + 1 < steps) step(std::true_type{}, std::false_type{});
+      step(std::false_type{}, std::false_type{});
+    } else {
+      Frags f0, f1;
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
       frag_load(f0, 0);
-      static_for<BESIDE, STEP_MFMAS>([&](auto x) { mma(f0, f1, x); });
-    };
-    int t = 0;
-    for (; t + 2 < steps; t++) step(std::true_type{});
-    if (t + 1 < steps) step(std::false_type{});
-    frag_load(f1, 1);
-    static_for<0, STEP_MFMAS>([&](auto x) { mma(f0, f1, x); });
+      // one K-step beside the staging of the next
+      constexpr int LAST = STEP_MFMAS / 6, BESIDE = STEP_MFMAS - LAST;
+      auto step = [&](auto load_tag) {
+        frag_load(f1, 1);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        static_for<0, PA + PB>([&](auto i_tag) {
+          constexpr int I = decltype(i_tag)::value;
+          constexpr int w0 = I < PA ? I * WA : PA * WA + (I - PA) * WB, w1 = w0 + (I < PA ? WA : WB);
+          static_for<BESIDE * w0 / WSUM, BESIDE * w1 / WSUM>([&](auto x) { mma(f0, f1, x); });
+          store_piece(i_tag);
+          if constexpr (decltype(load_tag)::value) load_after(i_tag);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (decltype(load_tag)::value) advance();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        frag_load(f0, 0);
+        static_for<BESIDE, STEP_MFMAS>([&](auto x) { mma(f0, f1, x); });
+      };
+      int t = 0;
+      for (; t + 2 < steps; t++) step(std::true_type{});
+      if (t + 1 < steps) step(std::false_type{});
+      frag_load(f1, 1);
+      static_for<0, STEP_MFMAS>([&](auto x) { mma(f0, f1, x); });
+    }
   }
 
   // ---- sums of the waves ------------------------------------------------------

@@ -21,19 +21,17 @@ struct KWavesForm {
 //
 // All of it fitted on 188 products (84 real, m and n 64 - 4096, K 64 - 8192, 60 real
 // batches of up to 1024 matrices of 32 - 640, 44 complex; four layouts, padded, with
-// and without C), each timed with every form and tiled, in every precision.  On 10000
-// other products that the rule sends here, drawn over the same ranges: time over the
-// tiled time, geometric mean (the fastest side by hindsight); share that is slower by
-// 5 % and 10 %, and the largest loss:
-//               real                             real batches
-//   FP16TCEC    0.65 (0.64) 2.4 %, 1.4 %, 1.25   0.64 (0.63) 3.3 %, 1.7 %, 1.34
-//   bf16x3      0.64 (0.63) 0.7 %, 0.1 %, 1.10   0.64 (0.63) 1.9 %, 1.1 %, 1.15
-//   FP16TC      0.59 (0.58) 3.6 %, 1.9 %, 1.46   0.63 (0.62) 2.4 %, 1.1 %, 1.31
-//   bf16x2      0.64 (0.63) 1.5 %, 0.7 %, 1.33   0.64 (0.63) 2.7 %, 1.3 %, 1.25
-// complex 0.50 - 0.60, none slower by 5 %; AUTO calls 0.84 real, 0.74 complex.
-// (Tried beside these and left out, within 1 %: 64 x 32 and 32 x 64 with four and
-// eight waves, 64 x 64 with one and two; 128 x 64 spills.  Complex with one or two
-// waves: batches are faster tiled.)
+// and without C), each timed with every form and tiled, in every precision; the forms
+// with two waves to a SIMD on 640 others.  On 640 more, time over the tiled time,
+// geometric mean (the fastest side by hindsight): real FP16TCEC 0.72 (0.70), FP16TC
+// 0.69 (0.65), bf16x3 0.72 (0.69), bf16x2 0.72 (0.70); complex 0.60 (0.58), 0.61 (0.58),
+// 0.62 (0.62), 0.68 (0.66); 2 % are slower by 5 %, complex none.  Before there were two
+// waves to a SIMD: 0.73, 0.70, 0.72, 0.73; 0.66, 0.63, 0.62, 0.74.
+// (Tried beside these and left out: 64 x 64 with eight waves at two to a SIMD, up to
+// 10 % faster than four where K >= 2048 and 256 tiles or fewer, 0 - 4 % else, no better
+// over the 640; 64 x 32 and 32 x 64 with four and eight waves, 64 x 64 with one and two,
+// within 1 %; 128 x 64 spills.  Complex with one or two waves: batches are faster tiled;
+// 64 x 32: never ahead of these by 5 %.)
 struct KWavesModel {
   KWavesForm form[kKWavesForms];
   double tiled0, tiled_per_step, tiled_split;
@@ -41,15 +39,15 @@ struct KWavesModel {
 // `prec`: 0 FP16TCEC, 1 FP16TC, 2 bf16x3, 3 bf16x2
 inline const KWavesModel &kwaves_model(int prec, bool cplx) {
   static const KWavesModel real[4] = {
-      {{{64, 64, 4, 1, 3.6, 0.93, 0.0}, {32, 32, 8, 2, 1.13, 0.88, 0.71}, {32, 32, 4, 4, 1.08, 0.50, 0.74}, {32, 32, 1, 16, 2.4, 0.37, 0.22}}, 4.1, 1.63, -2.1},
-      {{{64, 64, 4, 1, 3.0, 0.72, 0.0}, {32, 32, 8, 2, 0.98, 0.87, 0.55}, {32, 32, 4, 4, 1.00, 0.47, 0.67}, {32, 32, 1, 16, 2.4, 0.23, 0.37}}, 4.8, 1.27, 0.9},
+      {{{64, 64, 4, 2, 3.11, 1.10, 0.79}, {32, 32, 8, 2, 1.13, 0.88, 0.71}, {32, 32, 4, 4, 1.08, 0.50, 0.74}, {32, 32, 1, 16, 2.4, 0.37, 0.22}}, 4.1, 1.63, -2.1},
+      {{{64, 64, 4, 2, 2.03, 0.72, 1.41}, {32, 32, 8, 2, 0.98, 0.87, 0.55}, {32, 32, 4, 4, 1.00, 0.47, 0.67}, {32, 32, 1, 16, 2.4, 0.23, 0.37}}, 4.8, 1.27, 0.9},
       {{{64, 64, 4, 1, 3.6, 1.65, 0.0}, {32, 32, 8, 1, 1.62, 1.17, 0.0}, {32, 32, 4, 3, 1.29, 0.76, 0.55}, {32, 32, 1, 12, 2.2, 0.68, 0.17}}, 2.5, 2.29, -2.4},
-      {{{64, 64, 4, 1, 3.7, 0.95, 0.0}, {32, 32, 8, 2, 1.12, 0.87, 0.78}, {32, 32, 4, 4, 1.09, 0.50, 0.73}, {32, 32, 1, 16, 2.5, 0.39, 0.21}}, 4.0, 1.61, -1.6}};
+      {{{64, 64, 4, 2, 2.78, 1.04, 0.90}, {32, 32, 8, 2, 1.12, 0.87, 0.78}, {32, 32, 4, 4, 1.09, 0.50, 0.73}, {32, 32, 1, 16, 2.5, 0.39, 0.21}}, 4.0, 1.61, -1.6}};
   static const KWavesModel complex[4] = {
-      {{{32, 32, 4, 1, 2.2, 1.02, 0.0}, {64, 32, 4, 1, 3.5, 1.67, 0.0}, {}, {}}, 2.8, 2.05, -5.4},
-      {{{32, 32, 4, 1, 1.8, 0.74, 0.0}, {64, 32, 4, 1, 2.2, 1.12, 0.0}, {}, {}}, 3.6, 1.50, -3.4},
+      {{{32, 32, 4, 2, 1.50, 1.02, 0.94}, {32, 32, 8, 1, 1.15, 1.77, 0.0}, {}, {}}, 2.8, 2.05, -5.4},
+      {{{32, 32, 4, 2, 1.09, 0.51, 1.72}, {32, 32, 8, 1, 0.74, 1.28, 0.0}, {}, {}}, 3.6, 1.50, -3.4},
       {{{32, 32, 4, 1, 2.3, 1.71, 0.0}, {}, {}, {}}, 0.9, 3.83, -14.3},
-      {{{32, 32, 4, 1, 2.2, 1.06, 0.0}, {64, 32, 4, 1, 3.7, 1.72, 0.0}, {}, {}}, 3.1, 2.09, -6.1}};
+      {{{32, 32, 4, 2, 1.55, 0.97, 1.06}, {32, 32, 8, 1, 0.99, 1.85, 0.0}, {}, {}}, 3.1, 2.09, -6.1}};
   return (cplx ? complex : real)[prec];
 }
 
@@ -96,8 +94,9 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
   const double tiled = model.tiled0 + layout * model.tiled_per_step * tiled_steps + (tiled_split ? model.tiled_split : 0.0);
   // Both sides are estimates, within 10 - 30 % of the times: with 1.0 here the number of products that get more than
   // 3 % slower doubles and the mean stays; with 0.8 (long ones 0.7) a third of the losses is left, and the mean of 10000
-  // real products goes from 0.643 to 0.660 of the tiled time.  Long ones have less to gain: 0.8.
-  double best_time = (tiled > 30.0 ? 0.8 : 0.9) * tiled;
+  // real products goes from 0.643 to 0.660 of the tiled time.  Long ones have less to gain: 0.8.  (Complex ones: 0.95;
+  // 3 of 240 slower by 5 %, with 1.0 for short ones 5.)
+  double best_time = (p.cplx ? 0.95 : tiled > 30.0 ? 0.8 : 0.9) * tiled;
   int best = -1;
   for (int i = 0; i < kKWavesForms; i++) {
     const KWavesForm &f = model.form[i];
@@ -118,7 +117,7 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
       best_time = t;
     }
   }
-  if (asked < 0 && best >= 0 && model.form[best].waves == 8) {
+  if (asked < 0 && !p.cplx && best >= 0 && model.form[best].waves == 8) {
     // Eight waves on a tile pay while all workgroups are on the chip at once: the fit makes their second round too cheap.
     // 36 of 10000 drawn products were sent to one.  The 32 up to K = 512 take 0.72 - 1.01 of the time with four waves on
     // the same tile (2560 x 586 x 224 FP16TC NN, us: 9.1, four waves 6.8, tiled 6.7; 231^3 x 22 NT 11.4, 8.9, 11.1).

@@ -14,7 +14,7 @@ FP32, AUTO, SCALING = 12, 9, 11
 KWAVES = 6  # module id
 
 LAYOUTS = [(False, N, N), (False, T, N), (False, N, T), (False, T, T), (True, N, N), (True, C, N), (True, N, C), (True, T, T)]
-# (form 1: 64 x 64, four waves, 2, 3, 4: 32 x 32, eight, four, one; complex 1: 32 x 32, 2: 64 x 32; 32 K-values a step)
+# (form 1: 64 x 64, four waves, 2, 3, 4: 32 x 32, eight, four, one; complex 32 x 32, 1: four, 2: eight; 32 K-values a step)
 SIZES = [(64, 64, 1), (65, 129, 31), (70, 100, 33), (127, 64, 128), (96, 65, 160), (129, 70, 257), (64, 130, 995), (200, 90, 64)]
 NARROWER = [(1, 1, 40), (31, 5, 33), (40, 17, 300)]  # than a tile: K-contiguous operands only
 
@@ -197,3 +197,21 @@ def test_complex_two_wave_groups_are_exact_on_integers(O, handle, dev, monkeypat
             co = oracle_gemm(O, FP16TCEC if mode == SCALING else mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, beta,
                              c0.copy(), m)
             assert np.array_equal(c, co), (m, n, k, beta)
+
+
+@pytest.mark.parametrize("mode", [FP16TCEC, FP16TC, TF32TC])
+@pytest.mark.parametrize("cplx,opa,opb,m,n,k", [(False, N, N, 1100, 1000, 290), (False, T, N, 1090, 1030, 257),
+                                                (False, N, T, 1153, 1000, 161), (True, N, N, 580, 540, 290),
+                                                (True, N, C, 577, 545, 130)])
+def test_more_tiles_than_cus_are_exact_on_integers(O, handle, dev, monkeypatch, mode, cplx, opa, opb, m, n, k):
+    """Two workgroups of the 64 x 64 (complex 32 x 32) form on one CU."""
+    monkeypatch.setenv("CUMPSGEMM_KWAVES", "1")
+    rng = np.random.default_rng(9)
+    a, lda = _padded_ints(rng, opa, m, k, 3, cplx)
+    b, ldb = _padded_ints(rng, opb, k, n, 1, cplx)
+    c0 = rng.integers(-9, 10, m * n).astype(np.complex64 if cplx else np.float32)
+    c, st, mid = run_gemm(handle, dev, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, 1.0, c0.copy(), m, cplx,
+                          want_module_id=True)
+    assert (st, mid) == (0, KWAVES)
+    # |x| <= 30: every partial sum is an integer below 2^24
+    assert np.array_equal(c, oracle_gemm(O, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, 1.0, c0.copy(), m))
