@@ -1,7 +1,8 @@
 """Python binding of libcumpsgemm.so, the MI355X (gfx950) split-and-correct
-SGEMM/CGEMM library.  Thin ctypes layer over the C ABI declared in
-include/cumpsgemm/cumpsgemm.h and include/cumpsgemm/cumpsgemm_ext.h; device
-memory is passed as raw pointers (ints) or as objects with ``data_ptr()``.
+SGEMM/CGEMM library.  Thin layer over the C ABI declared in
+include/cumpsgemm/cumpsgemm.h and include/cumpsgemm/cumpsgemm_ext.h: ctypes, and
+for the products csrc/call.cpp; device memory is passed as raw pointers (ints) or
+as objects with ``data_ptr()``.
 
 There is no CPU fallback: if the shared library is missing, loading raises.
 """

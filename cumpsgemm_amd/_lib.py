@@ -41,11 +41,17 @@ def build(jobs=8):
 
 
 _lib = None
+# csrc/call.cpp: converts the arguments of the calls that programs make often at a sixth of what ctypes
+# takes.  Its functions return None, with nothing done, for arguments of unusual types.
+_native = None
+_CALL_FUNCTIONS = ("cuMpSGEMM_sgemm", "cuMpSGEMM_cgemm", "cuMpSGEMM_sgemm_strided_batch", "cuMpSGEMM_cgemm_strided_batch",
+                   "cuMpSGEMM_sgemm_pipeline", "cuMpSGEMM_cgemm_pipeline", "cuMpSGEMM_sgemm_Mx2x2",
+                   "cuMpSGEMM_cgemm_Mx2x2", "cuMpSGEMM_sgemm_2xNx2", "cuMpSGEMM_cgemm_2xNx2")
 
 
 def lib():
     """The loaded shared library (raises if it has not been built)."""
-    global _lib
+    global _lib, _native
     if _lib is None:
         if not os.path.exists(_LIB):
             raise RuntimeError(
@@ -61,6 +67,12 @@ def lib():
             pass
         L = ctypes.CDLL(_LIB)
         _declare(L)
+        try:
+            from . import _call
+            _call.bind(*(ctypes.cast(getattr(L, name), _ptr).value for name in _CALL_FUNCTIONS))
+            _native = _call
+        except ImportError:
+            _native = None  # not built: every call goes through ctypes
         _lib = L
     return _lib
 
@@ -196,13 +208,14 @@ class Handle:
         if st != STATUS_SUCCESS:
             raise RuntimeError(f"cuMpSGEMM_create failed with hipblasStatus {st}")
         self._h = h
+        self._addr = h.value
         if stream is not None:
             self.set_stream(stream)
 
     def close(self):
         if getattr(self, "_h", None):
             self._L.cuMpSGEMM_destroy(self._h)
-            self._h = None
+            self._h = self._addr = None
 
     def __del__(self):
         try:
@@ -229,6 +242,10 @@ class Handle:
     # ---- GEMM ----
     def gemm(self, op_a, op_b, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, mode, cplx=False,
              want_module_id=False):
+        if _native is not None and not want_module_id:
+            st = _native.gemm(cplx, self._addr, op_a, op_b, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, mode)
+            if st is not None:
+                return st
         fn = self._L.cuMpSGEMM_cgemm_ex if cplx else self._L.cuMpSGEMM_sgemm_ex
         mid = _u32(0)
         st = fn(self._h, op_a, op_b, m, n, k, _scalar(alpha, cplx), _dptr(a), lda, _dptr(b), ldb,
@@ -243,12 +260,22 @@ class Handle:
 
     def gemm_strided_batch(self, op_a, op_b, m, n, k, alpha, a, lda, stridea, b, ldb, strideb, beta,
                            c, ldc, stridec, batch, mode, cplx=False):
+        if _native is not None:
+            st = _native.strided_batch(cplx, self._addr, op_a, op_b, m, n, k, alpha, a, lda, stridea, b, ldb, strideb,
+                                       beta, c, ldc, stridec, batch, mode)
+            if st is not None:
+                return st
         fn = self._L.cuMpSGEMM_cgemm_strided_batch if cplx else self._L.cuMpSGEMM_sgemm_strided_batch
         return fn(self._h, op_a, op_b, m, n, k, _scalar(alpha, cplx), _dptr(a), lda, stridea,
                   _dptr(b), ldb, strideb, _scalar(beta, cplx), _dptr(c), ldc, stridec, batch, int(mode))
 
     def gemm_pipeline(self, op_a, op_b, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, mode,
                       cplx=False, stridea=0, strideb=0, stridec=0, batch=1, restore_ab=True):
+        if _native is not None:
+            st = _native.pipeline(cplx, self._addr, op_a, op_b, m, n, k, alpha, a, lda, stridea, b, ldb, strideb, beta, c,
+                                  ldc, stridec, batch, mode, 1 if restore_ab else 0)
+            if st is not None:
+                return st
         fn = self._L.cuMpSGEMM_cgemm_pipeline if cplx else self._L.cuMpSGEMM_sgemm_pipeline
         ids = (_u32 * 3)()
         st = fn(self._h, op_a, op_b, m, n, k, _scalar(alpha, cplx), _dptr(a), lda, stridea, _dptr(b),
@@ -258,12 +285,22 @@ class Handle:
 
     def gemm_Mx2x2(self, op_a, op_b, m, alpha, a, lda, b, ldb, beta, c, ldc, cplx=False,
                    stridea=0, strideb=0, stridec=0, batch=1):
+        if _native is not None:
+            st = _native.mx2x2(cplx, self._addr, op_a, op_b, m, alpha, a, lda, stridea, b, ldb, strideb, beta, c, ldc,
+                               stridec, batch)
+            if st is not None:
+                return st
         fn = self._L.cuMpSGEMM_cgemm_Mx2x2 if cplx else self._L.cuMpSGEMM_sgemm_Mx2x2
         return fn(self._h, op_a, op_b, m, _scalar(alpha, cplx), _dptr(a), lda, stridea, _dptr(b),
                   ldb, strideb, _scalar(beta, cplx), _dptr(c), ldc, stridec, batch)
 
     def gemm_2xNx2(self, op_a, op_b, n, alpha, a, lda, b, ldb, beta, c, ldc, cplx=False,
                    stridea=0, strideb=0, stridec=0, batch=1):
+        if _native is not None:
+            st = _native.twoxnx2(cplx, self._addr, op_a, op_b, n, alpha, a, lda, stridea, b, ldb, strideb, beta, c, ldc,
+                                 stridec, batch)
+            if st is not None:
+                return st
         fn = self._L.cuMpSGEMM_cgemm_2xNx2 if cplx else self._L.cuMpSGEMM_sgemm_2xNx2
         return fn(self._h, op_a, op_b, n, _scalar(alpha, cplx), _dptr(a), lda, stridea, _dptr(b),
                   ldb, strideb, _scalar(beta, cplx), _dptr(c), ldc, stridec, batch)

@@ -426,6 +426,7 @@ PreSplitChoice choose_pre_split(const cuMpSGEMM_handle *h, bool a_kc, bool b_kc,
   // (the pre-pass launches workgroups of 64 rows x 32 .. 256 K-values on a 2-D grid)
   const bool shape_ok = batch == 1 && k >= 128 &&
                         (forced || (uint64_t)m * n >= (uint64_t)h->num_cus * ch.bm * ch.bn) && k / 32 < 65535;
+  if (!shape_ok) return ch; // (neither taken nor cut)
   const double mn_ratio = (double)m * (double)n / ((double)m + (double)n);
   // (in-loop -> pre-split, TFLOP/s: 4096^2 x 256 198 -> 211, 4096^2 x 384 224 -> 260, 5120^2 x 256 176 -> 209,
   // 3072^2 x 512 177 -> 191, 3072^2 x 1024 201 -> 237, 8192 x 4096 x 256 211 -> 245, 4096 x 8192 x 384 232 -> 316;
@@ -507,7 +508,7 @@ PreSplitChoice choose_pre_split(const cuMpSGEMM_handle *h, bool a_kc, bool b_kc,
   const bool mode_ok = mode == CUMPSGEMM_FP16TCEC || ch.bf16 || ch.auto_ok || ch.tc_only;
   // (CUMPSGEMM_FORCE_TILE_CLASS / _FORCE_KSPLIT pick among the in-loop kernels and keep a call off this
   // path -- except a call of the entry point that allocates nothing, which is defined to take it)
-  const bool base_ok = mode_ok && !never && shape_ok && (forced || (force_cls <= 0 && force_split <= 1));
+  const bool base_ok = mode_ok && !never && (forced || (force_cls <= 0 && force_split <= 1));
   ch.take = base_ok && worth_if(rounds_ok);
   // With a mostly empty last round the path still pays for the rounds before
   // it: the caller cuts C there (6000^2 x 2048: 332 TFLOP/s in-loop, 384 with

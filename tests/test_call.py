@@ -1,0 +1,122 @@
+"""The native calls of the Python binding (csrc/call.cpp) against the ctypes ones: the same arguments arrive, and what
+is not of the usual types is converted or refused as ctypes does."""
+import ctypes
+import subprocess
+
+import numpy as np
+import pytest
+import torch
+
+import cumpsgemm_amd as cg
+from cumpsgemm_amd import _lib
+
+STUB = """
+#include <stdint.h>
+#include <string.h>
+extern "C" {
+double got[32];
+static int put(int n, const double *v) { memcpy(got, v, n * sizeof(double)); return n; }
+#define P(x) (double)(uintptr_t)(x)
+#define V P(h), (double)oa, (double)ob
+int sgemm(void *h, int oa, int ob, uint64_t m, uint64_t n, uint64_t k, const float *al, void *a, uint64_t lda, void *b,
+          uint64_t ldb, const float *be, void *c, uint64_t ldc, int mode) {
+  const double v[] = {V, (double)m, (double)n, (double)k, al[0], P(a), (double)lda, P(b), (double)ldb, be[0], P(c), (double)ldc, (double)mode};
+  return put(15, v); }
+int cgemm(void *h, int oa, int ob, uint64_t m, uint64_t n, uint64_t k, const float *al, void *a, uint64_t lda, void *b,
+          uint64_t ldb, const float *be, void *c, uint64_t ldc, int mode) {
+  const double v[] = {V, (double)m, (double)n, (double)k, al[0], al[1], P(a), (double)lda, P(b), (double)ldb, be[0], be[1], P(c), (double)ldc, (double)mode};
+  return put(17, v); }
+int sbatch(void *h, int oa, int ob, uint64_t m, uint64_t n, uint64_t k, const float *al, void *a, uint64_t lda, uint64_t sa,
+           void *b, uint64_t ldb, uint64_t sb, const float *be, void *c, uint64_t ldc, uint64_t sc, uint64_t batch, int mode) {
+  const double v[] = {V, (double)m, (double)n, (double)k, al[0], P(a), (double)lda, (double)sa, P(b), (double)ldb, (double)sb, be[0], P(c), (double)ldc, (double)sc, (double)batch, (double)mode};
+  return put(19, v); }
+int cbatch(void *h, int oa, int ob, uint64_t m, uint64_t n, uint64_t k, const float *al, void *a, uint64_t lda, uint64_t sa,
+           void *b, uint64_t ldb, uint64_t sb, const float *be, void *c, uint64_t ldc, uint64_t sc, uint64_t batch, int mode) {
+  const double v[] = {V, (double)m, (double)n, (double)k, al[0], al[1], P(a), (double)lda, (double)sa, P(b), (double)ldb, (double)sb, be[0], be[1], P(c), (double)ldc, (double)sc, (double)batch, (double)mode};
+  return put(21, v); }
+int spipe(void *h, int oa, int ob, uint64_t m, uint64_t n, uint64_t k, const float *al, void *a, uint64_t lda, uint64_t sa,
+          void *b, uint64_t ldb, uint64_t sb, const float *be, void *c, uint64_t ldc, uint64_t sc, uint64_t batch, int mode,
+          int restore, unsigned *ids) {
+  ids[0] = 7; ids[1] = 8; ids[2] = 9u + restore;
+  return sbatch(h, oa, ob, m, n, k, al, a, lda, sa, b, ldb, sb, be, c, ldc, sc, batch, mode); }
+int cpipe(void *h, int oa, int ob, uint64_t m, uint64_t n, uint64_t k, const float *al, void *a, uint64_t lda, uint64_t sa,
+          void *b, uint64_t ldb, uint64_t sb, const float *be, void *c, uint64_t ldc, uint64_t sc, uint64_t batch, int mode,
+          int restore, unsigned *ids) {
+  ids[0] = 7; ids[1] = 8; ids[2] = 9u + restore;
+  return cbatch(h, oa, ob, m, n, k, al, a, lda, sa, b, ldb, sb, be, c, ldc, sc, batch, mode); }
+int s2x2(void *h, int oa, int ob, uint64_t m, const float *al, void *a, uint64_t lda, uint64_t sa, void *b, uint64_t ldb,
+         uint64_t sb, const float *be, void *c, uint64_t ldc, uint64_t sc, uint64_t batch) {
+  return sbatch(h, oa, ob, m, 0, 0, al, a, lda, sa, b, ldb, sb, be, c, ldc, sc, batch, 0); }
+int c2x2(void *h, int oa, int ob, uint64_t m, const float *al, void *a, uint64_t lda, uint64_t sa, void *b, uint64_t ldb,
+         uint64_t sb, const float *be, void *c, uint64_t ldc, uint64_t sc, uint64_t batch) {
+  return cbatch(h, oa, ob, m, 0, 0, al, a, lda, sa, b, ldb, sb, be, c, ldc, sc, batch, 0); }
+}
+"""
+NAMES = ("sgemm", "cgemm", "sbatch", "cbatch", "spipe", "cpipe", "s2x2", "c2x2", "s2x2", "c2x2")
+
+
+@pytest.fixture
+def calls(tmp_path):
+    """(handle without a library behind it, the arguments its last call passed)"""
+    assert _lib.lib() is not None and _lib._native is not None, "csrc/call.cpp is not built"
+    (tmp_path / "stub.cpp").write_text(STUB)
+    so = tmp_path / "stub.so"
+    subprocess.check_call(["g++", "-shared", "-fPIC", "-o", str(so), str(tmp_path / "stub.cpp")])
+    stub = ctypes.CDLL(str(so))
+    address = [ctypes.cast(getattr(stub, n), ctypes.c_void_p).value for n in NAMES]
+    real = [ctypes.cast(getattr(_lib.lib(), n), ctypes.c_void_p).value for n in _lib._CALL_FUNCTIONS]
+    h = cg.Handle.__new__(cg.Handle)
+    h._L, h._h, h._addr = _lib.lib(), None, 0x1230
+    got = (ctypes.c_double * 32).in_dll(stub, "got")
+    _lib._native.bind(*address)
+    yield h, got
+    _lib._native.bind(*real)
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+def test_every_argument_arrives_in_its_place(calls, cplx):
+    h, got = calls
+    a, b, c = torch.zeros(4), torch.zeros(4), torch.zeros(4)
+    pa, pb, pc = a.data_ptr(), b.data_ptr(), c.data_ptr()
+    al, be = (2.5 - 1.5j, 0.5 + 0.25j) if cplx else (2.5, 0.5)
+    sc = [2.5, -1.5] if cplx else [2.5], [0.5, 0.25] if cplx else [0.5]
+    st = h.gemm(111, 112, 3, 4, 5, al, a, 6, pb, 7, be, c, 8, 1, cplx=cplx)
+    assert list(got)[:st] == [0x1230, 111, 112, 3, 4, 5, *sc[0], pa, 6, pb, 7, *sc[1], pc, 8, 1]
+    batch = [*sc[0], pa, 6, 60, pb, 7, 70, *sc[1], pc, 8, 80]
+    st = h.gemm_strided_batch(111, 112, 3, 4, 5, al, a, 6, 60, b, 7, 70, be, c, 8, 80, 9, 2, cplx=cplx)
+    assert list(got)[:st] == [0x1230, 111, 112, 3, 4, 5, *batch, 9, 2]
+    st, ids = h.gemm_pipeline(111, 112, 3, 4, 5, al, a, 6, b, 7, be, c, 8, 9, cplx=cplx, stridea=60, strideb=70, stridec=80,
+                              batch=9, restore_ab=True)
+    assert list(got)[:st] == [0x1230, 111, 112, 3, 4, 5, *batch, 9, 9] and ids == (7, 8, 10)
+    for f in (h.gemm_Mx2x2, h.gemm_2xNx2):
+        st = f(111, 112, 3, al, a, 6, b, 7, be, c, 8, cplx=cplx, stridea=60, strideb=70, stridec=80, batch=9)
+        assert list(got)[:st] == [0x1230, 111, 112, 3, 0, 0, *batch, 9, 0]
+    # a real scalar of a complex product; a null pointer
+    st = h.gemm(111, 112, 3, 4, 5, 1.0, None, 6, b, 7, 0.0, c, 8, 1, cplx=cplx)
+    assert list(got)[6:st] == [1, *[0] * cplx, 0, 6, pb, 7, 0, *[0] * cplx, pc, 8, 1]
+
+
+class Pointer:
+    def data_ptr(self):
+        raise ValueError("gone")
+
+
+@pytest.mark.parametrize("where,value", [
+    (2, np.int64(3)), (2, 3.0), (2, "3"), (2, -1), (2, 1 << 70), (0, np.int32(111)), (0, True), (5, 1), (5, np.float32(1)),
+    (5, 1j), (5, "x"), (5, None), (5, torch.tensor(1.0)), (6, 0), (6, np.zeros(4)), (6, Pointer()), (6, "a"), (13, 1.0), (13, np.int64(1))])
+def test_other_types_are_what_ctypes_makes_of_them(monkeypatch, where, value):
+    """Without a handle the library itself refuses the call: status 3 from either side, or the exception of ctypes."""
+    _lib.lib()
+    h = cg.Handle.__new__(cg.Handle)
+    h._L, h._h, h._addr = _lib.lib(), None, None
+    args = [111, 111, 2, 2, 2, 1.0, 16, 2, 16, 2, 0.0, 16, 2, 1]
+    args[where] = value
+
+    def outcome():
+        try:
+            return h.gemm(*args)
+        except Exception as e:  # noqa: BLE001
+            return type(e)
+    native = outcome()
+    monkeypatch.setattr(_lib, "_native", None)
+    assert native == outcome()
