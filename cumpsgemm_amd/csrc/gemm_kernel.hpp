@@ -900,7 +900,8 @@ struct tile_loader {
 
   // split and write to LDS: planes laid out [comp][plane][row][chunk]
   // SCALED: the values are multiplied by s (s2048 = s * 2^11) on the way
-  template <Prec P, bool SCALED = false>
+  // BY_PAIRS: split by `split_pair`
+  template <Prec P, bool SCALED = false, bool BY_PAIRS = false>
   __device__ static inline void store(Regs &reg, char *lds_op, int tid, float s = 1.0f,
                                       float s2048 = 2048.0f) {
     constexpr int NP = prec_traits<P>::NP;
@@ -938,7 +939,15 @@ struct tile_loader {
 #pragma unroll
       for (int c = 0; c < NC; c++) {
         u4_t out[NP];
-        if constexpr (SCALED) {
+        if constexpr (BY_PAIRS) {
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            uint32_t terms[NP];
+            split_pair<P, SCALED>(part[c][2 * q], part[c][2 * q + 1], s, s2048, terms);
+#pragma unroll
+            for (int p = 0; p < NP; p++) out[p][q] = terms[p];
+          }
+        } else if constexpr (SCALED) {
           splitter<P>::run_scaled(part[c], out, s, s2048);
         } else {
           splitter<P>::run(part[c], out);
@@ -1169,8 +1178,12 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void gemm_tcec_kernel(c
         LB::template store_packed<NP * NCOMP>(rb, sb, tid);
       }
     } else {
-      LA::template store<P, Cfg::SCALED>(ra, sa, tid, coef_a, coef_a2048);
-      LB::template store<P, Cfg::SCALED>(rb, sb, tid, coef_b, coef_b2048);
+      // (FP16TCEC on 16x16x32 MFMAs, 256x128 and 128x256: full-rate instructions though more of them, us: 512^3 x 64 NN
+      // 63.0 -> 57.9, TT 61.0 -> 56.9, 1024^3 x 8 54.6 -> 52.4, 4096^2 x 256 TT 36.8 -> 34.0.  On 32x32x16 MFMAs, whose
+      // schedule then puts vector instructions behind the last of them, 3000^2 x 768 NN 64.8 -> 69.3.)
+      constexpr bool BY_PAIRS = P == Prec::FP16TCEC && !CPLX && Cfg::MT == 16 && BM * BN == 256 * 128;
+      LA::template store<P, Cfg::SCALED, BY_PAIRS>(ra, sa, tid, coef_a, coef_a2048);
+      LB::template store<P, Cfg::SCALED, BY_PAIRS>(rb, sb, tid, coef_b, coef_b2048);
     }
   };
 
