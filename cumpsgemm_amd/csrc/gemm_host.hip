@@ -959,6 +959,23 @@ hipblasStatus_t run_gemm(cuMpSGEMM_handle *h, hipblasOperation_t op_A,
   }
   (void)beta_zero;
 
+  // AUTO, both candidates of the pipeline in one launch
+  if (nlaunch == 2 && h->fused_scaling) {
+    const KWavesProblem problem{CPLX, a_kc, b_kc, m, n, k, batch, lda, ldb};
+    const int form = choose_kwaves_either_form(problem, h->num_cus, kwaves[0], kwaves[1]);
+    if (form >= 0) {
+      const KWavesForm &f = kwaves_model((int)Prec::FP16TCEC, CPLX).form[form];
+      args.tiles_m = (uint32_t)((m + f.bm - 1) / f.bm);
+      args.tiles_n = (uint32_t)((n + f.bn - 1) / f.bn);
+      args.batch = (uint32_t)batch;
+      set_fused_scaling(args);
+      const int layout = (a_kc ? 1 : 0) + (b_kc ? 2 : 0);
+      (CPLX ? g_kwaves_either_c : g_kwaves_either_s)[layout][form](
+          args, launches[0].accept, launches[1].accept, dim3(args.tiles_m * args.tiles_n * args.batch, 1, 1), h->stream);
+      if (used_id != nullptr) *used_id = ~0u;
+      nlaunch = 0;
+    }
+  }
   for (int i = 0; i < nlaunch; i++) {
     if (kwaves[i] >= 0) {
       const KWavesForm &f = kwaves_model((int)launches[i].p, CPLX).form[kwaves[i]];

@@ -204,18 +204,13 @@ template <int LO, int HI, class F> __device__ inline void static_for(F &&f) {
   }
 }
 
-template <class Cfg>
-__global__ __launch_bounds__(Cfg::NT)
-__attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void kwaves_gemm_tcec_kernel(const GemmArgs args) {
+// The product (called by the kernels at the end of this file).
+template <class Cfg> __device__ inline void kwaves_product(const GemmArgs &args) {
   constexpr Prec P = Cfg::P;
   using PT = prec_traits<P>;
   constexpr bool CPLX = Cfg::CPLX;
   constexpr int BM = Cfg::BM, BN = Cfg::BN, TM = Cfg::TM, TN = Cfg::TN, NP = Cfg::NP, NC = Cfg::NC, W = Cfg::W;
 
-  if (args.launch_flag != nullptr) {
-    const int flag = *args.launch_flag;
-    if (((1u << (flag & 31)) & args.flag_accept_mask) == 0) return;
-  }
   float coef_a = 1.0f, coef_b = 1.0f, coef_c = 1.0f;
   if constexpr (Cfg::SCALED) {
     const int sflag = *args.scale_flag;
@@ -504,5 +499,30 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void kwaves_gemm_tcec_k
         if (inside(x, e / NC)) p[e] = out[e];
     }
   }
+}
+
+__device__ inline bool kwaves_accepts(const int flag, const uint32_t mask) { return ((1u << (flag & 31)) & mask) != 0; }
+
+template <class Cfg>
+__global__ __launch_bounds__(Cfg::NT)
+__attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void kwaves_gemm_tcec_kernel(const GemmArgs args) {
+  if (args.launch_flag != nullptr && !kwaves_accepts(*args.launch_flag, args.flag_accept_mask)) return;
+  kwaves_product<Cfg>(args);
+}
+
+// Both of AUTO's candidates, on the same tile: the launch flag says which product a
+// workgroup computes, instead of a launch each of which one finds nothing to do.  What
+// bounds a call this small is the boundaries between its kernels: statistics, decision
+// and one product instead of two.  us, whole calls, decided for FP16TCEC / bf16x3: 64^3
+// 8.9 -> 7.3 / 10.7 -> 8.8, 512^3 NN 15.5 -> 13.9 / 21.4 -> 19.5, 1200^3 NN 41.4 -> 37.2 /
+// 58.8 -> 54.2; complex 128^3 12.3 -> 11.0 / 16.6 -> 14.5, 512^3 18.9 -> 17.6 / 27.0 -> 25.0.
+template <class CfgA, class CfgB>
+__global__ __launch_bounds__(CfgA::NT)
+__attribute__((amdgpu_waves_per_eu(CfgA::OCC < CfgB::OCC ? CfgA::OCC : CfgB::OCC, CfgA::OCC < CfgB::OCC ? CfgA::OCC : CfgB::OCC)))
+void kwaves_either_gemm_tcec_kernel(const GemmArgs args, const uint32_t accept_a, const uint32_t accept_b) {
+  static_assert(CfgA::NT == CfgB::NT && CfgA::BM == CfgB::BM && CfgA::BN == CfgB::BN, "one grid for both");
+  const int flag = *args.launch_flag;
+  if (kwaves_accepts(flag, accept_a)) kwaves_product<CfgA>(args);
+  else if (kwaves_accepts(flag, accept_b)) kwaves_product<CfgB>(args);
 }
 } // namespace cumpsgemm_amd

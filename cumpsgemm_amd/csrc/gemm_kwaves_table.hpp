@@ -21,4 +21,9 @@ CUMPSGEMM_DECLARE_KWAVES(bf16x3_c)
 CUMPSGEMM_DECLARE_KWAVES(bf16x2_s)
 CUMPSGEMM_DECLARE_KWAVES(bf16x2_c)
 #undef CUMPSGEMM_DECLARE_KWAVES
+
+// AUTO: bf16x3 or FP16TCEC with fused scaling, by the launch flag; [layout][form], nullptr: no such form.
+typedef void (*kwaves_either_t)(const GemmArgs &, uint32_t accept_bf16, uint32_t accept_fp16, dim3 grid, hipStream_t stream);
+extern kwaves_either_t g_kwaves_either_s[4][kKWavesForms];
+extern kwaves_either_t g_kwaves_either_c[4][kKWavesForms];
 } // namespace cumpsgemm_amd

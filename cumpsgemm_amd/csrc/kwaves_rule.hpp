@@ -2,6 +2,7 @@
 // tile.  Host arithmetic on sizes and layouts alone.
 #pragma once
 #include <cstdint>
+#include <initializer_list>
 
 namespace cumpsgemm_amd {
 
@@ -132,6 +133,32 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
       // products, 19 of them 1.05 - 1.63 times as long as with K split (1090 x 256 x 3360 FP16TC 34.0 us, tiled 22.3;
       // FP16TCEC 528 x 528 x 2880 24.3, 22.3).  K 2048 - 2559: 8 of 18 longer, 7 shorter; other layouts level.
       best = -1;
+    }
+  }
+  return best;
+}
+
+// AUTO's candidates (bf16x3, FP16TCEC) where both go to this kernel with the forms given: which of the two forms one
+// launch takes for both, or -1: a launch each.  Apart, a call pays for the launch that finds nothing to do (1.7 us in a
+// graph, 3 - 5 in a loop of calls); together they hold as many workgroups on a CU as the larger of them, which must
+// cost neither more than that (complex 640^3, 400 tiles: FP16TCEC runs two to a CU apart, 26.5 us a call, and one
+// together, 27.3).
+inline int choose_kwaves_either_form(const KWavesProblem &p, unsigned cus, int form_bf16, int form_fp16) {
+  constexpr double LAUNCH = 1.7;
+  if (form_bf16 < 0 || form_fp16 < 0) return -1;
+  const KWavesModel &ma = kwaves_model(2, p.cplx), &mb = kwaves_model(0, p.cplx);
+  const double apart_a = kwaves_time(ma.form[form_bf16], p, cus), apart_b = kwaves_time(mb.form[form_fp16], p, cus);
+  double best_time = apart_a + apart_b + 2 * LAUNCH;
+  int best = -1;
+  for (const int i : {form_fp16, form_bf16}) {
+    KWavesForm a = ma.form[i], b = mb.form[i];
+    if (a.bm == 0 || b.bm == 0 || a.waves != b.waves || !kwaves_can_serve(a, p)) continue;
+    a.resident = b.resident = a.resident < b.resident ? a.resident : b.resident;
+    if (a.waves == 8 && (kwaves_tiles(a, p) + cus - 1) / cus > (uint64_t)a.resident) continue; // (one round only, as above)
+    const double ta = kwaves_time(a, p, cus), tb = kwaves_time(b, p, cus);
+    if (ta < apart_a + LAUNCH && tb < apart_b + LAUNCH && ta + tb < best_time) {
+      best = i;
+      best_time = ta + tb;
     }
   }
   return best;

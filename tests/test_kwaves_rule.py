@@ -27,6 +27,11 @@ def rule(tmp_path_factory):
             tile[0] = x.bm, tile[1] = x.bn, tile[2] = x.waves;
           }
           return f;
+        }
+        extern "C" int either(int cplx, int a_kc, int b_kc, uint64_t m, uint64_t n, uint64_t k, uint64_t batch, uint64_t lda,
+                              uint64_t ldb, int form_bf16, int form_fp16) {
+          return choose_kwaves_either_form({cplx != 0, a_kc != 0, b_kc != 0, m, n, k, batch, lda, ldb}, 256, form_bf16,
+                                           form_fp16);
         }""")
     so = d / "rule.so"
     subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, "-o", str(so), str(d / "rule.cpp")])
@@ -39,6 +44,11 @@ def rule(tmp_path_factory):
         f = lib.form(prec, int(cplx), int(op[0] != "N"), int(op[1] == "N"), u64(m), u64(n), u64(k), u64(batch), u64(lda),
                      u64(ldb), ctypes.c_double(steps), int(split), asked, tile)
         return (f, *tile) if f >= 0 else None
+
+    def either(cplx, op, m, n, k, batch, form_bf16, form_fp16):
+        return lib.either(int(cplx), int(op[0] != "N"), int(op[1] == "N"), u64(m), u64(n), u64(k), u64(batch),
+                          u64(m if op[0] == "N" else k), u64(k if op[1] == "N" else n), form_bf16, form_fp16)
+    call.either = either
     return call
 
 
@@ -93,3 +103,26 @@ def test_a_long_k_of_two_row_contiguous_operands_is_split(rule, prec, m, n, k, s
     assert rule(prec, False, "NT", m, n, k, steps=steps, split=True) is None
     for op, kk, split in (("TN", k, True), ("NT", 1500, True), ("NT", k, False)):
         assert rule(prec, False, op, m, n, kk, steps=2 * steps, split=split) is not None
+
+
+@pytest.mark.parametrize("op", ["NN", "TN", "NT", "TT"])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_one_launch_for_both_candidates_of_auto(rule, cplx, op):
+    """It takes the form of one of the two, which can serve the product in either precision; none where a candidate is
+    not here or where FP16TCEC would lose its second workgroup per CU."""
+    taken = 0
+    sizes = (1, 31, 32, 64, 100, 512, 640, 1200, 1 << 26, (1 << 31) - 1)
+    for m, n, k, batch in itertools.product(sizes, sizes, (1, 100, 1000, (1 << 31) - 1), (1, 65535)):
+        a, b = rule(2, cplx, op, m, n, k, batch), rule(0, cplx, op, m, n, k, batch)
+        form = rule.either(cplx, op, m, n, k, batch, a[0] if a else -1, b[0] if b else -1)
+        if form < 0:
+            continue
+        taken += 1
+        assert form in (a[0], b[0])
+        tiles = [rule(prec, cplx, op, m, n, k, batch, asked=form + 1) for prec in (2, 0)]
+        assert tiles[0] is not None and tiles[0] == tiles[1]
+    assert taken > 50
+    assert rule.either(cplx, op, 512, 512, 512, 1, 0, -1) == rule.either(cplx, op, 512, 512, 512, 1, -1, 0) == -1
+    assert rule.either(cplx, op, 512, 512, 512, 1, 0, 0) == 0
+    if cplx:
+        assert rule.either(cplx, op, 640, 640, 640, 1, 0, 0) == -1
