@@ -130,6 +130,29 @@ template <Prec P, bool CPLX, bool KC, int ROWS, bool SCALED> struct WaveOperand 
       v[I] = load16(rsrc, off[0], (uint32_t)kwave_k_of<CPLX>(I >> 3, I & 7) * line);
     }
   }
+  // zero for a lane's K-values before `from` (the partial K-step loaded as the last 32 K-values of the matrix)
+  __device__ inline void drop_before(const int from, const int lane) {
+    if constexpr (KC) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const bool in = k_of(0, lane, j) >= from; // (the same for every piece)
+#pragma unroll
+        for (int i = 0; i < PIECES; i++)
+#pragma unroll
+          for (int q = 0; q < NC; q++) {
+            f4u_t &x = v[i * NC + j * NC / 4];
+            x[(j * NC + q) % 4] = in ? x[(j * NC + q) % 4] : 0.0f;
+          }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < KPL; i++) {
+        const bool in = k_of(0, lane, i) >= from;
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[i][e] = in ? v[i][e] : 0.0f;
+      }
+    }
+  }
   // the partial K-step at the end (k_left < 32 K-values): a K-value past it is read from the step's first and replaced by zero
   __device__ inline void load_tail(const float *base, const uint32_t ld, const int rows, const int k_left, const int lane) {
     const __amdgpu_buffer_rsrc_t rsrc =
@@ -329,7 +352,21 @@ template <class Cfg> __device__ inline void kwaves_product(const GemmArgs &args)
     bp += b_kstep * W;
   };
   if (steps > 0) {
-    if (has_tail) {
+    if (W > 1 && has_tail && whole > 0) {
+      // The last 32 K-values without those of the step before: loads of 16 bytes, where load_tail reads a K-contiguous
+      // operand value by value.  (us, load_tail -> so: real 500^3 NN 5.57 -> 5.33, TN 5.34 -> 5.10, complex TN 8.64 ->
+      // 8.29.  Not with one wave to a tile: many small matrices are bound by the bytes they read, and the step before is
+      // not on the chip yet.  128 x 128 x 100 x 1000 NT 32 -> 38.)
+      const uint64_t back = 32 - tail;
+      const float *const ap0 = ap, *const bp0 = bp;
+      ap = a_tile + whole * a_kstep - back * (Cfg::A_KC ? 1 : lda) * NC;
+      bp = b_tile + whole * b_kstep - back * (Cfg::B_KC ? 1 : ldb) * NC;
+      static_for<0, PA + PB>(load_after);
+      oa.drop_before((int)back, lane);
+      ob.drop_before((int)back, lane);
+      ap = ap0;
+      bp = bp0;
+    } else if (has_tail) {
       oa.load_tail(a_tile + whole * a_kstep, (uint32_t)lda, rows_a, tail, lane);
       ob.load_tail(b_tile + whole * b_kstep, (uint32_t)ldb, rows_b, tail, lane);
     } else {
