@@ -65,7 +65,12 @@ inline double kwaves_time(const KWavesForm &f, const KWavesProblem &p, unsigned 
   const uint64_t steps = ((p.k + 31) / 32 + f.waves - 1) / f.waves;
   const uint64_t per_cu = (kwaves_tiles(f, p) + cus - 1) / cus, rounds = (per_cu + f.resident - 1) / f.resident;
   const double beside = (double)((per_cu < (uint64_t)f.resident ? per_cu : (uint64_t)f.resident) - 1);
-  return 2.2 + (double)rounds * (f.fill + (double)steps * f.step * (1.0 + f.beside * beside));
+  // Workgroups of one wave hardly run in rounds: as one ends the next begins.  Half way between whole rounds and none, on
+  // 350 drawn batches against whole ones: 11 take 0.55 - 0.96 of the time (416^3 x 35 bf16x2 TN 64 -> 35 us, 262^3 x 152
+  // FP16TCEC NT 88 -> 69, 128 x 36 x 102 x 870 bf16x3 NN 41 -> 30), 4 are slower by 3 - 5 %; with no rounds at all two of
+  // 150 by 10 - 13 % (256^3 x 77 FP16TCEC TT 18.5 -> 21.0).
+  const double part = (double)kwaves_tiles(f, p) / ((double)cus * f.resident);
+  return 2.2 + (f.waves == 1 && part > 1.0 ? 0.5 * (part + (double)rounds) : (double)rounds) * (f.fill + (double)steps * f.step * (1.0 + f.beside * beside));
 }
 
 // Whether a form can serve the product at all.
