@@ -416,8 +416,8 @@ PreSplitChoice choose_pre_split(const cuMpSGEMM_handle *h, bool a_kc, bool b_kc,
   const bool forced = h->ws_override != nullptr;
   // (depth 2: the whole rounds of a problem that was cut for this path)
   const bool never = tuning().packed == 0 && !forced, always = tuning().packed == 1 || forced || depth == 2;
-  // bf16x3 (explicit TF32TCEC mode): its in-loop three-way split costs 5.4
-  // vector instructions per MFMA, so the pre-pass pays for every layout
+  // bf16x3 (explicit TF32TCEC mode): its in-loop three-way split costs 5.5
+  // vector instructions per value, so the pre-pass pays for every layout
   ch.bf16 = (mode == CUMPSGEMM_TF32TCEC);
   ch.bm = CPLX ? kPackedCplxBM : (ch.bf16 ? kPackedBf16BM : kPackedBM);
   ch.bn = CPLX ? kPackedCplxBN : (ch.bf16 ? kPackedBf16BN : kPackedBN);
