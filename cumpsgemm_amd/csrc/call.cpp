@@ -6,7 +6,8 @@
 // addresses that `bind` is given (the library that ctypes has loaded).  An argument
 // of a type that is not the usual one -- anything but int sizes, float / complex
 // scalars, and ints, None or objects with data_ptr() as pointers -- makes a call
-// return None with nothing done: ctypes then converts it, or refuses it.
+// return None with nothing done: ctypes then converts it, or refuses it.  What an
+// object's data_ptr() raises is raised by the call.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <cstring>
@@ -30,7 +31,7 @@ constexpr Py_ssize_t kFunctions = sizeof(Functions) / sizeof(void *);
 PyObject *data_ptr_name;
 
 // The arguments of a call, taken one after the other; `ok` goes false at the first
-// one that is not of the usual type.
+// one that is not of the usual type, or whose data_ptr() raised (the exception is set).
 struct Args {
   PyObject *const *arg;
   bool ok = true;
@@ -55,7 +56,7 @@ struct Args {
     if (PyLong_Check(o)) return reinterpret_cast<T *>(integer(o));
     PyObject *const p = PyObject_CallMethodNoArgs(o, data_ptr_name);
     if (p == nullptr) {
-      PyErr_Clear();
+      if (PyErr_ExceptionMatches(PyExc_AttributeError)) PyErr_Clear(); // (no data_ptr)
       ok = false;
       return nullptr;
     }
@@ -79,7 +80,10 @@ struct Args {
 };
 
 template <class Call> PyObject *status(const Args &a, Call &&call) {
-  if (!a.ok) Py_RETURN_NONE;
+  if (!a.ok) {
+    if (PyErr_Occurred()) return nullptr;
+    Py_RETURN_NONE;
+  }
   hipblasStatus_t st;
   Py_BEGIN_ALLOW_THREADS
   st = call();

@@ -120,3 +120,24 @@ def test_other_types_are_what_ctypes_makes_of_them(monkeypatch, where, value):
     native = outcome()
     monkeypatch.setattr(_lib, "_native", None)
     assert native == outcome()
+
+
+@pytest.mark.parametrize("raised", [KeyboardInterrupt, MemoryError, ValueError])
+@pytest.mark.parametrize("where", [6, 8, 11])
+def test_what_a_pointer_raises_ends_the_call(calls, where, raised):
+    """An interrupt that arrives inside data_ptr() is not lost, and the object is not asked again."""
+    h, got = calls
+    asked = []
+
+    class Once:
+        def data_ptr(self):
+            asked.append(1)
+            if len(asked) == 1:
+                raise raised
+            return 16
+    args = [111, 111, 2, 2, 2, 1.0, 16, 2, 16, 2, 0.0, 16, 2, 1]
+    args[where] = Once()
+    got[0] = 0
+    with pytest.raises(raised):
+        h.gemm(*args)
+    assert len(asked) == 1 and got[0] == 0
