@@ -1,6 +1,7 @@
 """The native calls of the Python binding (csrc/call.cpp) against the ctypes ones: the same arguments arrive, and what
 is not of the usual types is converted or refused as ctypes does."""
 import ctypes
+import os
 import subprocess
 
 import numpy as np
@@ -141,3 +142,22 @@ def test_what_a_pointer_raises_ends_the_call(calls, where, raised):
     with pytest.raises(raised):
         h.gemm(*args)
     assert len(asked) == 1 and got[0] == 0
+
+
+CSRC = os.path.join(os.path.dirname(os.path.abspath(_lib.__file__)), "csrc")
+
+
+def _commands(**env):
+    """What `make -B` would run."""
+    return subprocess.run(["make", "-n", "-B", "-C", CSRC], check=True, capture_output=True, text=True,
+                          env=dict(os.environ, **env)).stdout
+
+
+def test_the_library_builds_without_pythons_headers(tmp_path):
+    """C and C++ programs do not need call.cpp; where it cannot be compiled nothing asks for it."""
+    fake = tmp_path / "python3"
+    fake.write_text(f"#!/bin/sh\necho {tmp_path}\n")
+    fake.chmod(0o755)
+    without = _commands(PATH=f"{tmp_path}:{os.environ['PATH']}")
+    assert "call.cpp" not in without and "libcumpsgemm.so" in without and "libcumpsgemm_rule.so" in without
+    assert "call.cpp" in _commands()
