@@ -1,6 +1,7 @@
 import ctypes
 import os
 import subprocess
+import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # CUMPSGEMM_LIBRARY: another build of the library (a diagnostic one, say) instead of the in-tree file
@@ -36,8 +37,9 @@ def rule_lib_path():
 
 
 def build(jobs=8):
-    """Compile libcumpsgemm.so and libcumpsgemm_rule.so for gfx950 in-tree."""
-    subprocess.check_call(["make", "-s", "-B", "-j", str(jobs), "-C", os.path.join(_HERE, "csrc")])
+    """Compile libcumpsgemm.so and libcumpsgemm_rule.so for gfx950 in-tree, and _call for this interpreter."""
+    subprocess.check_call(["make", "-s", "-B", "-j", str(jobs), "-C", os.path.join(_HERE, "csrc"),
+                           f"PYTHON={sys.executable}"])
 
 
 _lib = None

@@ -1,4 +1,4 @@
-// CPython entry to the GEMM calls of the library (cumpsgemm_amd/_call.so).
+// CPython entry to the GEMM calls of the library (cumpsgemm_amd/_call.<suffix>.so).
 //
 // A small product is bound by what one call costs on the host.  Through ctypes the
 // conversion of its 17 arguments takes 1.8 us of the 5.3 us of a 128^3 product in a

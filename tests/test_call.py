@@ -3,6 +3,8 @@ is not of the usual types is converted or refused as ctypes does."""
 import ctypes
 import os
 import subprocess
+import sys
+import sysconfig
 
 import numpy as np
 import pytest
@@ -147,9 +149,9 @@ def test_what_a_pointer_raises_ends_the_call(calls, where, raised):
 CSRC = os.path.join(os.path.dirname(os.path.abspath(_lib.__file__)), "csrc")
 
 
-def _commands(**env):
+def _commands(*variables, **env):
     """What `make -B` would run."""
-    return subprocess.run(["make", "-n", "-B", "-C", CSRC], check=True, capture_output=True, text=True,
+    return subprocess.run(["make", "-n", "-B", "-C", CSRC, *variables], check=True, capture_output=True, text=True,
                           env=dict(os.environ, **env)).stdout
 
 
@@ -161,3 +163,21 @@ def test_the_library_builds_without_pythons_headers(tmp_path):
     without = _commands(PATH=f"{tmp_path}:{os.environ['PATH']}")
     assert "call.cpp" not in without and "libcumpsgemm.so" in without and "libcumpsgemm_rule.so" in without
     assert "call.cpp" in _commands()
+
+
+def test_the_calls_are_built_for_one_interpreter(tmp_path, monkeypatch):
+    """The one that asks, under its own suffix: another version finds no module and goes through ctypes."""
+    suffix = sysconfig.get_config_var("EXT_SUFFIX")
+    assert suffix != ".so"
+    assert _lib.lib() is not None and _lib._native.__file__.endswith("_call" + suffix)
+    other = tmp_path / "python4"
+    other.write_text(f"#!{sys.executable}\nimport sys, sysconfig\nv = sysconfig.get_config_var\n"
+                     "sysconfig.get_config_var = lambda n: '.cpython-400.so' if n == 'EXT_SUFFIX' else v(n)\n"
+                     "exec(sys.argv[2])\n")
+    other.chmod(0o755)
+    assert f"/_call.cpython-400.so {CSRC}/call.cpp" in _commands(f"PYTHON={other}")
+    assert f"/_call{suffix} {CSRC}/call.cpp" in _commands(f"PYTHON={sys.executable}")
+    ran = []
+    monkeypatch.setattr(_lib.subprocess, "check_call", ran.append)
+    _lib.build()
+    assert f"PYTHON={sys.executable}" in ran[0]
