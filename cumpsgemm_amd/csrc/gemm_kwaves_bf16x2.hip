@@ -3,11 +3,13 @@
 namespace cumpsgemm_amd {
 #define ROW(A, B) \
   { kwaves_entry<Prec::BF16X2, false, A, B, 64, 64, 4, 2>(), kwaves_entry<Prec::BF16X2, false, A, B, 32, 32, 8, 4>(), \
-    kwaves_entry<Prec::BF16X2, false, A, B, 32, 32, 4, 4>(), kwaves_entry<Prec::BF16X2, false, A, B, 32, 32, 1, 4>() }
+    kwaves_entry<Prec::BF16X2, false, A, B, 32, 32, 4, 4>(), kwaves_entry<Prec::BF16X2, false, A, B, 32, 32, 1, 4>(), \
+    KWavesEntry{} }
 CUMPSGEMM_KWAVES_TABLE(bf16x2_s, ROW)
 #undef ROW
 #define ROW(A, B) \
-  { kwaves_entry<Prec::BF16X2, true, A, B, 32, 32, 4, 2>(), kwaves_entry<Prec::BF16X2, true, A, B, 32, 32, 8, 2>(), KWavesEntry{}, KWavesEntry{} }
+  { kwaves_entry<Prec::BF16X2, true, A, B, 32, 32, 4, 2>(), kwaves_entry<Prec::BF16X2, true, A, B, 32, 32, 8, 2>(), KWavesEntry{}, KWavesEntry{}, \
+    kwaves_entry<Prec::BF16X2, true, A, B, 64, 32, 4, 1>() }
 CUMPSGEMM_KWAVES_TABLE(bf16x2_c, ROW)
 #undef ROW
 } // namespace cumpsgemm_amd

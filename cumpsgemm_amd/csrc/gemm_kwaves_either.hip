@@ -18,11 +18,11 @@ template <bool CPLX, bool AKC, bool BKC, int BM, int BN, int W, int OCC_A, int O
 } // namespace
 #define ROW(A, B) \
   { either<false, A, B, 64, 64, 4, 1, 2>(), either<false, A, B, 32, 32, 8, 3, 4>(), either<false, A, B, 32, 32, 4, 3, 4>(), \
-    either<false, A, B, 32, 32, 1, 3, 4>() }
+    either<false, A, B, 32, 32, 1, 3, 4>(), nullptr }
 kwaves_either_t g_kwaves_either_s[4][kKWavesForms] = {ROW(false, false), ROW(true, false), ROW(false, true), ROW(true, true)};
 #undef ROW
 #define ROW(A, B) \
-  { either<true, A, B, 32, 32, 4, 1, 2>(), nullptr, nullptr, nullptr }
+  { either<true, A, B, 32, 32, 4, 1, 2>(), nullptr, nullptr, nullptr, nullptr }
 kwaves_either_t g_kwaves_either_c[4][kKWavesForms] = {ROW(false, false), ROW(true, false), ROW(false, true), ROW(true, true)};
 #undef ROW
 } // namespace cumpsgemm_amd

@@ -6,7 +6,8 @@
 
 namespace cumpsgemm_amd {
 
-constexpr int kKWavesForms = 4; // tiles per precision, real or complex
+constexpr int kKWavesForms = 5; // tiles per precision, real or complex
+constexpr int kKWavesAlone = 4; // the form for one workgroup on a CU
 constexpr int kKWavesFourWaves = 2; // real: the tile of the eight-wave form with four
 constexpr unsigned kKWavesModuleId = 6; // what used_kernel_module_id reports (0 - 4 are the tile classes, 5 the narrow kernel)
 
@@ -28,11 +29,15 @@ struct KWavesForm {
 // 0.69 (0.65), bf16x3 0.72 (0.69), bf16x2 0.72 (0.70); complex 0.60 (0.58), 0.61 (0.58),
 // 0.62 (0.62), 0.68 (0.66); 2 % are slower by 5 %, complex none.  Before there were two
 // waves to a SIMD: 0.73, 0.70, 0.72, 0.73; 0.66, 0.63, 0.62, 0.74.
+// Forms of one wave to a SIMD, which has the registers for two sets of fragments or for a 64 x 32 complex tile, are the
+// faster ones where a CU has no second workgroup anyway.  2100 real and 1500 complex products, geometric mean: real
+// FP16TCEC against two sets of registers to a SIMD up to K = 256 1.04, 512 0.99, 1024 0.97, 2048 0.96, 4096 0.94 (FP16TC and
+// bf16x2 1.00, 0.98: left out); complex against the faster of its other two, where those are two to a CU: K <= 256
+// 1.2 - 1.3, 1024 FP16TC 0.93, others 1.06 - 1.09, beyond 2048 0.83 and 0.94 - 0.95.
 // (Tried beside these and left out: 64 x 64 with eight waves at two to a SIMD, up to
 // 10 % faster than four where K >= 2048 and 256 tiles or fewer, 0 - 4 % else, no better
 // over the 640; 64 x 32 and 32 x 64 with four and eight waves, 64 x 64 with one and two,
-// within 1 %; 128 x 64 spills.  Complex with one or two waves: batches are faster tiled;
-// 64 x 32: never ahead of these by 5 %.)
+// within 1 %; 128 x 64 spills.  Complex with one or two waves: batches are faster tiled.)
 struct KWavesModel {
   KWavesForm form[kKWavesForms];
   double tiled0, tiled_per_step, tiled_split;
@@ -40,15 +45,15 @@ struct KWavesModel {
 // `prec`: 0 FP16TCEC, 1 FP16TC, 2 bf16x3, 3 bf16x2
 inline const KWavesModel &kwaves_model(int prec, bool cplx) {
   static const KWavesModel real[4] = {
-      {{{64, 64, 4, 2, 3.11, 1.10, 0.79}, {32, 32, 8, 2, 1.13, 0.88, 0.71}, {32, 32, 4, 4, 1.08, 0.50, 0.74}, {32, 32, 1, 16, 2.4, 0.37, 0.22}}, 4.1, 1.63, -2.1},
+      {{{64, 64, 4, 2, 3.11, 1.10, 0.79}, {32, 32, 8, 2, 1.13, 0.88, 0.71}, {32, 32, 4, 4, 1.08, 0.50, 0.74}, {32, 32, 1, 16, 2.4, 0.37, 0.22}, {64, 64, 4, 1, 3.6, 0.93, 0.0}}, 4.1, 1.63, -2.1},
       {{{64, 64, 4, 2, 2.03, 0.72, 1.41}, {32, 32, 8, 2, 0.98, 0.87, 0.55}, {32, 32, 4, 4, 1.00, 0.47, 0.67}, {32, 32, 1, 16, 2.4, 0.23, 0.37}}, 4.8, 1.27, 0.9},
       {{{64, 64, 4, 1, 3.6, 1.65, 0.0}, {32, 32, 8, 1, 1.62, 1.17, 0.0}, {32, 32, 4, 3, 1.29, 0.76, 0.55}, {32, 32, 1, 12, 2.2, 0.68, 0.17}}, 2.5, 2.29, -2.4},
       {{{64, 64, 4, 2, 2.78, 1.04, 0.90}, {32, 32, 8, 2, 1.12, 0.87, 0.78}, {32, 32, 4, 4, 1.09, 0.50, 0.73}, {32, 32, 1, 16, 2.5, 0.39, 0.21}}, 4.0, 1.61, -1.6}};
   static const KWavesModel complex[4] = {
-      {{{32, 32, 4, 2, 1.50, 1.02, 0.94}, {32, 32, 8, 1, 1.15, 1.77, 0.0}, {}, {}}, 2.8, 2.05, -5.4},
-      {{{32, 32, 4, 2, 1.09, 0.51, 1.72}, {32, 32, 8, 1, 0.74, 1.28, 0.0}, {}, {}}, 3.6, 1.50, -3.4},
+      {{{32, 32, 4, 2, 1.50, 1.02, 0.94}, {32, 32, 8, 1, 1.15, 1.77, 0.0}, {}, {}, {64, 32, 4, 1, 3.5, 1.67, 0.0}}, 2.8, 2.05, -5.4},
+      {{{32, 32, 4, 2, 1.09, 0.51, 1.72}, {32, 32, 8, 1, 0.74, 1.28, 0.0}, {}, {}, {64, 32, 4, 1, 2.2, 1.12, 0.0}}, 3.6, 1.50, -3.4},
       {{{32, 32, 4, 1, 2.3, 1.71, 0.0}, {}, {}, {}}, 0.9, 3.83, -14.3},
-      {{{32, 32, 4, 2, 1.55, 0.97, 1.06}, {32, 32, 8, 1, 0.99, 1.85, 0.0}, {}, {}}, 3.1, 2.09, -6.1}};
+      {{{32, 32, 4, 2, 1.55, 0.97, 1.06}, {32, 32, 8, 1, 0.99, 1.85, 0.0}, {}, {}, {64, 32, 4, 1, 3.7, 1.72, 0.0}}, 3.1, 2.09, -6.1}};
   return (cplx ? complex : real)[prec];
 }
 
@@ -115,6 +120,7 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
     // reads, which the fit misses (1536^3 TT 41 us tiled, 52 here; 1664^3 NT 44, 53).
     const uint64_t per_cu = (kwaves_tiles(f, p) + cus - 1) / cus;
     if (per_cu > 2ull * f.resident && p.k > 512) continue;
+    if (i == kKWavesAlone && (per_cu > 1 || (!p.cplx && p.k <= 512))) continue;
     // (complex, more than one round of tiles: the fit is up to 10 % short.  FP16TC 1000^3 NN 23.2 us tiled, 26.1 here.)
     const bool rounds = p.cplx && per_cu > (uint64_t)f.resident;
     const double t = kwaves_time(f, p, cus) * (rounds ? 1.1 : 1.0);
@@ -150,6 +156,7 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
 // together, 27.3).
 inline int choose_kwaves_either_form(const KWavesProblem &p, unsigned cus, int form_bf16, int form_fp16) {
   constexpr double LAUNCH = 1.7;
+  if (!p.cplx && form_fp16 == kKWavesAlone) form_fp16 = 0; // (the same tile and waves; 1 - 6 % of the product for a launch)
   if (form_bf16 < 0 || form_fp16 < 0) return -1;
   const KWavesModel &ma = kwaves_model(2, p.cplx), &mb = kwaves_model(0, p.cplx);
   const double apart_a = kwaves_time(ma.form[form_bf16], p, cus), apart_b = kwaves_time(mb.form[form_fp16], p, cus);

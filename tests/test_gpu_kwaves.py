@@ -215,3 +215,24 @@ def test_more_tiles_than_cus_are_exact_on_integers(O, handle, dev, monkeypatch, 
     assert (st, mid) == (0, KWAVES)
     # |x| <= 30: every partial sum is an integer below 2^24
     assert np.array_equal(c, oracle_gemm(O, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, 1.0, c0.copy(), m))
+
+
+@pytest.mark.parametrize("mode", [FP16TCEC, FP16TC, TF32TC])
+@pytest.mark.parametrize("cplx,opa,opb", LAYOUTS)
+def test_forms_for_one_workgroup_on_a_cu(O, handle, dev, monkeypatch, mode, cplx, opa, opb):
+    """Form 5: real FP16TCEC 64 x 64 with two sets of fragments, complex 64 x 32."""
+    monkeypatch.setenv("CUMPSGEMM_KWAVES", "5")
+    rng = np.random.default_rng(10)
+    for m, n, k in _sizes(opa, opb):
+        a, lda = _padded_ints(rng, opa, m, k, 3, cplx)
+        b, ldb = _padded_ints(rng, opb, k, n, 1, cplx)
+        c0 = rng.integers(-9, 10, m * n).astype(np.complex64 if cplx else np.float32)
+        c, st, mid = run_gemm(handle, dev, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, 1.0, c0.copy(), m, cplx,
+                              want_module_id=True)
+        assert st == 0 and (mid == KWAVES) == (cplx or mode == FP16TCEC)
+        # (as above: every partial sum is an integer below 2^24)
+        assert np.array_equal(c, oracle_gemm(O, mode, opa, opb, m, n, k, 1.0, a, lda, b, ldb, 1.0, c0.copy(), m)), (m, n, k)
+    if mode == FP16TCEC:
+        test_small_products_with_correction_terms(O, handle, dev, monkeypatch, mode, cplx, opa, opb, 5)
+        for args in ((SCALING, True, FP16TCEC), (AUTO, True, FP16TCEC)):
+            test_small_products_scaled_and_gated_with_correction_terms(handle, dev, monkeypatch, *args, cplx, opa, opb, 5)

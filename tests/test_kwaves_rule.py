@@ -126,3 +126,20 @@ def test_one_launch_for_both_candidates_of_auto(rule, cplx, op):
     assert rule.either(cplx, op, 512, 512, 512, 1, 0, 0) == 0
     if cplx:
         assert rule.either(cplx, op, 640, 640, 640, 1, 0, 0) == -1
+
+
+# (`steps`, `split`: the tiled plan's cost, whether it splits K)
+@pytest.mark.parametrize("prec,cplx,op,m,n,k,steps,split,tile", [
+    (0, False, "NN", 3968, 173, 2378, 18.86, True, (64, 64, 4)), (0, False, "TT", 1485, 530, 2754, 21.33, True, (64, 64, 4)),
+    (0, False, "NT", 310, 1884, 1600, 14.63, True, (64, 64, 4)), (1, True, "NT", 431, 1024, 3798, 30.48, True, (64, 32, 4)),
+    (1, True, "NN", 384, 1118, 2033, 23.52, True, (64, 32, 4))])
+def test_one_workgroup_on_a_cu_has_the_registers_of_a_simd_to_itself(rule, prec, cplx, op, m, n, k, steps, split, tile):
+    """Measured 1.05 - 1.35 times as long on the forms of two waves to a SIMD, or on the kernel taken instead."""
+    p = rule(prec, cplx, op, m, n, k, steps=steps, split=split)
+    assert p and p[1:] == tile and p[0] == 4
+    # never where a CU has a second workgroup, nor for a short K
+    for mm, nn in itertools.product((m, 2 * m, 3 * m), (n, 3 * n)):
+        q = rule(prec, cplx, op, mm, nn, k, steps=1e3, split=split)
+        assert q is None or q[0] != 4 or -(-mm // tile[0]) * -(-nn // tile[1]) <= CUS
+    q = rule(prec, cplx, op, m, n, 200, steps=1e3, split=split)
+    assert q is None or q[0] != 4
