@@ -129,6 +129,14 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
       best_time = t;
     }
   }
+  if (asked < 0 && p.cplx && best >= 0 && model.form[best].waves == 8 &&
+      kwaves_tiles(model.form[best], p) > (uint64_t)cus * model.form[best].resident) {
+    // Complex tiles with eight waves as well: beyond one round the fit makes them too cheap.  670 products of more tiles
+    // than CUs: 1.16 - 1.3 times the faster of the other two forms.  Of 23 sent to them four waves take 0.74 - 0.89 of
+    // that, and 0.82 of the tiled time, two of them 1.05 and 1.12 (us, eight / four waves / tiled: FP16TC 1088 x 512 x 480 TN
+    // 13.5, 10.8, 11.3; 768 x 768 x 203 NN 11.0, 8.5, 11.0; bf16x2 960 x 576 x 448 NN 18.3, 16.1, 14.4).
+    best = 0;
+  }
   if (asked < 0 && !p.cplx && best >= 0 && model.form[best].waves == 8) {
     // Eight waves on a tile pay while all workgroups are on the chip at once: the fit makes their second round too cheap.
     // 36 of 10000 drawn products were sent to one.  The 32 up to K = 512 take 0.72 - 1.01 of the time with four waves on

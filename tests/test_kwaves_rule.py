@@ -143,3 +143,13 @@ def test_one_workgroup_on_a_cu_has_the_registers_of_a_simd_to_itself(rule, prec,
         assert q is None or q[0] != 4 or -(-mm // tile[0]) * -(-nn // tile[1]) <= CUS
     q = rule(prec, cplx, op, m, n, 200, steps=1e3, split=split)
     assert q is None or q[0] != 4
+
+
+@pytest.mark.parametrize("prec,op,m,n,k,steps", [(3, "TT", 528, 1440, 447, 7.97), (3, "NN", 960, 576, 448, 7.97),
+                                                (1, "NN", 768, 768, 203, 4.76), (0, "TT", 208, 2496, 512, 8.85)])
+def test_eight_waves_on_a_complex_tile_in_one_round_only(rule, prec, op, m, n, k, steps):
+    """More tiles than CUs: measured 1.1 - 1.35 times as long as with four waves."""
+    assert rule(prec, True, op, m, n, k, steps=steps) == (0, 32, 32, 4)
+    for prec, mm, nn, kk in itertools.product((0, 1, 3), (256, 512, 1024), (300, 512, 2000), (64, 400, 3000)):
+        p = rule(prec, True, op, mm, nn, kk, steps=1e3)
+        assert p is None or p[3] != 8 or -(-mm // 32) * -(-nn // 32) <= CUS
