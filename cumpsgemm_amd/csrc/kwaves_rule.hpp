@@ -24,7 +24,9 @@ struct KWavesForm {
 // All of it fitted on 188 products (84 real, m and n 64 - 4096, K 64 - 8192, 60 real
 // batches of up to 1024 matrices of 32 - 640, 44 complex; four layouts, padded, with
 // and without C), each timed with every form and tiled, in every precision; the forms
-// with two waves to a SIMD on 640 others.  On 640 more, time over the tiled time,
+// with two waves to a SIMD on 640 others, real ones again on 2800 (their `fill` was 0.5 - 1.1 us
+// too low: 256 - 512 tiles of a short K went to 64 x 64 that are faster on 32 x 32 or tiled,
+// bf16x2 512 x 2254 x 128 NN 6.1 us, 64 x 64 7.5).  On 640 more, before that, time over the tiled time,
 // geometric mean (the fastest side by hindsight): real FP16TCEC 0.72 (0.70), FP16TC
 // 0.69 (0.65), bf16x3 0.72 (0.69), bf16x2 0.72 (0.70); complex 0.60 (0.58), 0.61 (0.58),
 // 0.62 (0.62), 0.68 (0.66); 2 % are slower by 5 %, complex none.  Before there were two
@@ -45,10 +47,10 @@ struct KWavesModel {
 // `prec`: 0 FP16TCEC, 1 FP16TC, 2 bf16x3, 3 bf16x2
 inline const KWavesModel &kwaves_model(int prec, bool cplx) {
   static const KWavesModel real[4] = {
-      {{{64, 64, 4, 2, 3.11, 1.10, 0.79}, {32, 32, 8, 2, 1.13, 0.88, 0.71}, {32, 32, 4, 4, 1.08, 0.50, 0.74}, {32, 32, 1, 16, 2.4, 0.37, 0.22}, {64, 64, 4, 1, 3.6, 0.93, 0.0}}, 4.1, 1.63, -2.1},
-      {{{64, 64, 4, 2, 2.03, 0.72, 1.41}, {32, 32, 8, 2, 0.98, 0.87, 0.55}, {32, 32, 4, 4, 1.00, 0.47, 0.67}, {32, 32, 1, 16, 2.4, 0.23, 0.37}}, 4.8, 1.27, 0.9},
+      {{{64, 64, 4, 2, 3.60, 1.07, 0.72}, {32, 32, 8, 2, 1.13, 0.88, 0.71}, {32, 32, 4, 4, 1.08, 0.50, 0.74}, {32, 32, 1, 16, 2.4, 0.37, 0.22}, {64, 64, 4, 1, 3.6, 0.93, 0.0}}, 4.1, 1.63, -2.1},
+      {{{64, 64, 4, 2, 3.10, 0.67, 1.25}, {32, 32, 8, 2, 0.98, 0.87, 0.55}, {32, 32, 4, 4, 1.00, 0.47, 0.67}, {32, 32, 1, 16, 2.4, 0.23, 0.37}}, 4.8, 1.27, 0.9},
       {{{64, 64, 4, 1, 3.6, 1.65, 0.0}, {32, 32, 8, 1, 1.62, 1.17, 0.0}, {32, 32, 4, 3, 1.29, 0.76, 0.55}, {32, 32, 1, 12, 2.2, 0.68, 0.17}}, 2.5, 2.29, -2.4},
-      {{{64, 64, 4, 2, 2.78, 1.04, 0.90}, {32, 32, 8, 2, 1.12, 0.87, 0.78}, {32, 32, 4, 4, 1.09, 0.50, 0.73}, {32, 32, 1, 16, 2.5, 0.39, 0.21}}, 4.0, 1.61, -1.6}};
+      {{{64, 64, 4, 2, 3.75, 0.94, 0.93}, {32, 32, 8, 2, 1.12, 0.87, 0.78}, {32, 32, 4, 4, 1.09, 0.50, 0.73}, {32, 32, 1, 16, 2.5, 0.39, 0.21}}, 4.0, 1.61, -1.6}};
   static const KWavesModel complex[4] = {
       {{{32, 32, 4, 2, 1.50, 1.02, 0.94}, {32, 32, 8, 1, 1.15, 1.77, 0.0}, {}, {}, {64, 32, 4, 1, 3.5, 1.67, 0.0}}, 2.8, 2.05, -5.4},
       {{{32, 32, 4, 2, 1.09, 0.51, 1.72}, {32, 32, 8, 1, 0.74, 1.28, 0.0}, {}, {}, {64, 32, 4, 1, 2.2, 1.12, 0.0}}, 3.6, 1.50, -3.4},

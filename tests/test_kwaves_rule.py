@@ -153,3 +153,11 @@ def test_eight_waves_on_a_complex_tile_in_one_round_only(rule, prec, op, m, n, k
     for prec, mm, nn, kk in itertools.product((0, 1, 3), (256, 512, 1024), (300, 512, 2000), (64, 400, 3000)):
         p = rule(prec, True, op, mm, nn, kk, steps=1e3)
         assert p is None or p[3] != 8 or -(-mm // 32) * -(-nn // 32) <= CUS
+
+
+@pytest.mark.parametrize("prec,op,m,n,k,batch,pad,steps", [
+    (3, "NN", 512, 2254, 128, 1, 0, 3.27), (3, "TN", 2891, 416, 100, 1, 4, 3.27), (1, "TN", 4576, 288, 160, 1, 0, 3.68),
+    (1, "TT", 96, 96, 96, 117, 4, 2.86), (0, "TT", 608, 2560, 192, 1, 0, 4.09), (0, "NN", 224, 5088, 104, 1, 0, 3.27)])
+def test_a_short_k_of_257_to_512_large_tiles_takes_small_ones(rule, prec, op, m, n, k, batch, pad, steps):
+    """Measured 1.2 - 1.3 times as long on 64 x 64 tiles as on 32 x 32."""
+    assert rule(prec, False, op, m, n, k, batch, pad, steps=steps)[1:3] == (32, 32)
