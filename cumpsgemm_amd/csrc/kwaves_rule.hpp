@@ -118,8 +118,9 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
       if (asked == i + 1) return i;
       continue;
     }
-    // More than two tiles per workgroup that a CU holds, and more than a short K: bound by what a tile this small
-    // reads, which the fit misses (1536^3 TT 41 us tiled, 52 here; 1664^3 NT 44, 53).
+    // More than a short K, and more than two rounds of workgroups: bound by what a tile this small reads, which the fit
+    // misses.  With more than 1024 tiles of 64 x 64, 70 products take 1.05 - 1.13 of the tiled time (5256 x 805 x 545 FP16TCEC
+    // NT 35.7 us, tiled 34.1; 2216 x 1984 x 3200 TN 126, 113).
     const uint64_t per_cu = (kwaves_tiles(f, p) + cus - 1) / cus;
     if (per_cu > 2ull * f.resident && p.k > 512) continue;
     if (i == kKWavesAlone && (per_cu > 1 || (!p.cplx && p.k <= 512))) continue;
@@ -130,6 +131,14 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
       best = i;
       best_time = t;
     }
+  }
+  if (asked < 0 && !p.cplx && best == 0 && model.form[0].resident == 2 && p.k > 512 && (p.a_kc || p.b_kc) &&
+      (kwaves_tiles(model.form[0], p) + cus - 1) / cus == 3) {
+    // Three tiles of 64 x 64 on a CU that holds two: a round for the third, and where the estimates still send them here
+    // that of the tiled kernels is too dear.  16 drawn products, 513 - 600 tiles: 1.12 of the tiled time, 0.90 - 1.41
+    // (3392 x 591 x 2932 FP16TCEC TT 106 us, tiled 76).  Not with two row-contiguous operands (7: 0.91), nor with four
+    // tiles (47: 0.84).
+    best = -1;
   }
   if (asked < 0 && p.cplx && best >= 0 && model.form[best].waves == 8 &&
       kwaves_tiles(model.form[best], p) > (uint64_t)cus * model.form[best].resident) {

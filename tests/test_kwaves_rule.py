@@ -161,3 +161,15 @@ def test_eight_waves_on_a_complex_tile_in_one_round_only(rule, prec, op, m, n, k
 def test_a_short_k_of_257_to_512_large_tiles_takes_small_ones(rule, prec, op, m, n, k, batch, pad, steps):
     """Measured 1.2 - 1.3 times as long on 64 x 64 tiles as on 32 x 32."""
     assert rule(prec, False, op, m, n, k, batch, pad, steps=steps)[1:3] == (32, 32)
+
+
+@pytest.mark.parametrize("prec", [0, 1, 3])
+def test_two_rounds_of_large_tiles_at_most_and_no_third_tile_on_a_cu(rule, prec):
+    """64 x 64 tiles, K beyond 512, two workgroups to a CU; `steps`: the tiled kernels are estimated at 1.7 times as long."""
+    for op in ("NN", "TN", "NT", "TT"):
+        for tiles_m, tiles_n, taken in ((16, 32, True), (19, 27, op == "NT"), (24, 32, op == "NT"), (25, 31, True), (32, 32, True),
+                                        (25, 41, False)):
+            m, n, rounds = 64 * tiles_m, 64 * tiles_n, 1 if tiles_m * tiles_n <= 2 * CUS else 2
+            p = rule(prec, False, op, m, n, 2000, steps={0: 42, 1: 45, 3: 42}[prec] * rounds)
+            assert (p and p[:3]) == ((0, 64, 64) if taken else None), (op, tiles_m, tiles_n)
+        assert rule(prec, False, op, 64 * 19, 64 * 27, 500, steps=40) is not None
