@@ -634,13 +634,14 @@ struct tile_loader {
   //   KC:  16-byte global loads at base + constant per-thread offset.
   // (16-byte *buffer* loads are avoided on purpose: this toolchain narrows them
   // incorrectly when the loaded vector is taken apart element-wise.)
-  template <bool BESIDE_TAIL>
+  // (units U0 .. U1 - 1)
+  template <bool BESIDE_TAIL, int U0 = 0, int U1 = U>
   __device__ static inline void load_fast(Regs &reg, const float *__restrict__ base, uint64_t ld,
                                           const uint32_t (&boff)[U]) {
     if (!active(threadIdx.x)) return;
     if constexpr (KC) {
 #pragma unroll
-      for (int u = 0; u < U; u++) {
+      for (int u = U0; u < U1; u++) {
         // rows of a K-contiguous operand are 16-byte aligned only if ld is a
         // multiple of 4: the vector type promises 4-byte alignment and leaves
         // the choice of instruction to the compiler
@@ -672,7 +673,7 @@ struct tile_loader {
       uint32_t line = (uint32_t)ld * (uint32_t)(ES * 4);
       if constexpr (BESIDE_TAIL) line = __builtin_amdgcn_readfirstlane(line);
 #pragma unroll
-      for (int u = 0; u < U; u++) {
+      for (int u = U0; u < U1; u++) {
 #pragma unroll
         for (int j = 0; j < KV; j++) {
           if constexpr (!CPLX) {
@@ -901,14 +902,15 @@ struct tile_loader {
   // split and write to LDS: planes laid out [comp][plane][row][chunk]
   // SCALED: the values are multiplied by s (s2048 = s * 2^11) on the way
   // BY_PAIRS: split by `split_pair`
-  template <Prec P, bool SCALED = false, bool BY_PAIRS = false>
+  // (units U0 .. U1 - 1)
+  template <Prec P, bool SCALED = false, bool BY_PAIRS = false, int U0 = 0, int U1 = U>
   __device__ static inline void store(Regs &reg, char *lds_op, int tid, float s = 1.0f,
                                       float s2048 = 2048.0f) {
     constexpr int NP = prec_traits<P>::NP;
     constexpr int PLANE = ROWS * 64;
     if (!active(tid)) return;
 #pragma unroll
-    for (int u = 0; u < U; u++) {
+    for (int u = U0; u < U1; u++) {
       int row, chunk;
       unit_coords(u, tid, row, chunk);
       f8_t part[2];
@@ -957,6 +959,16 @@ struct tile_loader {
           *reinterpret_cast<u4_t *>(lds_op + (c * NP + p) * PLANE + lds_offset(row, chunk)) = out[p];
         }
       }
+    }
+  }
+  // store and load_fast, unit by unit
+  template <Prec P, bool SCALED, bool BESIDE_TAIL, int u = 0>
+  __device__ static inline void store_and_reload(Regs &reg, char *lds_op, int tid, float s, float s2048,
+                                                 const float *base, uint64_t ld, const uint32_t (&boff)[U]) {
+    if constexpr (u < U) {
+      store<P, SCALED, false, u, u + 1>(reg, lds_op, tid, s, s2048);
+      load_fast<BESIDE_TAIL, u, u + 1>(reg, base, ld, boff);
+      store_and_reload<P, SCALED, BESIDE_TAIL, u + 1>(reg, lds_op, tid, s, s2048, base, ld, boff);
     }
   }
 };
@@ -1855,11 +1867,26 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void gemm_tcec_kernel(c
       block_sync_lds();
       frag_load(f0, 0, 0);
       int b0 = 0, b1 = 1, b2 = 2; // buffers of tiles t, t+1, t+2
+      // bf16x2, two K-contiguous operands: each unit's registers are asked for again as soon as it is split.  Split pair by
+      // pair and reloaded together, the loads end up behind the last MFMA but six and the next step waits for them where
+      // rows start anywhere in a cache line.  us, split whole / by pairs / so: 2236^3 93.5 / 99.6 / 89.3, 768 x 5760 x 2991
+      // 113 / 120 / 108, 2208^3 89.5 / 87.4 / 81.5, 1600^3 42.6 / 39.7 / 36.5; complex 1210^3 52.3 / 55.7 / 50.5, 1501^2 x 777
+      // 72.1 / 76.3 / 70.9, 500^3 x 32 119 / 126 / 118.
+      constexpr bool RELOAD_BY_UNIT = P == Prec::BF16X2 && Cfg::A_KC && Cfg::B_KC && !Cfg::PACKED;
       for (int t = 0; t < nk; t++) {
         frag_load(f1, b0, 1);
         frag_mma(f0, f1);
-        lstore(b2);
-        gload(clamp(t + 3), fast_tag);
+        if constexpr (decltype(fast_tag)::value && RELOAD_BY_UNIT) {
+          char *const sa = lds + b2 * Cfg::STAGE_BYTES;
+          const uint64_t kt = (uint64_t)clamp(t + 3);
+          LA::template store_and_reload<P, Cfg::SCALED, !Cfg::PERSIST>(ra, sa, tid, coef_a, coef_a2048, a_tile + kt * a_kstep,
+                                                                      args.lda, offa);
+          LB::template store_and_reload<P, Cfg::SCALED, !Cfg::PERSIST>(rb, sa + Cfg::A_STAGE_BYTES, tid, coef_b, coef_b2048,
+                                                                      b_tile + kt * b_kstep, args.ldb, offb);
+        } else {
+          lstore(b2);
+          gload(clamp(t + 3), fast_tag);
+        }
         frag_load(f0, b1, 0);
         if constexpr (decltype(fast_tag)::value) {
           // 24 (real) MFMAs per step: after each one up to 4 vector ALU

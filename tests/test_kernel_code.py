@@ -71,3 +71,27 @@ def test_scaled_large_kernel_of_k_contiguous_operands_keeps_its_addresses_in_reg
     # GemmCfg<FP16TCEC, real, K-contiguous, K-contiguous, 256, 128, 64, 64, 2, DEEP, one tile, SCALED, in-loop>
     (code,) = [c for n, c in kernels.items() if "PrecE0ELb0ELb1ELb1ELi256ELi128ELi64ELi64ELi2ELb1ELb0ELb1ELb0E" in n]
     assert scratch_accesses_of_k_loops(code) == 0
+
+
+def first_loads_of_k_loops(code):
+    """Share of a loop's MFMAs that stand before its first global load, for every loop that multiplies and loads."""
+    out = []
+    for i, (text, at, target) in enumerate(code):
+        if target is not None and target <= at:
+            body = [t for t, a, _ in code[:i + 1] if a >= target]
+            mfma = [j for j, t in enumerate(body) if t.startswith("v_mfma")]
+            loads = [j for j, t in enumerate(body) if t.startswith(("global_load", "buffer_load"))]
+            if mfma and loads:
+                out.append(sum(j < loads[0] for j in mfma) / len(mfma))
+    return out
+
+
+@pytest.mark.parametrize("tile", ["Lb0ELb1ELb1ELi256ELi128ELi64ELi64E", "Lb0ELb1ELb1ELi128ELi128ELi64ELi32E",
+                                  "Lb1ELb1ELb1ELi128ELi64ELi32ELi32E"])
+def test_loads_of_two_k_contiguous_bf16x2_operands_are_not_left_behind_the_split(kernels, tile):
+    """The one-tile kernels ask for a step's operands while they split the one before it."""
+    # GemmCfg<bf16x2, real / complex, K-contiguous, K-contiguous, tile, 2, DEEP, one tile, not scaled, in-loop>
+    found = [c for n, c in kernels.items() if "PrecE3E" + tile in n and "Li2ELb1ELb0ELb0ELb0E" in n]
+    assert len(found) == 1
+    first = first_loads_of_k_loops(found[0])
+    assert first and min(first) <= 0.6, first
