@@ -1,5 +1,8 @@
 """Shared helpers of the GPU parity tests: build operands in column-major flat
 buffers, run the library through its C ABI, run the oracle on the same data."""
+import ctypes
+import os
+
 import numpy as np
 
 N, T, C = 111, 112, 113
@@ -51,3 +54,38 @@ def assert_same_up_to_summation_order(x, y, k):
     bar = 2.0 ** -24 * np.sqrt(k)
     assert np.linalg.norm(d) <= 2.0 * bar * np.linalg.norm(yv), (np.linalg.norm(d) / np.linalg.norm(yv), bar)
     assert d.max() <= 16.0 * bar * np.abs(yv).max(), (d.max() / np.abs(yv).max(), bar)
+
+
+class _KernelNode(ctypes.Structure):  # hipKernelNodeParams
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
+                ("grid", ctypes.c_uint * 3), ("args", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+
+def launched_kernels(torch, handle, call):
+    """(name, workgroups) of the kernels that `call` launches on the handle's stream, in no particular order: the nodes of
+    a graph that it is captured into, which is not run."""
+    hip = ctypes.CDLL(os.path.join(torch.__path__[0], "lib", "libamdhip64.so"))
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    p = ctypes.c_void_p
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    handle.set_stream(side)
+    graph, count = p(), ctypes.c_size_t()
+    try:
+        assert hip.hipStreamBeginCapture(p(side.cuda_stream), 2) == 0  # relaxed
+        try:
+            call()
+        finally:
+            assert hip.hipStreamEndCapture(p(side.cuda_stream), ctypes.byref(graph)) == 0
+    finally:
+        handle.set_stream(torch.cuda.current_stream())
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0
+    nodes = (p * count.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(count)) == 0
+    out = []
+    for node in nodes:
+        params = _KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(p(node), ctypes.byref(params)) == 0
+        out.append((hip.hipKernelNameRefByPtr(p(params.func), p(side.cuda_stream)).decode(), tuple(params.grid)))
+    assert hip.hipGraphDestroy(graph) == 0
+    return out

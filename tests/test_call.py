@@ -125,6 +125,93 @@ def test_other_types_are_what_ctypes_makes_of_them(monkeypatch, where, value):
     assert native == outcome()
 
 
+SEEN = """
+#include <stdint.h>
+#include <string.h>
+extern "C" {
+uint64_t seen[20];
+static uint64_t bits(const float *p) { uint32_t b; memcpy(&b, p, 4); return b; }
+#define ARGS void *h, int oa, int ob, uint64_t m, uint64_t n, uint64_t k, const float *al, void *a, uint64_t lda, void *b, \
+  uint64_t ldb, const float *be, void *c, uint64_t ldc, int mode
+#define PASS h, oa, ob, m, n, k, al, a, lda, b, ldb, be, c, ldc, mode
+#define U(x) (uint64_t)(uintptr_t)(x)
+static int put(int cplx, ARGS) {
+  const uint64_t v[17] = {U(h), (uint32_t)oa, (uint32_t)ob, m, n, k, bits(al), U(a), lda, U(b), ldb, bits(be), U(c), ldc,
+                          (uint32_t)mode, cplx ? bits(al + 1) : 0, cplx ? bits(be + 1) : 0};
+  memcpy(seen, v, sizeof v);
+  return 0; }
+int s(ARGS) { return put(0, PASS); }
+int c(ARGS) { return put(1, PASS); }
+int s_ex(ARGS, unsigned *) { return put(0, PASS); }
+int c_ex(ARGS, unsigned *) { return put(1, PASS); }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def seen_stub(tmp_path_factory):
+    d = tmp_path_factory.mktemp("seen")
+    (d / "seen.cpp").write_text(SEEN)
+    subprocess.check_call(["g++", "-shared", "-fPIC", "-o", str(d / "seen.so"), str(d / "seen.cpp")])
+    return ctypes.CDLL(str(d / "seen.so"))
+
+
+@pytest.fixture
+def seen(seen_stub):
+    """(handle, what the last call passed, to the last bit): both routes end in the same functions"""
+    assert _lib.lib() is not None and _lib._native is not None, "csrc/call.cpp is not built"
+    stub = seen_stub
+    address = [ctypes.cast(stub.s if i % 2 == 0 else stub.c, ctypes.c_void_p).value for i in range(len(NAMES))]
+    real = [ctypes.cast(getattr(_lib.lib(), n), ctypes.c_void_p).value for n in _lib._CALL_FUNCTIONS]
+
+    class Library:
+        cuMpSGEMM_sgemm_ex, cuMpSGEMM_cgemm_ex = stub.s_ex, stub.c_ex
+    for name in ("cuMpSGEMM_sgemm_ex", "cuMpSGEMM_cgemm_ex"):
+        getattr(Library, name).argtypes = getattr(_lib.lib(), name).argtypes
+        assert getattr(Library, name).argtypes, name
+    h = cg.Handle.__new__(cg.Handle)
+    h._L, h._h, h._addr = Library, ctypes.c_void_p(0x1230), 0x1230
+    h.close = lambda: None
+    _lib._native.bind(*address)
+    yield h, (ctypes.c_uint64 * 20).in_dll(stub, "seen")
+    _lib._native.bind(*real)
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("where,value", [
+    (2, np.int64(3)), (2, 3.0), (2, "3"), (2, -1), (2, 1 << 63), (2, 1 << 70), (2, (1 << 70) + 5), (2, True), (2, None),
+    (0, np.int32(111)), (0, True), (0, -1), (0, 1 << 40), (0, (1 << 40) + 112), (0, (1 << 31) + 7),
+    (5, 1), (5, np.float32(1)), (5, np.float64(2.5)), (5, 1j), (5, 1e300), (5, -1e-300), (5, float("nan")), (5, float("inf")),
+    (5, -0.0), (5, "x"), (5, "2"), (5, None), (5, True), (5, torch.tensor(1.5)), (10, 3), (10, 2.5 - 1e300j),
+    (6, 0), (6, None), (6, -1), (6, 1 << 63), (6, (1 << 70) + 16), (6, True), (6, np.int64(64)), (6, np.zeros(4)),
+    (6, Pointer()), (6, "a"), (6, "32"), (6, 48.7), (11, torch.zeros(3)), (11, torch.zeros(0)),
+    (13, 1.0), (13, "9"), (13, np.int64(1)), (13, -1), (13, (1 << 32) + 9), (13, None)])
+def test_what_arrives_is_what_ctypes_passes(seen, monkeypatch, cplx, where, value):
+    """To the last bit, or the same exception: sizes and pointers beyond 64 bits, scalars beyond FP32, other types."""
+    h, got = seen
+    args = [111, 112, 2, 3, 4, 1.0, 16, 5, 24, 6, 0.0, 32, 7, 1]
+    args[where] = value
+
+    def outcome():
+        got[:] = [77] * 20
+        try:
+            return h.gemm(*args, cplx=cplx), list(got)
+        except Exception as e:  # noqa: BLE001
+            return type(e), list(got)
+    native = outcome()
+    monkeypatch.setattr(_lib, "_native", None)
+    assert native == outcome()
+    assert isinstance(native[0], type) or native[1][0] == 0x1230
+
+
+def test_usual_arguments_do_not_go_through_ctypes(seen):
+    h, got = seen
+    h = type("Native", (), {"_L": None, "_h": None, "_addr": h._addr, "gemm": cg.Handle.gemm})()
+    for pointer in (16, None, torch.zeros(1)):
+        got[0] = 0
+        assert h.gemm(111, 112, 2, 3, 4, 1.0, pointer, 5, 24, 6, 0.0, 32, 7, 1) == 0 and got[0] == 0x1230
+
+
 @pytest.mark.parametrize("raised", [KeyboardInterrupt, MemoryError, ValueError])
 @pytest.mark.parametrize("where", [6, 8, 11])
 def test_what_a_pointer_raises_ends_the_call(calls, where, raised):

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from cumpsgemm_amd import inputs
-from gpu_util import C, N, T, make_operand, oracle_gemm, rel_diff, run_gemm
+from gpu_util import C, N, T, launched_kernels, make_operand, oracle_gemm, rel_diff, run_gemm
 from test_gpu_ragged_k import FP16TC, FP16TCEC, TF32TC, TF32TCEC, _padded_ints
 
 pytestmark = pytest.mark.gpu
@@ -236,3 +236,64 @@ def test_forms_for_one_workgroup_on_a_cu(O, handle, dev, monkeypatch, mode, cplx
         test_small_products_with_correction_terms(O, handle, dev, monkeypatch, mode, cplx, opa, opb, 5)
         for args in ((SCALING, True, FP16TCEC), (AUTO, True, FP16TCEC)):
             test_small_products_scaled_and_gated_with_correction_terms(handle, dev, monkeypatch, *args, cplx, opa, opb, 5)
+
+
+def _auto_call(handle, dev, opa, opb, m, n, k, batch, cplx, decided, before_reference, after_reference):
+    """(call, C on the device, the explicit mode's result of the same call): padded, with gaps, beta != 0.
+    `decided`: what the operands make AUTO decide for."""
+    gen = inputs.complex_normal if cplx else inputs.uniform
+    ra, ca = (m, k) if opa == N else (k, m)
+    rb, cb = (k, n) if opb == N else (n, k)
+    lda, ldb, ldc = ra + 1, rb + 2, m + 3
+    sa, sb, sc = lda * ca + 5, ldb * cb + 3, ldc * n + 7
+    a, b, c0 = gen(94, sa * batch), gen(95, sb * batch), gen(96, sc * batch)
+    if decided == TF32TCEC:
+        b[::2] *= np.float32(2.0 ** -60)
+    da, db, dc, dr = dev.up(a), dev.up(b), dev.up(c0), dev.up(c0)
+
+    def call():
+        st, ids = handle.gemm_pipeline(opa, opb, m, n, k, 0.75, da, lda, db, ldb, -0.5, dc, ldc, AUTO, cplx=cplx, stridea=sa,
+                                       strideb=sb, stridec=sc, batch=batch)
+        assert st == 0
+        return ids[2]
+    before_reference()
+    st = handle.gemm_strided_batch(opa, opb, m, n, k, 0.75, da, lda, sa, db, ldb, sb, -0.5, dr, ldc, sc, batch, decided, cplx=cplx)
+    after_reference()
+    assert st == 0
+    return call, dc, dr
+
+
+# as dispatched (then: the form that the shared launch takes), and every form that both candidates have forced; K = 2000:
+# bf16x3's tiled plan splits K and would prepare C
+@pytest.mark.parametrize("decided", [FP16TCEC, TF32TCEC])
+@pytest.mark.parametrize("cplx,m,n,k,batch,form,one_launch", [
+    (False, 512, 512, 512, 1, "as dispatched 2", True), (False, 130, 100, 250, 3, "1", True), (False, 101, 77, 129, 5, "2", True),
+    (False, 66, 129, 95, 3, "3", True), (False, 130, 66, 250, 4, "4", True), (True, 256, 256, 256, 1, "as dispatched 1", True),
+    (True, 101, 77, 129, 3, "1", True), (True, 577, 545, 1000, 1, "1", False), (True, 577, 545, 2000, 1, "1", False),
+    (True, 300, 290, 1000, 4, "1", False)])
+def test_auto_in_one_launch_or_two(torch_gpu, handle, dev, monkeypatch, decided, cplx, m, n, k, batch, form, one_launch):
+    """Which kernels run, and that the result is the decided mode's bit for bit, gaps of C included."""
+    forced, form = not form.startswith("as"), form[-1]
+
+    def force():
+        monkeypatch.setenv("CUMPSGEMM_KWAVES", form)
+
+    def release():
+        if not forced:
+            monkeypatch.delenv("CUMPSGEMM_KWAVES")
+    if forced:
+        force()
+    handle.set_exp_stats_params(0.0, 2.0 ** -15, 0.1)
+    try:
+        for opa, opb in ((N, N), (C if cplx else T, N), (N, T), (T, C if cplx else T)):
+            call, dc, dr = _auto_call(handle, dev, opa, opb, m, n, k, batch, cplx, decided, force, release)
+            assert handle.get_dynamic_launch_flag(call()) & 31 == decided
+            out = np.complex64 if cplx else np.float32
+            assert np.array_equal(dev.down(dc, out).view(np.uint32), dev.down(dr, out).view(np.uint32)), (opa, opb)
+            ran = [(name, grid) for name, grid in launched_kernels(torch_gpu, handle, call) if "exp_stats" not in name]
+            assert len(ran) == (1 if one_launch else 2), ran
+            assert all(("kwaves_either_gemm" if one_launch else "kwaves_gemm") in name for name, _ in ran), ran
+            bm = 64 if not cplx and form == "1" else 32
+            assert all(grid[0] == -(-m // bm) * -(-n // bm) * batch for _, grid in ran), ran
+    finally:
+        handle.set_exp_stats_params(0.0, 2.0 ** -15, 0.0)
