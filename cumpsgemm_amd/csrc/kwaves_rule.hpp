@@ -13,10 +13,11 @@ constexpr unsigned kKWavesModuleId = 6; // what used_kernel_module_id reports (0
 
 // Tile and waves of a form, workgroups that a CU holds at once, and the time of a
 // tile in us: `fill` for prologue, sums and write-out, `step` per K-step of a wave,
-// longer by `beside` for every other workgroup on the CU.  bm == 0: no such form.
+// longer by `beside` for every other workgroup on the CU; `once` is paid by the first
+// round alone.  bm == 0: no such form.
 struct KWavesForm {
   int bm, bn, waves, resident;
-  double fill, step, beside;
+  double fill, step, beside, once;
 };
 // ... and what the plan of the tiled kernels takes: us = tiled0 + tiled_per_step *
 // cost, the plan's cost in K-steps of a 256 x 128 tile, + tiled_split if K is split.
@@ -24,9 +25,10 @@ struct KWavesForm {
 // All of it fitted on 188 products (84 real, m and n 64 - 4096, K 64 - 8192, 60 real
 // batches of up to 1024 matrices of 32 - 640, 44 complex; four layouts, padded, with
 // and without C), each timed with every form and tiled, in every precision; the forms
-// with two waves to a SIMD on 640 others, real ones again on 2800 (their `fill` was 0.5 - 1.1 us
-// too low: 256 - 512 tiles of a short K went to 64 x 64 that are faster on 32 x 32 or tiled,
-// bf16x2 512 x 2254 x 128 NN 6.1 us, 64 x 64 7.5).  On 640 more, before that, time over the tiled time,
+// with two waves to a SIMD on 640 others, real ones again on 3200 (without `once` a short K of
+// 257 - 512 tiles went to 64 x 64 that is faster on 32 x 32 or tiled, bf16x2 512 x 2254 x 128
+// NN 6.1 us, 64 x 64 7.5; with it in every round batches went back to the tiled kernels, 320^3
+// x 116 bf16x2 NT 47 us, tiled 86).  On 640 more, before that, time over the tiled time,
 // geometric mean (the fastest side by hindsight): real FP16TCEC 0.72 (0.70), FP16TC
 // 0.69 (0.65), bf16x3 0.72 (0.69), bf16x2 0.72 (0.70); complex 0.60 (0.58), 0.61 (0.58),
 // 0.62 (0.62), 0.68 (0.66); 2 % are slower by 5 %, complex none.  Before there were two
@@ -47,15 +49,15 @@ struct KWavesModel {
 // `prec`: 0 FP16TCEC, 1 FP16TC, 2 bf16x3, 3 bf16x2
 inline const KWavesModel &kwaves_model(int prec, bool cplx) {
   static const KWavesModel real[4] = {
-      {{{64, 64, 4, 2, 3.60, 1.07, 0.72}, {32, 32, 8, 2, 1.13, 0.88, 0.71}, {32, 32, 4, 4, 1.08, 0.50, 0.74}, {32, 32, 1, 16, 2.4, 0.37, 0.22}, {64, 64, 4, 1, 3.6, 0.93, 0.0}}, 4.1, 1.63, -2.1},
-      {{{64, 64, 4, 2, 3.10, 0.67, 1.25}, {32, 32, 8, 2, 0.98, 0.87, 0.55}, {32, 32, 4, 4, 1.00, 0.47, 0.67}, {32, 32, 1, 16, 2.4, 0.23, 0.37}}, 4.8, 1.27, 0.9},
+      {{{64, 64, 4, 2, 3.11, 1.07, 0.72, 0.5}, {32, 32, 8, 2, 1.13, 0.88, 0.71}, {32, 32, 4, 4, 1.08, 0.50, 0.74}, {32, 32, 1, 16, 2.4, 0.37, 0.22}, {64, 64, 4, 1, 3.6, 0.93, 0.0}}, 4.1, 1.63, -2.1},
+      {{{64, 64, 4, 2, 2.10, 0.67, 1.25, 1.0}, {32, 32, 8, 2, 0.98, 0.87, 0.55}, {32, 32, 4, 4, 1.00, 0.47, 0.67}, {32, 32, 1, 16, 2.4, 0.23, 0.37}}, 4.8, 1.27, 0.9},
       {{{64, 64, 4, 1, 3.6, 1.65, 0.0}, {32, 32, 8, 1, 1.62, 1.17, 0.0}, {32, 32, 4, 3, 1.29, 0.76, 0.55}, {32, 32, 1, 12, 2.2, 0.68, 0.17}}, 2.5, 2.29, -2.4},
-      {{{64, 64, 4, 2, 3.75, 0.94, 0.93}, {32, 32, 8, 2, 1.12, 0.87, 0.78}, {32, 32, 4, 4, 1.09, 0.50, 0.73}, {32, 32, 1, 16, 2.5, 0.39, 0.21}}, 4.0, 1.61, -1.6}};
+      {{{64, 64, 4, 2, 2.78, 0.94, 0.93, 0.97}, {32, 32, 8, 2, 1.12, 0.87, 0.78}, {32, 32, 4, 4, 1.09, 0.50, 0.73}, {32, 32, 1, 16, 2.5, 0.39, 0.21}}, 4.0, 1.61, -1.6}};
   static const KWavesModel complex[4] = {
-      {{{32, 32, 4, 2, 1.50, 1.02, 0.94}, {32, 32, 8, 1, 1.15, 1.77, 0.0}, {}, {}, {64, 32, 4, 1, 3.5, 1.67, 0.0}}, 2.8, 2.05, -5.4},
-      {{{32, 32, 4, 2, 1.09, 0.51, 1.72}, {32, 32, 8, 1, 0.74, 1.28, 0.0}, {}, {}, {64, 32, 4, 1, 2.2, 1.12, 0.0}}, 3.6, 1.50, -3.4},
+      {{{32, 32, 4, 2, 1.50, 1.02, 0.94}, {32, 32, 8, 1, 1.15, 1.77, 0.0}, {}, {}, {64, 32, 4, 1, 3.7, 1.75, 0.0}}, 2.8, 2.05, -5.4},
+      {{{32, 32, 4, 2, 1.09, 0.51, 1.72}, {32, 32, 8, 1, 0.74, 1.28, 0.0}, {}, {}, {64, 32, 4, 1, 2.5, 1.12, 0.0}}, 3.6, 1.50, -3.4},
       {{{32, 32, 4, 1, 2.3, 1.71, 0.0}, {}, {}, {}}, 0.9, 3.83, -14.3},
-      {{{32, 32, 4, 2, 1.55, 0.97, 1.06}, {32, 32, 8, 1, 0.99, 1.85, 0.0}, {}, {}, {64, 32, 4, 1, 3.7, 1.72, 0.0}}, 3.1, 2.09, -6.1}};
+      {{{32, 32, 4, 2, 1.55, 0.97, 1.06}, {32, 32, 8, 1, 0.99, 1.85, 0.0}, {}, {}, {64, 32, 4, 1, 3.8, 1.80, 0.0}}, 3.1, 2.09, -6.1}};
   return (cplx ? complex : real)[prec];
 }
 
@@ -77,7 +79,7 @@ inline double kwaves_time(const KWavesForm &f, const KWavesProblem &p, unsigned 
   // FP16TCEC NT 88 -> 69, 128 x 36 x 102 x 870 bf16x3 NN 41 -> 30), 4 are slower by 3 - 5 %; with no rounds at all two of
   // 150 by 10 - 13 % (256^3 x 77 FP16TCEC TT 18.5 -> 21.0).
   const double part = (double)kwaves_tiles(f, p) / ((double)cus * f.resident);
-  return 2.2 + (f.waves == 1 && part > 1.0 ? 0.5 * (part + (double)rounds) : (double)rounds) * (f.fill + (double)steps * f.step * (1.0 + f.beside * beside));
+  return 2.2 + f.once + (f.waves == 1 && part > 1.0 ? 0.5 * (part + (double)rounds) : (double)rounds) * (f.fill + (double)steps * f.step * (1.0 + f.beside * beside));
 }
 
 // Whether a form can serve the product at all.

@@ -173,3 +173,11 @@ def test_two_rounds_of_large_tiles_at_most_and_no_third_tile_on_a_cu(rule, prec)
             p = rule(prec, False, op, m, n, 2000, steps={0: 42, 1: 45, 3: 42}[prec] * rounds)
             assert (p and p[:3]) == ((0, 64, 64) if taken else None), (op, tiles_m, tiles_n)
         assert rule(prec, False, op, 64 * 19, 64 * 27, 500, steps=40) is not None
+
+
+@pytest.mark.parametrize("prec,op,m,n,k,batch,pad,steps", [
+    (0, "TN", 53, 265, 411, 608, 0, 49.27), (1, "TT", 320, 320, 320, 159, 0, 52.19), (1, "NT", 128, 128, 128, 331, 0, 9.94),
+    (0, "TT", 704, 393, 231, 17, 0, 13.31)])
+def test_batches_of_several_rounds_keep_their_large_tiles(rule, prec, op, m, n, k, batch, pad, steps):
+    """Measured 0.61 - 0.91 of the tiled time on 64 x 64 tiles."""
+    assert rule(prec, False, op, m, n, k, batch, pad, steps=steps)[:3] == (0, 64, 64)
