@@ -134,12 +134,12 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
       best_time = t;
     }
   }
-  if (asked < 0 && !p.cplx && best == 0 && model.form[0].resident == 2 && p.k > 512 && (p.a_kc || p.b_kc) &&
+  if (asked < 0 && !p.cplx && p.batch == 1 && best == 0 && model.form[0].resident == 2 && p.k > 512 && (p.a_kc || p.b_kc) &&
       (kwaves_tiles(model.form[0], p) + cus - 1) / cus == 3) {
     // Three tiles of 64 x 64 on a CU that holds two: a round for the third, and where the estimates still send them here
     // that of the tiled kernels is too dear.  16 drawn products, 513 - 600 tiles: 1.12 of the tiled time, 0.90 - 1.41
     // (3392 x 591 x 2932 FP16TCEC TT 106 us, tiled 76).  Not with two row-contiguous operands (7: 0.91), nor with four
-    // tiles (47: 0.84).
+    // tiles (47: 0.84), nor batches, whose tiled estimate has not that fault (160 x 288 x 640 x 47 FP16TC NN 31 us, tiled 49).
     best = -1;
   }
   if (asked < 0 && p.cplx && best >= 0 && model.form[best].waves == 8 &&

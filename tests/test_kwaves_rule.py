@@ -177,7 +177,7 @@ def test_two_rounds_of_large_tiles_at_most_and_no_third_tile_on_a_cu(rule, prec)
 
 @pytest.mark.parametrize("prec,op,m,n,k,batch,pad,steps", [
     (0, "TN", 53, 265, 411, 608, 0, 49.27), (1, "TT", 320, 320, 320, 159, 0, 52.19), (1, "NT", 128, 128, 128, 331, 0, 9.94),
-    (0, "TT", 704, 393, 231, 17, 0, 13.31)])
+    (0, "TT", 704, 393, 231, 17, 0, 13.31), (1, "NN", 160, 288, 640, 47, 1, 45.0)])
 def test_batches_of_several_rounds_keep_their_large_tiles(rule, prec, op, m, n, k, batch, pad, steps):
     """Measured 0.61 - 0.91 of the tiled time on 64 x 64 tiles."""
     assert rule(prec, False, op, m, n, k, batch, pad, steps=steps)[:3] == (0, 64, 64)
