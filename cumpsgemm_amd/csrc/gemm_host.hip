@@ -416,8 +416,8 @@ PreSplitChoice choose_pre_split(const cuMpSGEMM_handle *h, bool a_kc, bool b_kc,
   const bool forced = h->ws_override != nullptr;
   // (depth 2: the whole rounds of a problem that was cut for this path)
   const bool never = tuning().packed == 0 && !forced, always = tuning().packed == 1 || forced || depth == 2;
-  // bf16x3 (explicit TF32TCEC mode): its in-loop three-way split costs 5.5
-  // vector instructions per value, so the pre-pass pays for every layout
+  // bf16x3 (explicit TF32TCEC mode): its in-loop three-way split costs 5.5 vector instructions
+  // per value; the pre-pass pays for every layout from the sizes of `pays_bf16` on
   ch.bf16 = (mode == CUMPSGEMM_TF32TCEC);
   ch.bm = CPLX ? kPackedCplxBM : (ch.bf16 ? kPackedBf16BM : kPackedBM);
   ch.bn = CPLX ? kPackedCplxBN : (ch.bf16 ? kPackedBf16BN : kPackedBN);
@@ -428,23 +428,26 @@ PreSplitChoice choose_pre_split(const cuMpSGEMM_handle *h, bool a_kc, bool b_kc,
                         (forced || (uint64_t)m * n >= (uint64_t)h->num_cus * ch.bm * ch.bn) && k / 32 < 65535;
   if (!shape_ok) return ch; // (neither taken nor cut)
   const double mn_ratio = (double)m * (double)n / ((double)m + (double)n);
-  // (in-loop -> pre-split, TFLOP/s: 4096^2 x 256 198 -> 211, 4096^2 x 384 224 -> 260, 5120^2 x 256 176 -> 209,
-  // 3072^2 x 512 177 -> 191, 3072^2 x 1024 201 -> 237, 8192 x 4096 x 256 211 -> 245, 4096 x 8192 x 384 232 -> 316;
-  // 3072^2 x 2048 level)
+  // (The lines of this function were drawn with an in-loop split that took longer than today's; both sides are as measured
+  // with today's.  Where a figure speaks against its line the line has not been moved yet.)
+  // (in-loop -> pre-split, TFLOP/s: 4096 x 8192 x 384 280 -> 309, 4096^2 x 384 257 -> 253, 5120^2 x 256 level; beyond the
+  // line for the other side by now: 4096^2 x 256 223 -> 207, 8192 x 4096 x 256 263 -> 247, 3072^2 x 512 217 -> 188,
+  // x 1024 267 -> 233, x 2048 295 -> 258 -- when it was drawn 198 -> 211, 211 -> 245, 177 -> 191, 201 -> 237, level)
   const bool pays_nt_shape = !a_kc && !b_kc && ((k >= 384 && mn_ratio >= 1500.0) || (k >= 256 && mn_ratio >= 2000.0));
   // Every other layout: the pre-split kernel, freed of the split arithmetic,
   // outruns the in-loop one by more than the pre-pass costs once the problem
-  // is large (8192^3: 381 vs 361 - 372 TFLOP/s; 8192^2 x 1024: 351 vs 318 -
-  // 343) -- provided the last round of CU slots is at least half full or one
+  // is large (8192^3: 429 vs 369 - 371 TFLOP/s; 8192^2 x 1024: 405 vs 355 -
+  // 373) -- provided the last round of CU slots is at least half full or one
   // of many: the path has no column split for a mostly empty last round.
   const uint64_t ptiles = ((m + ch.bm - 1) / ch.bm) * ((n + ch.bn - 1) / ch.bn);
   const uint64_t last_round = ptiles % h->num_cus;
   const bool rounds_ok = last_round == 0 || 2 * last_round >= h->num_cus || ptiles >= 6ull * h->num_cus;
   // (complex: four times the MFMA work per element split, so the pre-pass weighs less)
-  // (5120^3, 800 tiles = 3.1 rounds: 329 TFLOP/s this way, 356 in-loop, whose planner cuts C in two)
-  // With fused scaling the in-loop split costs one more instruction per pair
-  // and those kernels run 8 - 25 % below the plain ones, so the pre-pass (which
-  // scales as it splits) pays for every layout.
+  // (5120^3, 800 tiles = 3.1 rounds: 367 TFLOP/s this way, 361 in-loop, 395 cut after three rounds)
+  // With fused scaling the in-loop split costs two more instructions per pair, so the pre-pass (which scales as it splits)
+  // pays for every layout once K is long or C large (whole pipelines, in-loop -> pre-split, NN / TN / NT, TFLOP/s: 4096^3
+  // 354 / 366 / 340 -> 391 / 389 / 390, 8192^2 x 256 259 / - / 244 -> 275 / - / 281, 4096^2 x 512 259 / 262 / 238 -> 254 / 254 /
+  // 260; 4096^2 x 256 205 / 213 / 194 -> 189 / 190 / 188 is on the wrong side by now)
   const bool pays_scaled = h->fused_scaling && k >= 256 && mn_ratio >= 1800.0;
   // AUTO: the FP16TCEC candidate may take the path as well, gated by the
   // launch flag like every AUTO kernel (pre-pass included).  Both candidates
@@ -452,10 +455,11 @@ PreSplitChoice choose_pre_split(const cuMpSGEMM_handle *h, bool a_kc, bool b_kc,
   if (!CPLX && mode == CUMPSGEMM_AUTO && pays_scaled && depth == 0) {
     ch.auto_ok = make_plan(h, Prec::BF16X3, CPLX, a_kc, b_kc, m, n, k, batch, force_cls, force_split).ksplit == 1;
   }
-  // (measured against the in-loop 256x128 class, NN / TN, TFLOP/s: 8192^2 x 256 167 / 172 -> 189 / 187,
-  // 6144^2 x 256 152 / 157 -> 173 / 178, 4096^2 x 512 182 / 189 -> 190 / 191, 4096^3 208 / 213 -> 231 / 228,
-  // 3072^2 x 1024 157 / 162 -> 171 / 171, 2048^2 x 2048 188 / 178 -> 200 / 198; 4096^2 x 384, 3072^2 x 512 and
-  // 2048^2 x 1024 are level, shorter K loses)
+  // (in-loop -> pre-split, NN / TN / NT, TFLOP/s: 8192^2 x 256 159 / 163 / 156 -> 204 / 201 / 205, 6144^2 x 256 168 / 173 / 178 ->
+  // 182 / 187 / 193, 4096^2 x 512 181 / 189 / 180 -> 200, 4096^3 208 / 211 / 206 -> 232 / 226 / 228, 3072^2 x 1024 163 / 166 / 158
+  // -> 170 / 171 / 171, 4000 x 3000 x 2000 187 / 174 / 184 -> 212 / 208 / 207, 2048^2 x 2048 196 / 191 / 195 -> 194 / 196 / 196;
+  // on the other side 3072^2 x 512 152 / 154 / 148 -> 148, 2048^2 x 1024 191 / 190 / 188 -> 172 / 175 / 174, but also 4096^2 x
+  // 384 174 / 179 / 173 -> 187 / 186 / 184)
   const bool pays_bf16 = (k >= 256 && mn_ratio >= 3000.0) || (k >= 512 && mn_ratio >= 2000.0) ||
                          (k >= 1024 && mn_ratio >= 1500.0) || (k >= 2048 && mn_ratio >= 1000.0);
   // The rules that depend on how well the rounds of CU slots are filled (ro:
@@ -463,13 +467,11 @@ PreSplitChoice choose_pre_split(const cuMpSGEMM_handle *h, bool a_kc, bool b_kc,
   auto worth_if = [&](const bool ro) {
     const bool pays_nt = pays_nt_shape && ro;
     // Shorter K: per tile the in-loop kernels lose more to the split than the pre-pass
-    // costs once C is large (in-loop -> pre-split, TFLOP/s, NN / TN: 8192^2 x 256 261 / 270 -> 277 / 278,
-    // 8192^2 x 384 287 / 297 -> 314 / 313, 6144^2 x 384 254 / 266 -> 280 / 282, 6144^2 x 512 274 / 285 -> 306 / 307,
-    // 4096^2 x 1024 326 / 333 -> 343 / 343, 4096^2 x 2048 350 / 357 -> 384 / 384; 6144^2 x 256 and 4096^2 x 512
-    // are level and stay in-loop, 4096^2 x 256 would lose 8 - 11 %).
-    // (re-measured with the cheaper write-out of the pre-split kernels, NN / TN, packed over in-loop: 4096^2 x 384
-    // 1.00 / 0.99, 4096 x 8192 x 384 1.12 / 1.14, 6144^2 x 384 1.06 / 1.04, 4096^2 x 512 1.01 / 1.01, 4096^2 x 768
-    // 1.08 / 1.07, 6144^2 x 256 1.06 / 1.01, 8192 x 4096 x 256 0.96 / 0.95, 5120^2 x 256 0.91 / 0.90)
+    // costs once C is large (in-loop -> pre-split, TFLOP/s, NN / TN: 8192^2 x 384 315 / 322 -> 332 / 333, 6144^2 x 384
+    // 247 / 259 -> 292 / 293, x 512 261 / 278 -> 320 / 318, 4096^2 x 768 317 / 326 -> 330 / 325, x 1024 334 / 353 -> 350 / 346,
+    // x 2048 349 / 359 -> 388 / 393, 4096 x 8192 x 384 300 / 308 -> 304 / 310; 8192^2 x 256 297 / 310 -> 295 / 294.  In-loop:
+    // 4096^2 x 256 240 / 255 -> 212 / 210, x 384 275 / 289 -> 250 / 251, x 512 293 / 309 -> 278 / 279, 8192 x 4096 x 256
+    // 264 / 277 -> 241 / 238, 5120^2 x 256 216 / 218 -> 206 / 209, but also 6144^2 x 256 228 / 239 -> 250 / 250.)
     const bool pays_short = !CPLX && ro &&
                             ((k >= 256 && mn_ratio >= 4000.0) || (k >= 384 && mn_ratio >= 2500.0) ||
                              (k >= 768 && mn_ratio >= 2000.0));
@@ -487,21 +489,21 @@ PreSplitChoice choose_pre_split(const cuMpSGEMM_handle *h, bool a_kc, bool b_kc,
     // the former: it is taken for large square-ish problems only.
     // Measured (in-loop -> pre-split, TFLOP/s): FP16TC 8192^3 580 - 624 -> 930 - 940, 4096^3 586 - 706 ->
     // 852 - 870, 4096^2 x 1024 505 - 566 -> 634 - 654, 8192^2 x 512 482 - 520 -> 579 - 601, 16384^2 x 256
-    // 390 - 407 -> 461 - 480, 4096^2 x 512 level; bf16x2 8192^3 320 - 377 -> 394 - 396, 4096^2 x 1024
-    // 304 - 337 -> 348 - 355, 8192^2 x 512 275 - 308 -> 318 - 327, 4096^2 x 512 level except NT.
+    // 390 - 407 -> 461 - 480, 4096^2 x 512 level; bf16x2 8192^3 387 - 422 -> 440 - 442, 4096^2 x 1024
+    // 343 - 372 -> 358 - 367, 8192^2 x 512 336 - 357 -> 371 - 376, 4096^2 x 512 302 / 313 -> 291 / 294, NT 294 -> 298.
     // Complex (the 128x64 kernels): FP16TC 4096^3 560 - 678 -> 872 - 891, 2048^3 525 - 640 -> 760 - 779,
-    // 8192^2 x 256 477 - 543 -> 624 - 643; bf16x2 4096^3 350 -> 375, 4096^2 x 1024 333 - 339 -> 365,
-    // 4096^2 x 512 303 - 326 -> 336 - 347.
+    // 8192^2 x 256 477 - 543 -> 624 - 643; bf16x2 4096^3 408 - 414 -> 453 - 455, 4096^2 x 1024 379 - 386 -> 442 - 444,
+    // 4096^2 x 512 362 - 365 -> 411 - 418.
     const bool pays_tc =
         ro &&
         (CPLX ? (k >= 256 && mn_ratio >= 1000.0)
               : ((k >= 1024 && mn_ratio >= (mode == CUMPSGEMM_FP16TC ? 1500.0 : 2000.0)) ||
                  (k >= 512 && mn_ratio >= 4000.0) || (k >= 256 && mn_ratio >= 8000.0) ||
                  (mode == CUMPSGEMM_TF32TC && pays_nt_shape)));
-    // (complex bf16x3, two-buffer pre-split kernel against the in-loop one, NN / TN, TFLOP/s: 4096^3 228 / 238 ->
-    // 237 / 237, 3072^2 x 1024 205 / 215 -> 223 / 223, 4096^2 x 512 211 / 216 -> 230 / 226, 8192^2 x 256 197 / 205 ->
-    // 219 / 218, 3072^2 x 384 189 / 199 -> 203 / 202, 2048^2 x 1024 222 / 230 -> 231 / 231, 4096^2 x 256 198 / 205 ->
-    // 206 / 210; 2048^2 x 512 level: the complex rule above)
+    // (complex bf16x3, two-buffer pre-split kernel against the in-loop one, NN / TN, TFLOP/s: 4096^3 231 / 243 ->
+    // 236 / 236, 3072^2 x 1024 207 / 222 -> 224 / 226, 4096^2 x 512 215 / 220 -> 234 / 230, 8192^2 x 256 198 / 210 ->
+    // 215 / 216, 3072^2 x 384 187 / 203 -> 203 / 205, 2048^2 x 1024 226 / 237 -> 230 / 231, 4096^2 x 256 198 / 217 ->
+    // 213 / 214; 2048^2 x 512 211 / 223 -> 208 / 212: the complex rule above)
     const bool pays_b3 = CPLX ? pays_cplx : pays_bf16;
     return ch.bf16 ? (pays_b3 || always) : (ch.tc_only ? (pays_tc || always) : (pays || pays_scaled || always));
   };

@@ -17,19 +17,19 @@
 // unit from the SIMD's other waves).  All loads are 16 bytes a lane, of a
 // row-contiguous operand too: a quarter of the load instructions.
 //
-// Two waves to a SIMD where the registers allow it (not bf16x3): a wave alone issues a
+// Two waves to a SIMD where the registers allow it (not bf16x3) and a CU gets two workgroups,
+// or one of eight waves (otherwise: kwaves_rule.hpp, the forms for one workgroup on a CU): a wave alone issues a
 // vector instruction every 5 clocks and a conversion every 8, two of them together one
 // every 2 - 4, and MFMAs of one run beside splitting of the other.  On a 64 x 64 (complex
 // 32 x 32) tile that is two workgroups of four waves on a CU; complex products of no more
 // tiles than CUs take one of eight.  us, one workgroup of four waves per CU -> so: real
 // FP16TCEC 1152^3 NN 25.4 -> 20.3 (tiled 24.4), 1408^3 30.5 -> 26.8, 1531 x 1021 x 777 TT
 // 22.7 -> 18.8 (tiled 19.6); FP16TC 1152^3 17.5 -> 15.0; complex FP16TCEC 512^3 NN 8.5 -> 7.6,
-// 640^3 16.6 -> 12.9, 900 x 300 x 900 22.9 -> 17.5, 512 x 512 x 2048 22.0 -> 20.8; level on
-// 1024^3 (12.9), whose 256 tiles are one to a CU either way.
+// 640^3 16.6 -> 12.9, 900 x 300 x 900 22.9 -> 17.5, 512 x 512 x 2048 22.0 -> 20.8.
 //
-// FP16TCEC, us, tiled -> here (calls of a graph; a loop of single calls takes 5 at least):
-// 512^3 NN 9.5 -> 4.4, NT 9.7 -> 4.3, 1024^3 NN 16.1 -> 13.0, NT 22.1 -> 12.2, TN 13.4 -> 12.5;
-// complex 256^3 NN 13.1 -> 5.3, NT 13.5 -> 5.2, 512^3 NN 14.9 -> 7.6, NT 16.6 -> 7.5.
+// FP16TCEC, us, tiled -> here (calls of a graph; a loop of single calls takes 4 at least):
+// 512^3 NN 9.9 -> 4.7, NT 10.1 -> 4.6, 1024^3 NN 16.0 -> 12.9, NT 21.2 -> 12.2, TN 13.6 -> 12.8;
+// complex 256^3 NN 13.2 -> 5.5, NT 13.6 -> 5.4, 512^3 NN 14.9 -> 7.8, NT 16.9 -> 7.7.
 // Larger products are bound by what a small tile reads (2048^3 NN 58 -> 74): see kwaves_rule.hpp.
 #pragma once
 #include "gemm_kernel.hpp"

@@ -25,17 +25,21 @@ struct KWavesForm {
 // All of it fitted on 188 products (84 real, m and n 64 - 4096, K 64 - 8192, 60 real
 // batches of up to 1024 matrices of 32 - 640, 44 complex; four layouts, padded, with
 // and without C), each timed with every form and tiled, in every precision; the forms
-// with two waves to a SIMD on 640 others, real ones again on 3200 (without `once` a short K of
-// 257 - 512 tiles went to 64 x 64 that is faster on 32 x 32 or tiled, bf16x2 512 x 2254 x 128
-// NN 6.1 us, 64 x 64 7.5; with it in every round batches went back to the tiled kernels, 320^3
-// x 116 bf16x2 NT 47 us, tiled 86).  On 640 more, before that, time over the tiled time,
-// geometric mean (the fastest side by hindsight): real FP16TCEC 0.72 (0.70), FP16TC
-// 0.69 (0.65), bf16x3 0.72 (0.69), bf16x2 0.72 (0.70); complex 0.60 (0.58), 0.61 (0.58),
-// 0.62 (0.62), 0.68 (0.66); 2 % are slower by 5 %, complex none.  Before there were two
-// waves to a SIMD: 0.73, 0.70, 0.72, 0.73; 0.66, 0.63, 0.62, 0.74.
+// with two waves to a SIMD on 640 others, the first and the last form again on 3200 (without
+// `once` a short K of 257 - 512 tiles went to 64 x 64 that is faster on 32 x 32 or tiled,
+// bf16x2 512 x 2254 x 128 NN 6.1 us, 64 x 64 7.5; with it in every round batches went back to
+// the tiled kernels, 320^3 x 116 bf16x2 NT 47 us, tiled 86).  On 3900 other products, of which
+// the rule takes 2937: time over the tiled time, geometric mean (the fastest side by hindsight),
+//               real         real batches  complex      complex batches
+//   FP16TCEC    0.65 (0.63)  0.69 (0.67)   0.53 (0.52)  0.57 (0.57)
+//   bf16x3      0.61 (0.60)  0.67 (0.65)   0.47 (0.47)  0.62 (0.62)
+//   FP16TC      0.60 (0.59)  0.67 (0.66)   0.46 (0.46)  0.51 (0.51)
+//   bf16x2      0.69 (0.67)  0.68 (0.65)   0.57 (0.55)  0.61 (0.60)
+// 2.7 % are slower than tiled by 5 %, 1.5 % by 10 %, the worst takes 1.31 times as long; 400 AUTO
+// calls 0.77 real, 0.71 complex, none slower by 2 %.
 // Forms of one wave to a SIMD, which has the registers for two sets of fragments or for a 64 x 32 complex tile, are the
 // faster ones where a CU has no second workgroup anyway.  2100 real and 1500 complex products, geometric mean: real
-// FP16TCEC against two sets of registers to a SIMD up to K = 256 1.04, 512 0.99, 1024 0.97, 2048 0.96, 4096 0.94 (FP16TC and
+// FP16TCEC, against two waves on a SIMD, up to K = 256 1.04, 512 0.99, 1024 0.97, 2048 0.96, 4096 0.94 (FP16TC and
 // bf16x2 1.00, 0.98: left out); complex against the faster of its other two, where those are two to a CU: K <= 256
 // 1.2 - 1.3, 1024 FP16TC 0.93, others 1.06 - 1.09, beyond 2048 0.83 and 0.94 - 0.95.
 // (Tried beside these and left out: 64 x 64 with eight waves at two to a SIMD, up to
@@ -109,7 +113,7 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
   const double tiled = model.tiled0 + layout * model.tiled_per_step * tiled_steps + (tiled_split ? model.tiled_split : 0.0);
   // Both sides are estimates, within 10 - 30 % of the times: with 1.0 here the number of products that get more than
   // 3 % slower doubles and the mean stays; with 0.8 (long ones 0.7) a third of the losses is left, and the mean of 10000
-  // real products goes from 0.643 to 0.660 of the tiled time.  Long ones have less to gain: 0.8.  (Complex ones: 0.95;
+  // real products (drawn for the forms of one wave to a SIMD) goes from 0.643 to 0.660 of the tiled time.  Long ones have less to gain: 0.8.  (Complex ones: 0.95;
   // 3 of 240 slower by 5 %, with 1.0 for short ones 5.)
   double best_time = (p.cplx ? 0.95 : tiled > 30.0 ? 0.8 : 0.9) * tiled;
   int best = -1;
