@@ -444,7 +444,7 @@ PreSplitChoice choose_pre_split(const cuMpSGEMM_handle *h, bool a_kc, bool b_kc,
   const bool rounds_ok = last_round == 0 || 2 * last_round >= h->num_cus || ptiles >= 6ull * h->num_cus;
   // (complex: four times the MFMA work per element split, so the pre-pass weighs less)
   // (5120^3, 800 tiles = 3.1 rounds: 367 TFLOP/s this way, 361 in-loop, 395 cut after three rounds)
-  // With fused scaling the in-loop split costs two more instructions per pair, so the pre-pass (which scales as it splits)
+  // With fused scaling the in-loop split costs one or two more instructions per pair, so the pre-pass (which scales as it splits)
   // pays for every layout once K is long or C large (whole pipelines, in-loop -> pre-split, NN / TN / NT, TFLOP/s: 4096^3
   // 354 / 366 / 340 -> 391 / 389 / 390, 8192^2 x 256 259 / - / 244 -> 275 / - / 281, 4096^2 x 512 259 / 262 / 238 -> 254 / 254 /
   // 260; 4096^2 x 256 205 / 213 / 194 -> 189 / 190 / 188 is on the wrong side by now)

@@ -241,10 +241,11 @@ template <> struct splitter<Prec::BF16X2> {
 
 // Terms of one pair of values, packed (SCALED: of the pair times s, a power of
 // two; s2048 = s * 2^11), for kernels that are bound by issuing vector
-// instructions.  FP16TCEC: fma(hi, -2^11, x * 2^11) as above, but on values widened
-// again: 8 instructions instead of 5, which one wave alone on a SIMD issues in
-// 27 clocks instead of 29 (37 with the wait that two half writes in a row need):
-// the mixed-precision FMA that writes fp16 has a quarter of the FMA's rate.
+// instructions.  FP16TCEC: fma(hi, -2^11, x * 2^11) as above, but with an FP32 result, both
+// of which one instruction converts (the compiler lets the FMA read hi as fp16,
+// v_fma_mix_f32): 6 instructions instead of 5, 31 - 35 clocks a pair instead of 33 - 37 for a
+// wave alone on a SIMD, 29 - 32 instead of 32 - 37 for each of two.  The FMA that writes fp16
+// takes 9.5 - 11 clocks, the others 5, a conversion 8.
 template <Prec P, bool SCALED>
 __device__ inline void split_pair(float x0, float x1, const float s, const float s2048,
                                   uint32_t (&out)[prec_traits<P>::NP]) {
@@ -1190,7 +1191,7 @@ __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void gemm_tcec_kernel(c
         LB::template store_packed<NP * NCOMP>(rb, sb, tid);
       }
     } else {
-      // (FP16TCEC on 16x16x32 MFMAs, 256x128 and 128x256: full-rate instructions though more of them, us: 512^3 x 64 NN
+      // (FP16TCEC on 16x16x32 MFMAs, 256x128 and 128x256: shorter instructions though more of them, us: 512^3 x 64 NN
       // 63.0 -> 57.9, TT 61.0 -> 56.9, 1024^3 x 8 54.6 -> 52.4, 4096^2 x 256 TT 36.8 -> 34.0.  On 32x32x16 MFMAs, whose
       // schedule then puts vector instructions behind the last of them, 3000^2 x 768 NN 64.8 -> 69.3.  128x128 on 16x16x32:
       // level, 36 launches that fill the chip 0.96 - 1.04, geometric mean 1.000.  No complex FP16TCEC kernel has them.)

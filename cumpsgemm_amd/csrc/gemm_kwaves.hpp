@@ -19,8 +19,8 @@
 //
 // Two waves to a SIMD where the registers allow it (not bf16x3) and a CU gets two workgroups,
 // or one of eight waves (otherwise: kwaves_rule.hpp, the forms for one workgroup on a CU): a wave alone issues a
-// vector instruction every 5 clocks and a conversion every 8, two of them together one
-// every 2 - 4, and MFMAs of one run beside splitting of the other.  On a 64 x 64 (complex
+// vector instruction every 5 clocks and a conversion every 8, two of them together twice
+// as many, and MFMAs of one run beside splitting of the other.  On a 64 x 64 (complex
 // 32 x 32) tile that is two workgroups of four waves on a CU; complex products of no more
 // tiles than CUs take one of eight.  us, one workgroup of four waves per CU -> so: real
 // FP16TCEC 1152^3 NN 25.4 -> 20.3 (tiled 24.4), 1408^3 30.5 -> 26.8, 1531 x 1021 x 777 TT
