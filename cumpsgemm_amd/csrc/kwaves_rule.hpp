@@ -76,14 +76,16 @@ inline uint64_t kwaves_tiles(const KWavesForm &f, const KWavesProblem &p) {
 
 inline double kwaves_time(const KWavesForm &f, const KWavesProblem &p, unsigned cus) {
   const uint64_t steps = ((p.k + 31) / 32 + f.waves - 1) / f.waves;
-  const uint64_t per_cu = (kwaves_tiles(f, p) + cus - 1) / cus, rounds = (per_cu + f.resident - 1) / f.resident;
+  const uint64_t tiles = kwaves_tiles(f, p), per_cu = (tiles + cus - 1) / cus;
+  const uint64_t rounds = per_cu <= (uint64_t)f.resident ? 1 : (per_cu + f.resident - 1) / f.resident;
   const double beside = (double)((per_cu < (uint64_t)f.resident ? per_cu : (uint64_t)f.resident) - 1);
   // Workgroups of one wave hardly run in rounds: as one ends the next begins.  Half way between whole rounds and none, on
   // 350 drawn batches against whole ones: 11 take 0.55 - 0.96 of the time (416^3 x 35 bf16x2 TN 64 -> 35 us, 262^3 x 152
   // FP16TCEC NT 88 -> 69, 128 x 36 x 102 x 870 bf16x3 NN 41 -> 30), 4 are slower by 3 - 5 %; with no rounds at all two of
   // 150 by 10 - 13 % (256^3 x 77 FP16TCEC TT 18.5 -> 21.0).
-  const double part = (double)kwaves_tiles(f, p) / ((double)cus * f.resident);
-  return 2.2 + f.once + (f.waves == 1 && part > 1.0 ? 0.5 * (part + (double)rounds) : (double)rounds) * (f.fill + (double)steps * f.step * (1.0 + f.beside * beside));
+  double in_rounds = (double)rounds;
+  if (f.waves == 1 && rounds > 1) in_rounds = 0.5 * ((double)tiles / ((double)cus * f.resident) + in_rounds);
+  return 2.2 + f.once + in_rounds * (f.fill + (double)steps * f.step * (1.0 + f.beside * beside));
 }
 
 // Whether a form can serve the product at all.
@@ -113,12 +115,14 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
   const double tiled = model.tiled0 + layout * model.tiled_per_step * tiled_steps + (tiled_split ? model.tiled_split : 0.0);
   // Both sides are estimates, within 10 - 30 % of the times: with 1.0 here the number of products that get more than
   // 3 % slower doubles and the mean stays; with 0.8 (long ones 0.7) a third of the losses is left, and the mean of 10000
-  // real products (drawn for the forms of one wave to a SIMD) goes from 0.643 to 0.660 of the tiled time.  Long ones have less to gain: 0.8.  (Complex ones: 0.95;
-  // 3 of 240 slower by 5 %, with 1.0 for short ones 5.)
+  // real products (drawn for the forms of one wave to a SIMD) goes from 0.643 to 0.660 of the tiled time.  Long ones have
+  // less to gain: 0.8.  (Complex ones: 0.95; 3 of 240 slower by 5 %, with 1.0 for short ones 5.)
   double best_time = (p.cplx ? 0.95 : tiled > 30.0 ? 0.8 : 0.9) * tiled;
   int best = -1;
   for (int i = 0; i < kKWavesForms; i++) {
     const KWavesForm &f = model.form[i];
+    // (a small product's call is bound by the host: what rules a form out without a division comes first)
+    if (i == kKWavesAlone && asked < 0 && !p.cplx && p.k <= 512) continue;
     if (!kwaves_can_serve(f, p)) continue;
     if (asked > 0) {
       if (asked == i + 1) return i;
@@ -129,7 +133,7 @@ inline int choose_kwaves_form(int prec, const KWavesProblem &p, unsigned cus, do
     // NT 35.7 us, tiled 34.1; 2216 x 1984 x 3200 TN 126, 113).
     const uint64_t per_cu = (kwaves_tiles(f, p) + cus - 1) / cus;
     if (per_cu > 2ull * f.resident && p.k > 512) continue;
-    if (i == kKWavesAlone && (per_cu > 1 || (!p.cplx && p.k <= 512))) continue;
+    if (i == kKWavesAlone && per_cu > 1) continue;
     // (complex, more than one round of tiles: the fit is up to 10 % short.  FP16TC 1000^3 NN 23.2 us tiled, 26.1 here.)
     const bool rounds = p.cplx && per_cu > (uint64_t)f.resident;
     const double t = kwaves_time(f, p, cus) * (rounds ? 1.1 : 1.0);
